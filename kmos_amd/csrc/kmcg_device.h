@@ -124,6 +124,8 @@ struct KParams {
     int merged;                    // bit 0: the segments of a step share one apply;
                                    // bit 1: a lat_int group's segments post in one pass
     int off_seg, off_proc, off_touch, off_nli, off_nlitab;
+    const int *fz_recs;            // records of the fused step loop (kmcg_fused.hip)
+    int fz_nch;                    // chunks of 64 records per process
     double *srec;                  // in-loop sample records (or null)
     int sample_every, srec_cap, srec_width;
     int mode;                      // misc kernel mode

@@ -15,11 +15,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
+#include <map>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "kmcg.h"
@@ -1127,15 +1131,19 @@ struct NextSel {
     }
 };
 
-// Copy the op program to LDS (whole workgroup), then set up this wave.
-// Returns the replica index, or -1 for a wave without one.
-template <int PPL, int BITS, bool LDS_LAT>
+// Copy the op program to LDS (whole workgroup, PROG), then set up this wave.
+// Returns the replica index, or -1 for a wave without one.  Without PROG
+// (the fused form reads its records from global memory) a wave's LDS holds
+// the lattice, the list-tail windows and the species counts only.
+template <int PPL, int BITS, bool LDS_LAT, bool PROG = true>
 __device__ __forceinline__ int wave_setup(Wave<PPL, BITS> &W, const KParams &kp, unsigned char *smem)
 {
     int *sprog = (int *)smem;
-    for (int i = threadIdx.x; i < kp.prog_words; i += blockDim.x)
-        sprog[i] = kp.prog[i];
-    __syncthreads();
+    if (PROG) {
+        for (int i = threadIdx.x; i < kp.prog_words; i += blockDim.x)
+            sprog[i] = kp.prog[i];
+        __syncthreads();
+    }
     // wave-uniform values: keep them in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = blockIdx.x * kp.wpg + wave;
@@ -1182,7 +1190,7 @@ __device__ __forceinline__ int wave_setup(Wave<PPL, BITS> &W, const KParams &kp,
     }
     W.mrows = kp.mrows;
     W.cnt = W.mbox + kp.mrows * W.mstride;
-    W.win = W.cnt + W.mstride;
+    W.win = PROG ? W.cnt + W.mstride : W.mbox;
     W.occ = W.win + 64 * WIN;
     W.bvq = W.occ + ((kp.S * kp.spuck + 3) & ~3);
     W.track = false;
@@ -1194,8 +1202,9 @@ __device__ __forceinline__ int wave_setup(Wave<PPL, BITS> &W, const KParams &kp,
     W.nblk = W.napply = 0;
     W.tmark = __builtin_amdgcn_s_memtime();
 #endif
-    for (int i = W.lane; i < W.mstride; i += 64)
-        W.cnt[i] = 0;
+    if (PROG)
+        for (int i = W.lane; i < W.mstride; i += 64)
+            W.cnt[i] = 0;
 #pragma unroll
     for (int k = 0; k < PPL; ++k) {
         const int p = W.lane + 64 * k;
@@ -1448,6 +1457,55 @@ __device__ __forceinline__ void acf_after(const KParams &kp, int r)
     }
 }
 
+// The species counts per site type of a run that records samples, kept up to
+// date by the writes from here on.
+template <int PPL, int BITS>
+__device__ __forceinline__ void count_species(Wave<PPL, BITS> &W)
+{
+    W.track = true;
+    const int no = W.S * W.d.spuck;
+    for (int i = W.lane; i < no; i += 64)
+        W.occ[i] = 0;
+    wave_sync();
+    for (int s = W.lane; s < W.d.V; s += 64) {
+        const int q = W.lat.get(s);
+        if (q >= 0 && q < W.S)
+            atomicAdd(&W.occ[q * W.d.spuck + (s - divm(s, W.ms) * W.d.spuck)], 1);
+    }
+    wave_sync();
+}
+
+// The end of a run: the last record, then the replica's state back to HBM.
+template <int PPL, int BITS, bool LDS_LAT>
+__device__ __forceinline__ void steps_end(Wave<PPL, BITS> &W, const KParams &kp, int r, int slot, double t,
+                                          double dt_last, long long ks, unsigned long long ctr, int st,
+                                          long long done)
+{
+    if (W.track)
+        write_record<PPL, BITS>(W, kp, slot, done == 0 ? 0 : (done - 1) / kp.sample_every, t, dt_last, ks, st);
+    wave_store<PPL, BITS, LDS_LAT>(W, kp, r, true);
+#if KMCG_PHASES
+    PH_MARK(W, 4);
+    if (W.lane == 0 && kp.phase) {
+        for (int i = 0; i < 5; ++i)
+            kp.phase[PHASE_W * r + i] += W.tph[i];
+        kp.phase[PHASE_W * r + 5] += (unsigned long long)done;
+        kp.phase[PHASE_W * r + 6] += W.nblk;
+        kp.phase[PHASE_W * r + 7] += W.napply;
+    }
+#endif
+    if (W.lane == 0) {
+        kp.ktime[r] = t;
+        kp.kdt[r] = dt_last;
+        kp.kstep[r] = ks;
+        kp.rngctr[r] = ctr;
+        kp.status[r] = st;
+        kp.executed[slot] = done;
+        if (kp.budget)
+            kp.budget[slot] -= done;
+    }
+}
+
 // OV (one process slot per lane, no tracking): the next step's accumulate
 // and search run during the replay's HBM reads.  It shortens a trajectory's
 // chain of dependent steps and adds instructions, so it pays where few
@@ -1469,20 +1527,8 @@ __device__ __forceinline__ void steps_loop(const KParams &kp, unsigned char *sme
         n = min(n, kp.budget[slot]);
     if (st0 != ST_OK)
         n = 0;
-    if (kp.srec) {
-        // species counts per site type, then kept up to date by the writes
-        W.track = true;
-        const int no = kp.S * W.d.spuck;
-        for (int i = lane; i < no; i += 64)
-            W.occ[i] = 0;
-        wave_sync();
-        for (int s = lane; s < W.d.V; s += 64) {
-            const int q = W.lat.get(s);
-            if (q >= 0 && q < W.S)
-                atomicAdd(&W.occ[q * W.d.spuck + (s - divm(s, W.ms) * W.d.spuck)], 1);
-        }
-        wave_sync();
-    }
+    if (kp.srec)
+        count_species<PPL, BITS>(W);
     double t = kp.ktime[r], dt_last = kp.kdt[r];
     long long ks = kp.kstep[r];
     unsigned long long ctr = kp.rngctr[r];
@@ -1630,29 +1676,7 @@ __device__ __forceinline__ void steps_loop(const KParams &kp, unsigned char *sme
             rec_idx += 1;
         }
     }
-    if (W.track)
-        write_record<PPL, BITS>(W, kp, slot, done == 0 ? 0 : (done - 1) / kp.sample_every, t, dt_last, ks, st);
-    wave_store<PPL, BITS, LDS_LAT>(W, kp, r, true);
-#if KMCG_PHASES
-    PH_MARK(W, 4);
-    if (lane == 0 && kp.phase) {
-        for (int i = 0; i < 5; ++i)
-            kp.phase[PHASE_W * r + i] += W.tph[i];
-        kp.phase[PHASE_W * r + 5] += (unsigned long long)done;
-        kp.phase[PHASE_W * r + 6] += W.nblk;
-        kp.phase[PHASE_W * r + 7] += W.napply;
-    }
-#endif
-    if (lane == 0) {
-        kp.ktime[r] = t;
-        kp.kdt[r] = dt_last;
-        kp.kstep[r] = ks;
-        kp.rngctr[r] = ctr;
-        kp.status[r] = st;
-        kp.executed[slot] = done;
-        if (kp.budget)
-            kp.budget[slot] -= done;
-    }
+    steps_end<PPL, BITS, LDS_LAT>(W, kp, r, slot, t, dt_last, ks, ctr, st, done);
 }
 
 template <int PPL, int BITS, bool LDS_LAT, bool MSD, bool OV = false>
@@ -1671,6 +1695,8 @@ __global__ __launch_bounds__(64 * MAX_WPG) __attribute__((amdgpu_waves_per_eu(4)
     extern __shared__ __align__(16) unsigned char smem[];
     steps_loop<PPL, BITS, LDS_LAT, false, false, true>(kp, smem);
 }
+
+#include "kmcg_fused.hip"
 
 // touchups, run_proc_nr, get_next_kmc_step (one replica per wave)
 template <int PPL, int BITS, bool LDS_LAT>
@@ -2071,6 +2097,11 @@ struct kmcg_model {
     int mrows = 1;       // mailbox rows per wave
     int merged = 0;      // bit 0: one apply per step; bit 1: lat_int groups in one pass
     int off_seg = 0, off_proc = 0, off_touch = 0, off_nli = 0, off_init = 0, off_nlitab = 0;
+    // the fused step loop's records (kmcg_fused.hip; empty: not for this model)
+    std::vector<int> fz;
+    int fz_nc = 0;       // condition words per record (1 or 5)
+    int fz_nch = 1;      // chunks of 64 records per process
+    int fz_moff = 0;     // largest offset component of the records
     // a species id a lattice site may hold: 0..S-1, or the null species S of
     // a multi-layer model (sites of layers that are not populated)
     bool species_ok(int v) const { return (v >= 0 && v < S) || (nullsp >= 0 && v == nullsp); }
@@ -2096,6 +2127,7 @@ struct kmcg_batch {
     long long lat_total = 0, avail_total = 0;
     // device buffers
     int *prog = nullptr;
+    int *fz = nullptr;                  // fused records (behind prog)
     int4 *dims = nullptr;
     long long *lat_off_d = nullptr, *avail_off_d = nullptr;
     unsigned *seed = nullptr, *strm = nullptr;
@@ -2145,6 +2177,7 @@ struct kmcg_batch {
     // 1 per replica whose lists match its lattice (set by kmcg_init and
     // kmcg_set_config, cleared by kmcg_replace_species and kmcg_set_state)
     int *lists_ok = nullptr;
+    std::vector<unsigned char> lists_ok_h;   // the same on the host
     // displacement tracking (kmcg_msd_*): allocated by the first kmcg_msd_init
     int *msd_hop = nullptr;
     double *msd_d = nullptr;
@@ -2201,6 +2234,148 @@ void assign_rounds(SegH &sg, const std::vector<std::vector<int>> &group_procs, i
     }
 }
 
+// The fused step loop's records of a single-layer local_smart model: per
+// process the list updates of its routines as one list (see kmcg_fused.hip),
+// with every condition on a site whose species the process's own conditions
+// fix resolved here.  Leaves m->fz empty when the model does not qualify:
+// more than 64 processes, several layers, a write or a deletion whose
+// conditions are not known, more than five open conditions per update.
+void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector<std::vector<int>> &proc_items,
+                 const std::vector<std::vector<int>> &pconds, const std::vector<bool> &have)
+{
+    typedef std::array<int, 4> Co;                       // dx, dy, dz, site type
+    struct Up {
+        int proc;
+        bool del;
+        Co at;
+        std::vector<std::pair<Co, int>> conds;
+    };
+    if (m->backend != 0 || m->nullsp >= 0 || m->P > 64 || m->spuck > 32)
+        return;
+    const int code = m->lattice_bits() == 2 ? 1 : 0;     // species code of the records
+    std::vector<std::vector<Up>> ups(m->P);
+    std::vector<std::map<Co, std::pair<int, int>>> writes(m->P);    // old, new
+    size_t maxc = 0, most = 0;
+    int mo = 0;
+    auto reach = [&](const Co &c) {
+        for (int k = 0; k < 3; ++k)
+            mo = std::max(mo, std::abs(c[k]));
+    };
+    for (int p = 1; p <= m->P; ++p) {
+        if (!have[p])
+            return;
+        std::map<Co, int> known;
+        for (size_t c = 0; c + 5 <= pconds[p].size(); c += 5) {
+            const Co at = {pconds[p][c], pconds[p][c + 1], pconds[p][c + 2], pconds[p][c + 3]};
+            if (!known.emplace(at, pconds[p][c + 4]).second)
+                return;                                  // two conditions on one site
+            reach(at);
+        }
+        std::vector<Up> &list = ups[p - 1];
+        for (size_t i = 0; i < proc_items[p - 1].size(); i += 4) {
+            const int *it = &proc_items[p - 1][i];
+            const SegH &sg = segs[it[0]];
+            if (sg.writes.size() != 6)
+                return;
+            auto shift = [&](int dx, int dy, int dz, int n) { return Co{it[1] + dx, it[2] + dy, it[3] + dz, n}; };
+            const Co wc = shift(sg.writes[0], sg.writes[1], sg.writes[2], sg.writes[3]);
+            const auto kn = known.find(wc);
+            if (kn == known.end() || sg.writes[4] != 1 << kn->second)
+                return;                                  // the write's old species is open
+            bool written = false;
+            const size_t seg0 = list.size();
+            auto do_write = [&]() {
+                const auto w = writes[p - 1].emplace(wc, std::make_pair(kn->second, sg.writes[5]));
+                w.first->second.second = sg.writes[5];
+                kn->second = sg.writes[5];
+                written = true;
+            };
+            for (const OpH &op : sg.ops) {
+                const bool del = op.kind == OP_DEL_IF;
+                if (!del && !written)
+                    do_write();          // additions follow the deletions and see the write
+                if (del && (written || op.conds.empty()))
+                    return;
+                Up u{op.arg, del, shift(op.dx, op.dy, op.dz, op.n), {}};
+                bool can = true;
+                for (size_t c = 0; c + 5 <= op.conds.size() && can; c += 5) {
+                    const Co at = shift(op.conds[c], op.conds[c + 1], op.conds[c + 2], op.conds[c + 3]);
+                    const std::pair<Co, int> cd = {at, op.conds[c + 4]};
+                    const auto k = known.find(at);
+                    if (k != known.end())
+                        can = k->second == cd.second;
+                    else if (std::find(u.conds.begin(), u.conds.end(), cd) == u.conds.end())
+                        u.conds.push_back(cd);
+                }
+                if (!can)
+                    continue;
+                // one routine names an update once
+                for (size_t v = seg0; v < list.size(); ++v)
+                    if (list[v].proc == u.proc && list[v].del == u.del && list[v].at == u.at)
+                        return;
+                maxc = std::max(maxc, u.conds.size());
+                reach(u.at);
+                for (const auto &c : u.conds)
+                    reach(c.first);
+                list.push_back(u);
+            }
+            if (!written)
+                do_write();
+            reach(wc);
+        }
+        std::stable_sort(list.begin(), list.end(), [](const Up &a, const Up &b) { return a.proc < b.proc; });
+        most = std::max(most, list.size());
+        if (writes[p - 1].size() > 64)
+            return;
+    }
+    const int nch = std::max(1, (int)((most + 63) / 64));
+    const int nc = maxc <= 1 && nch == 1 ? 1 : 5;
+    const int rw = nc == 1 ? 4 : 8;
+    if (maxc > 5 || nch > 31 || mo > 31 || (size_t)m->P * nch * 64 * rw > (size_t)1 << 20)
+        return;
+    auto word = [&](const Co &c) {
+        return (c[0] & 127) | (c[1] & 127) << 7 | (c[2] & 127) << 14 | (c[3] - 1) << 21;
+    };
+    std::vector<int> fz((size_t)m->P * nch * 64 * rw, 0);
+    for (int p = 0; p < m->P; ++p) {
+        const std::vector<Up> &list = ups[p];
+        const int own_ch = std::max(1, (int)((list.size() + 63) / 64));
+        for (int ch = 0; ch < nch; ++ch) {
+            int *blk = &fz[((size_t)p * nch + ch) * 64 * rw];
+            for (int l = 0; l < 64; ++l) {
+                int *q = blk + l * rw;
+                // the run of process l + 1 in this chunk
+                int first = 0, len = 0;
+                for (int j = 0; j < 64 && 64 * ch + j < (int)list.size(); ++j)
+                    if (list[64 * ch + j].proc == l + 1) {
+                        if (!len)
+                            first = j;
+                        ++len;
+                    }
+                if (len > 31)
+                    return;
+                q[0] = (int)((unsigned)own_ch << 27) | first << 8 | len << 16;
+                if (64 * ch + l < (int)list.size()) {
+                    const Up &u = list[64 * ch + l];
+                    q[0] |= (u.proc - 1) | (u.del ? 1 << 6 : 0) | 1 << 7 | (int)u.conds.size() << 24;
+                    q[1] = word(u.at);
+                    for (size_t c = 0; c < u.conds.size(); ++c)
+                        q[2 + c] = word(u.conds[c].first) | (u.conds[c].second + code) << 26;
+                }
+                if (ch == 0 && l < (int)writes[p].size()) {
+                    auto w = writes[p].begin();
+                    std::advance(w, l);
+                    q[rw - 1] = word(w->first) | w->second.first << 26 | (int)((unsigned)w->second.second << 29);
+                }
+            }
+        }
+    }
+    m->fz.swap(fz);
+    m->fz_nc = nc;
+    m->fz_nch = nch;
+    m->fz_moff = mo;
+}
+
 int build_prog(kmcg_model *m)
 {
     const std::vector<int> &b = m->blob;
@@ -2233,6 +2408,10 @@ int build_prog(kmcg_model *m)
         std::vector<int> touchup;
         std::vector<std::vector<int>> group_procs;
         std::vector<std::vector<int>> nli_nodes;            // per group, relative offsets
+        // per local_smart process: its conditions, relative to the cell of
+        // its executing site, and whether they are known
+        std::vector<std::vector<int>> pconds(m->P + 1);
+        std::vector<bool> have(m->P + 1, false);
         if (m->backend == 0) {
             const int nrt = W(10), rtab = W(11);
             for (int r = 0; r < nrt; ++r) {
@@ -2273,8 +2452,6 @@ int build_prog(kmcg_model *m)
                 touchup.push_back(W(W(12) + n));
             // every process's conditions, relative to its executing site's
             // cell: the enable of the touchup routine of that site type
-            std::vector<std::vector<int>> pconds(m->P + 1);
-            std::vector<bool> have(m->P + 1, false);
             for (int n = 0; n < m->spuck; ++n) {
                 const int t = touchup[n];
                 if (t < 0 || t >= (int)segs.size())
@@ -2712,6 +2889,7 @@ int build_prog(kmcg_model *m)
         pg.insert(pg.end(), {0, 0, 0, 0});   // padding: condition words are read four at a time
         if (pg.size() * sizeof(int) > 64 * 1024)
             return fail(KMCG_EUNSUPPORTED, "op program larger than 64 KiB");
+        build_fused(m, segs, proc_items, pconds, have);
     } catch (const std::exception &e) {
         return fail(KMCG_EINVAL, std::string("malformed model blob: ") + e.what());
     }
@@ -2773,11 +2951,13 @@ struct Shape {
     bool lds_lat;
     bool ov;           // the step kernel's overlapped form
     bool li;           // the step kernel's one-pass lat_int form
+    bool fz;           // the fused step loop, with fz_nc condition words per record
+    int fz_nc;
     int wpg, grid;
     size_t lds;
 };
 
-Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wpg)
+Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wpg, bool steps = false)
 {
     long long maxlb = 0;
     for (int i = 0; i < n; ++i)
@@ -2792,8 +2972,9 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
     const size_t mbox = ((size_t)(b->m->mrows + 1) * 64 * ppl_of(b->m->P) + 64 * WIN + occ + bvq) * sizeof(int);
     const size_t prog = (size_t)kp.prog_lds;
     s.lds_lat = b->lds_mode == 0 ? false : (prog + (size_t)maxlb + mbox <= (size_t)b->max_lds);
-    const size_t per_wave = (s.lds_lat ? (size_t)maxlb : 0) + mbox;
+    size_t per_wave = (s.lds_lat ? (size_t)maxlb : 0) + mbox;
     s.wpg = std::max(1, std::min(max_wpg, std::min(MAX_WPG, n)));
+    s.fz_nc = 0;
     // automatic: local_smart runs with at most two replica-waves per SIMD
     // (four SIMDs per CU) and a prefix chain long enough to hide (more than
     // 16 processes; RuO2's 36 gain, ZGB's 7 lose); lat_int runs the
@@ -2801,10 +2982,33 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
     // faster than the overlap
     s.ov = b->ov_mode == 1 ||
            (b->ov_mode == -1 && b->m->backend == 0 && b->m->P > 16 && (long long)n <= 8LL * b->n_cu);
-    while (s.wpg > 1 && prog + s.wpg * per_wave > (size_t)b->max_lds)
+    size_t shared = prog;
+    // the fused step loop: the lists of every replica follow its lattice, no
+    // two offsets of the records meet on a lattice this small, the lattice
+    // fits LDS, and no other form was asked for
+    const size_t fz_wave = (size_t)maxlb + (64 * WIN + occ) * sizeof(int);
+    s.fz = steps && !b->m->fz.empty() && b->ov_mode == -1 && b->lds_mode != 0 && fz_wave <= (size_t)b->max_lds;
+    const int least = 2 * b->m->fz_moff + 1;
+    for (int i = 0; i < n && s.fz; ++i) {
+        const int r = ids[i];
+        s.fz = b->lists_ok_h[r] && b->X[r] >= least && (b->m->dim < 2 || b->Y[r] >= least) &&
+               (b->m->dim < 3 || b->Z[r] >= least) && b->V[r] < (1 << 24) - 2;
+    }
+    if (s.fz) {
+        s.lds_lat = true;
+        s.ov = s.li = false;
+        per_wave = fz_wave;
+        shared = 0;
+        kp.prog_lds = 0;
+        kp.moff = b->m->fz_moff;
+        kp.fz_recs = b->fz;
+        kp.fz_nch = b->m->fz_nch;
+        s.fz_nc = b->m->fz_nc;
+    }
+    while (s.wpg > 1 && shared + s.wpg * per_wave > (size_t)b->max_lds)
         s.wpg -= 1;
     s.grid = (n + s.wpg - 1) / s.wpg;
-    s.lds = prog + s.wpg * per_wave;
+    s.lds = shared + s.wpg * per_wave;
     kp.lat_lds = s.lds_lat ? (int)maxlb : 0;
     kp.wave_lds = (int)per_wave;
     kp.wpg = s.wpg;
@@ -2816,7 +3020,19 @@ template <int PPL, int BITS>
 hipError_t launch_t(bool steps, const Shape &s, hipStream_t st, const KParams &kp)
 {
     const dim3 grid(s.grid), block(64 * s.wpg);
-    if (steps && kp.msd_hop) {
+    if (steps && PPL == 1 && s.fz) {
+        if (kp.fz_nch == 1 && s.fz_nc == 1) {
+            if (kp.msd_hop)
+                hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, 1, true>), grid, block, s.lds, st, kp);
+            else
+                hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, 1, false>), grid, block, s.lds, st, kp);
+        } else {
+            if (kp.msd_hop)
+                hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, 5, true>), grid, block, s.lds, st, kp);
+            else
+                hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, 5, false>), grid, block, s.lds, st, kp);
+        }
+    } else if (steps && kp.msd_hop) {
         if (s.lds_lat)
             hipLaunchKernelGGL((kmc_steps_kernel<PPL, BITS, true, true>), grid, block, s.lds, st, kp);
         else
@@ -3003,6 +3219,16 @@ int kmcg_model_forms(const kmcg_model *m, int32_t *li)
     return KMCG_OK;
 }
 
+int kmcg_model_fused(const kmcg_model *m, int32_t *info4, int32_t *words)
+{
+    if (!m || !info4)
+        return fail(KMCG_EINVAL, "null argument");
+    info4[0] = (int32_t)m->fz.size(); info4[1] = m->fz_nc; info4[2] = m->fz_nch; info4[3] = m->fz_moff;
+    if (words && !m->fz.empty())
+        memcpy(words, m->fz.data(), m->fz.size() * sizeof(int));
+    return KMCG_OK;
+}
+
 static int sizes_ok(const kmcg_model *m, int32_t n, const int32_t *sizes)
 {
     if (!m || n < 1 || !sizes)
@@ -3128,7 +3354,11 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     if (hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess)
         return bail(fail(KMCG_EHIP, "event creation failed"));
     const long long P = m->P;
-    BALLOC(b->prog, m->prog.size());
+    // the op program, then the fused records (16-byte aligned)
+    const size_t fz_at = (m->prog.size() + 3) & ~(size_t)3;
+    BALLOC(b->prog, fz_at + m->fz.size());
+    b->fz = b->prog + fz_at;
+    b->lists_ok_h.assign(n, 0);
     BALLOC(b->dims, n);
     BALLOC(b->lat_off_d, n);
     BALLOC(b->avail_off_d, n);
@@ -3164,7 +3394,10 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     auto H2D = [&](void *d, const void *h, size_t bytes) {
         return hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, b->stream) == hipSuccess;
     };
-    if (!H2D(b->prog, m->prog.data(), m->prog.size() * sizeof(int)) ||
+    std::vector<int> progs(m->prog);
+    progs.resize(fz_at, 0);
+    progs.insert(progs.end(), m->fz.begin(), m->fz.end());
+    if (!H2D(b->prog, progs.data(), progs.size() * sizeof(int)) ||
         !H2D(b->dims, dims.data(), n * sizeof(int4)) ||
         !H2D(b->lat_off_d, b->lat_off.data(), n * sizeof(long long)) ||
         !H2D(b->avail_off_d, b->avail_off.data(), n * sizeof(long long)))
@@ -3233,6 +3466,7 @@ namespace {
 int set_lists_ok(kmcg_batch *b, int r0, int n, int v)
 {
     std::vector<int> f(n, v);
+    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)v);
     return copy_in(b, b->lists_ok + r0, f.data(), (size_t)n);
 }
 } // namespace
@@ -3403,7 +3637,7 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     if (budget)
         memcpy(b->h_budget, budget, n * sizeof(long long));
     KParams kp = make_params(b);
-    const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg);
+    const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg, true);
     kp.nsteps = steps;
     kp.budget = budget ? b->budget : nullptr;
     if (track & 4) {
@@ -3473,7 +3707,8 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
         HIPCHK(enqueue(true));
     } else {
         // the key: every value a captured node holds
-        const int flags[7] = {n, budget ? 1 : 0, records ? 1 : 0, s.lds_lat ? 1 : 0, s.wpg, s.grid, s.ov ? 1 : 0};
+        const int flags[8] = {n, budget ? 1 : 0, records ? 1 : 0, s.lds_lat ? 1 : 0, s.wpg, s.grid, s.ov ? 1 : 0,
+                              s.fz ? 1 : 0};
         const size_t lds = s.lds;
         const void *hs = b->h_srec;
         std::vector<unsigned char> key(sizeof kp + sizeof flags + sizeof lds + sizeof hs + sizeof cnt);

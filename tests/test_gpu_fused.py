@@ -1,0 +1,54 @@
+"""The fused step loop against the oracle where its rules have edges: the
+smallest extents it takes and the largest it leaves to the generic loop, one
+and several chunks of records per process, the refill of the uniforms after
+64 steps, a stopped replica in the launch."""
+import os
+
+import numpy as np
+import pytest
+
+from kmos_amd import workloads as W
+from kmos_amd.compiler import compile_model
+from kmos_amd.model import load_project
+from paritylib import compare_state, oracle_replica, random_config
+from test_fused_records import GOLDEN, fused_records
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # one chunk of one-condition records; several chunks of wide ones
+    ("zgb", W.zgb_project), ("ruo2", W.ruo2_project), ("pairwise", W.pairwise_project),
+    ("ab_ini", lambda: load_project(os.path.join(GOLDEN, "ab_model.ini"))),
+    ("quickstart", W.quickstart_project),
+]
+
+
+@pytest.mark.parametrize("small", [False, True], ids=["fused", "below_the_extent"])
+@pytest.mark.parametrize("name,factory", CASES, ids=[c[0] for c in CASES])
+def test_edges_match_oracle(engine, oracle, name, factory, small):
+    pt = factory()
+    cm = compile_model(pt, "local_smart")
+    rec, _, reach = fused_records(cm)
+    assert rec is not None
+    m = 2 * reach + 1
+    sizes = [(m, m), (m, m + 3), (m + 4, m), (31, 17), (64, 33)]
+    if small and reach > 1:
+        sizes.append((m - 1, m + 2))       # its offsets meet: the whole launch runs the generic loop
+    g = np.random.default_rng(17)
+    n = len(sizes)
+    rates = 10.0 ** g.uniform(-1, 3, (n, cm.nr_of_proc))
+    rates[0] = 0.0                          # no process possible: stops at once
+    seeds = g.integers(1 << 31, size=n).astype(np.uint32)
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init(seeds, np.arange(n, dtype=np.uint32))
+    b.set_rates(rates)
+    configs = [random_config(pt, int(v), g) for v in b.volumes]
+    b.set_config(configs)
+    orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), i, rates[i], configs[i]) for i, s in enumerate(sizes)]
+    for steps in (1, 2, 61, 1, 140, 795):
+        b.run(steps)
+        for i, o in enumerate(orcs):
+            o.run(steps)
+            compare_state(b, i, o, where="%s %s" % (name, sizes[i]))
+    assert b.scalars(0)[4] == 1 and (b.check_lists() == 0).all()
+    b.close()
