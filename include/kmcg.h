@@ -71,13 +71,13 @@ int kmcg_model_info(const kmcg_model *m, int32_t *info5);
  * reference (a profiling aid). */
 int kmcg_model_forms(const kmcg_model *m, int32_t *li);
 
-/* The fused step loop's records of a single-layer local_smart model (per
- * process the list updates of its routines as one flat list; layout in
- * kmos_amd/csrc/kmcg_fused.hip): info4 = words (0: the model has none),
- * condition words per record, chunks of 64 records per process, largest
- * offset; `words` may be NULL.  No counterpart in the reference (a test
- * aid). */
-int kmcg_model_fused(const kmcg_model *m, int32_t *info4, int32_t *words);
+/* The fused step loop's records (per process the list updates of its
+ * routines as one flat list; layout in kmos_amd/csrc/kmcg_fused.hip): info6
+ * = words in all (0: the model has none), form (1 one open condition, 4
+ * four, 2 lat_int), chunks of 64 records per process, largest offset, word
+ * offset and bytes of the lat_int tables; `words` may be NULL.  No
+ * counterpart in the reference (a test aid). */
+int kmcg_model_fused(const kmcg_model *m, int32_t *info6, int32_t *words);
 
 /* Device bytes a batch of n replicas of sizes[n][3] needs. */
 int kmcg_batch_footprint(const kmcg_model *m, int32_t n, const int32_t *sizes, int64_t *bytes);

@@ -126,6 +126,7 @@ struct KParams {
     int off_seg, off_proc, off_touch, off_nli, off_nlitab;
     const int *fz_recs;            // records of the fused step loop (kmcg_fused.hip)
     int fz_nch;                    // chunks of 64 records per process
+    int fz_tab_off;                // lat_int: word offset of the groups' tables behind the records
     double *srec;                  // in-loop sample records (or null)
     int sample_every, srec_cap, srec_width;
     int mode;                      // misc kernel mode

@@ -11,28 +11,30 @@ from kmos_amd import workloads as W
 from kmos_amd.compiler import compile_model
 from kmos_amd.model import load_project
 from paritylib import compare_state, oracle_replica, random_config
-from test_fused_records import GOLDEN, fused_records
+from test_fused_records import GOLDEN, Records
 
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # one chunk of one-condition records; several chunks of wide ones
-    ("zgb", W.zgb_project), ("ruo2", W.ruo2_project), ("pairwise", W.pairwise_project),
-    ("ab_ini", lambda: load_project(os.path.join(GOLDEN, "ab_model.ini"))),
-    ("quickstart", W.quickstart_project),
+    # one chunk of one-condition records, several chunks of wide ones, lat_int
+    ("quickstart", W.quickstart_project, "local_smart"), ("zgb", W.zgb_project, "local_smart"),
+    ("ruo2", W.ruo2_project, "local_smart"), ("pairwise", W.pairwise_project, "local_smart"),
+    ("ab_ini", lambda: load_project(os.path.join(GOLDEN, "ab_model.ini")), "local_smart"),
+    ("zgb_li", W.zgb_project, "lat_int"), ("ruo2_li", W.ruo2_project, "lat_int"),
+    ("pairwise_li", W.pairwise_project, "lat_int"),
 ]
 
 
 @pytest.mark.parametrize("small", [False, True], ids=["fused", "below_the_extent"])
-@pytest.mark.parametrize("name,factory", CASES, ids=[c[0] for c in CASES])
-def test_edges_match_oracle(engine, oracle, name, factory, small):
+@pytest.mark.parametrize("name,factory,backend", CASES, ids=[c[0] for c in CASES])
+def test_edges_match_oracle(engine, oracle, name, factory, backend, small):
     pt = factory()
-    cm = compile_model(pt, "local_smart")
-    rec, _, reach = fused_records(cm)
-    assert rec is not None
-    m = 2 * reach + 1
+    cm = compile_model(pt, backend)
+    R = Records(cm)
+    assert R.have
+    m = 2 * R.reach + 1
     sizes = [(m, m), (m, m + 3), (m + 4, m), (31, 17), (64, 33)]
-    if small and reach > 1:
+    if small and R.reach > 1:
         sizes.append((m - 1, m + 2))       # its offsets meet: the whole launch runs the generic loop
     g = np.random.default_rng(17)
     n = len(sizes)
