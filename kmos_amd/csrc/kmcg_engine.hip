@@ -1917,7 +1917,7 @@ __global__ __launch_bounds__(256) void kmc_init_lists_kernel(KParams kp)
 // The debug check of one replica's lists (kmcg_check_lists), one block per
 // (replica, process): the invariant add_proc/del_proc keep (base.mpy:
 // 211-301: sites[1..nr] distinct sites of the process's executing site type
-// with back[site] = position, every other slot and back entry 0), and the
+// with back[site] = position, every other back entry 0), and the
 // registered set against a scan of every cell with the process's
 // conditions (local_smart: the touchup's if-tree conditions; lat_int: the
 // nli case tree), the set kmc_init_lists_kernel builds.  Adds the number of
@@ -1950,10 +1950,9 @@ __global__ __launch_bounds__(256) void kmc_check_lists_kernel(KParams kp, int *b
     int nbad = (nr < 0 || nr > V || (never && nr != 0)) ? 1 : 0;
     for (int k = threadIdx.x + 1; k <= V; k += blockDim.x) {
         const int site = sp[k];
+        // (what the slots past the end hold means nothing)
         if (k <= nr)
             nbad += (site < 1 || site > V || bp[site] != k || (site - 1) % d.spuck + 1 != n_exec) ? 1 : 0;
-        else
-            nbad += site != 0 ? 1 : 0;
         const int back = bp[k];
         if (back != 0)
             nbad += (back < 0 || back > nr || sp[back] != k) ? 1 : 0;
@@ -3169,7 +3168,9 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
     const int least = 2 * b->m->fz_moff + 1;
     for (int i = 0; i < n && s.fz; ++i) {
         const int r = ids[i];
-        s.fz = b->lists_ok_h[r] && b->X[r] >= least && (b->m->dim < 2 || b->Y[r] >= least);
+        s.fz = b->lists_ok_h[r] && b->X[r] >= least && (b->m->dim < 2 || b->Y[r] >= least) &&
+               b->X[r] * b->m->spuck > 1 &&
+               (long long)b->V[r] * b->X[r] * b->m->spuck < (1LL << 32);    // rows by one multiply-high
     }
     if (s.fz) {
         s.lds_lat = true;
@@ -3199,17 +3200,20 @@ hipError_t launch_t(bool steps, const Shape &s, hipStream_t st, const KParams &k
 {
     const dim3 grid(s.grid), block(64 * s.wpg);
     if (steps && PPL == 1 && s.fz) {
-        switch (2 * s.fz_form + (kp.msd_hop ? 1 : 0)) {
-#define FZ_LAUNCH(FORM, MSD)                                                                                    \
-    case 2 * FORM + MSD:                                                                                        \
-        hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, FORM, MSD != 0>), grid, block, s.lds, st, kp);             \
+        switch (4 * s.fz_form + (kp.msd_hop ? FZ_MSD : kp.srec ? FZ_REC : FZ_PLAIN)) {
+#define FZ_LAUNCH(FORM, MODE)                                                                                  \
+    case 4 * FORM + MODE:                                                                                      \
+        hipLaunchKernelGGL((kmc_steps_kernel_fz<BITS, FORM, MODE>), grid, block, s.lds, st, kp);               \
         break;
-            FZ_LAUNCH(FZ_1, 0)
-            FZ_LAUNCH(FZ_1, 1)
-            FZ_LAUNCH(FZ_4, 0)
-            FZ_LAUNCH(FZ_4, 1)
-            FZ_LAUNCH(FZ_LI, 0)
-            FZ_LAUNCH(FZ_LI, 1)
+            FZ_LAUNCH(FZ_1, FZ_PLAIN)
+            FZ_LAUNCH(FZ_1, FZ_REC)
+            FZ_LAUNCH(FZ_1, FZ_MSD)
+            FZ_LAUNCH(FZ_4, FZ_PLAIN)
+            FZ_LAUNCH(FZ_4, FZ_REC)
+            FZ_LAUNCH(FZ_4, FZ_MSD)
+            FZ_LAUNCH(FZ_LI, FZ_PLAIN)
+            FZ_LAUNCH(FZ_LI, FZ_REC)
+            FZ_LAUNCH(FZ_LI, FZ_MSD)
 #undef FZ_LAUNCH
         }
     } else if (steps && kp.msd_hop) {
@@ -3509,6 +3513,9 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
         b->V[i] = b->X[i] * b->Y[i] * b->Z[i] * m->spuck;
         dims[i] = make_int4(b->X[i], b->Y[i], b->Z[i], b->V[i]);
         b->lat_off[i] = b->lat_total;
+        // (leading words: a fused step reads four words up to a list's slot)
+        if (i == 0)
+            b->avail_total = 64;
         b->lat_total += lattice_bytes(b->V[i], b->bits);
         b->avail_off[i] = b->avail_total;
         // 2 x P x (V+1) words, rounded to 64 words so replicas start on 256 B
@@ -4228,12 +4235,17 @@ int kmcg_get_avail(kmcg_batch *b, int32_t r, int32_t *sites, int32_t *back)
     if (rc)
         return rc;
     const long long P = b->m->P, V1 = b->V[r] + 1;
-    std::vector<int> blk(2 * P * V1);
+    std::vector<int> blk(2 * P * V1), nr(P);
     rc = copy_out(b, blk.data(), b->avail_pool + b->avail_off[r], blk.size());
+    if (!rc)
+        rc = copy_out(b, nr.data(), b->nr + (long long)r * P, nr.size());
     if (rc)
         return rc;
     for (long long p = 0; p < P; ++p) {
-        std::memcpy(sites + p * (V1 - 1), blk.data() + p * V1 + 1, (V1 - 1) * sizeof(int));
+        // slots past the end read 0; on the device they keep what they held
+        const long long used = std::min<long long>(std::max(nr[p], 0), V1 - 1);
+        std::memcpy(sites + p * (V1 - 1), blk.data() + p * V1 + 1, used * sizeof(int));
+        std::memset(sites + p * (V1 - 1) + used, 0, (V1 - 1 - used) * sizeof(int));
         std::memcpy(back + p * (V1 - 1), blk.data() + (P + p) * V1 + 1, (V1 - 1) * sizeof(int));
     }
     return KMCG_OK;

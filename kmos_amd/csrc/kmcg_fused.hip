@@ -34,10 +34,10 @@
 // register.
 //
 // Measured against the generic loops, per 1000 steps: ZGB 4096 x 128x128
-// 5.41 -> 2.73 ms, RuO2 mix of 2048 5.42 -> 3.06 ms, RuO2 lat_int, 300 odd
-// lattices 5.91 -> 2.25 ms, pairwise lat_int 512 x 256x256 4.48 -> 2.5 ms
-// (kernel); one RuO2 64x64 trajectory 3.8 -> 1.56 us per step; tracking on
-// the pairwise model (264 updates in five chunks) 14.1 -> 7.6 us per step.
+// 5.41 -> 2.38 ms, RuO2 mix of 2048 5.42 -> 2.65 ms, RuO2 lat_int, 300 odd
+// lattices 5.91 -> 1.79 ms, pairwise lat_int 512 x 256x256 4.48 -> 1.85 ms
+// (kernel); one RuO2 64x64 trajectory 3.8 -> 1.24 us per step; tracking on
+// the pairwise model (264 updates in five chunks) 14.1 -> 6.5 us per step.
 //
 // Record of one lane (RW words, 64 lanes per chunk, the chunks of a process
 // in turn):
@@ -115,72 +115,102 @@ __device__ __forceinline__ int fz_code(const unsigned char *lat, int s)
     return (int)__builtin_amdgcn_ubfe(w, (unsigned)s << 1, 2);
 }
 
-// Does this lane's update take place (FZ_1, FZ_4)?  s: its site.
-template <int BITS, int FORM, bool IN>
-__device__ __forceinline__ bool fz_eval(const unsigned char *lat, const FzAt &p, const FzRec<FORM> &q, int &s, int &ws)
+// species old -> v at site s by exclusive or, lanes with old == v on a spare
+// word of their own (no divergent region); other lanes may write other
+// sites of the same word
+template <int BITS>
+__device__ __forceinline__ void fz_write(unsigned char *lat, unsigned *spare, int s, int old, int v)
 {
-    constexpr int NC = FORM == FZ_1 ? 1 : 4, C0 = FORM == FZ_1 ? 2 : 3;
-    int got[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-        got[c] = fz_code<BITS>(lat, fz_site<IN>(p, q.w[C0 + c]));
-    s = fz_site<IN>(p, q.site());
-    ws = fz_site<IN>(p, q.write_site());
-    if (FORM == FZ_1)
-        return got[0] == bf_u(q.w[0], 18, 4);
-    int all = got[0];
-#pragma unroll
-    for (int c = 1; c < NC; ++c)
-        all |= got[c] << (4 * c);
-    return all == (q.w[1] & 0xFFFF);
+    unsigned *w = (unsigned *)lat + ((unsigned)s >> (BITS == 8 ? 2 : 4));
+    const unsigned x = BITS == 8 ? (unsigned)(old ^ v) << ((s & 3) * 8)
+                                 : (unsigned)((old + 1) ^ (v + 1)) << ((s << 1) & 31);
+    atomicXor(old != v ? w : spare, x);
 }
 
-// The variants this lane's (group, cell) pair has before and after the
-// writes (FZ_LI; 0: none).
-template <int BITS, bool IN>
-__device__ __forceinline__ void fz_eval_li(const unsigned char *lat, const unsigned char *tab, const FzAt &p,
-                                           const FzRec<FZ_LI> &q, int &s, int &ws, int &pd, int &pa)
-{
-    int got[4];
+// What a lane's record names around the picked site: its update's site, the
+// site it writes, the sites it tests.  The plain form first, without a
+// branch; near the faces the sites are formed again, wrapped.
+template <int FORM>
+struct FzSites {
+    static constexpr int NC = FORM == FZ_1 ? 1 : 4;
+    int s, ws, cs[NC];
+    template <bool IN>
+    __device__ __forceinline__ void form(const FzAt &p, const FzRec<FORM> &q)
+    {
+        s = fz_site<IN>(p, q.site());
+        ws = fz_site<IN>(p, q.write_site());
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-        got[c] = fz_code<BITS>(lat, fz_site<IN>(p, bf_s(q.w[3 + c], 0, 12), bf_s(q.w[3 + c], 12, 7)));
-    s = fz_site<IN>(p, q.site());
-    ws = fz_site<IN>(p, q.write_site());
-    int idx = 0;
+        for (int c = 0; c < NC; ++c) {
+            const int w = q.w[FORM == FZ_1 ? 2 : 3 + c];
+            cs[c] = FORM == FZ_LI ? fz_site<IN>(p, bf_s(w, 0, 12), bf_s(w, 12, 7)) : fz_site<IN>(p, w);
+        }
+    }
+    // Does this lane's update take place (FZ_1, FZ_4)?
+    template <int BITS>
+    __device__ __forceinline__ bool holds(const unsigned char *lat, const FzRec<FORM> &q) const
+    {
+        int all = fz_code<BITS>(lat, cs[0]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-        idx = (int)__umul24(got[c], (unsigned)q.w[3 + c] >> 19) + idx;
-    pd = tab[(q.w[2] & 0xFFFF) + idx];
-    pa = tab[(int)((unsigned)q.w[2] >> 16) + idx];
-}
+        for (int c = 1; c < NC; ++c)
+            all |= fz_code<BITS>(lat, cs[c]) << (4 * c);
+        return all == (FORM == FZ_1 ? bf_u(q.w[0], 18, 4) : (q.w[1] & 0xFFFF));
+    }
+    // The variants this lane's (group, cell) pair has before and after the
+    // writes (FZ_LI; 0: none).
+    template <int BITS>
+    __device__ __forceinline__ void variants(const unsigned char *lat, const unsigned char *tab,
+                                             const FzRec<FORM> &q, int &pd, int &pa) const
+    {
+        int got[NC], idx = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            got[c] = fz_code<BITS>(lat, cs[c]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            idx = (int)__umul24(got[c], (unsigned)q.w[FORM == FZ_1 ? 0 : 3 + c] >> 19) + idx;
+        pd = tab[(q.w[2] & 0xFFFF) + idx];
+        pa = tab[(int)((unsigned)q.w[2] >> 16) + idx];
+    }
+};
+
+// A replica's lists through a buffer descriptor: a lane whose offset is
+// FZ_NONE lies outside it, so its load returns 0 and its store is dropped by
+// the hardware's range check.  An access of some lanes costs one select that
+// way (8 cycles of a lone wave) where a divergent region costs compare,
+// save, branch and restore (45), and the code stays straight, so that the
+// wait for the next step's site does not wait for the stores behind it.
+constexpr unsigned FZ_NONE = 0x80000000u;
+constexpr unsigned FZ_LEAD = 16;     // bytes before the first list (the pool's leading words or another list)
+typedef int int4v __attribute__((ext_vector_type(4)));
 
 // What one owner lane replays its updates with.
 struct FzList {
-    Rows L;
+    unsigned so, bo; // byte offsets of this lane's sites[p] and back[p]
     int V;
     int pk;          // the slot the next step's site is read from (-1: another lane's list)
     int patch;       // its new content when an update of this step writes it
     int err;
 };
 
-// Up to RB updates of this lane's list, in order (add_proc/del_proc,
-// base.mpy:211-301).  bits: this lane's entries, relative to lane a (LI: 16
-// deletions, then 16 additions); ent: the update lanes' sites (+ bit 31: it
-// deletes), bv0 their back-indices; t<j>: list slot nr - j.  Everything an
-// entry may need from an earlier one of the block (the slot it wrote and
-// the site it put there) stays in registers, so no entry waits for memory
-// or LDS; every change is written through in order.  Each entry is two
-// stores, and two more when the last site moves into a freed slot.  Every
-// lane takes part.
-template <int RB, bool LI>
-__device__ __forceinline__ void fz_replay(FzList &F, int &nr, unsigned &bits, int a, int ent, int bv0, int t0, int t1,
-                                          int t2, int t3)
+// Entries [I0, I0 + N) of a block of this lane's updates, in order
+// (add_proc/del_proc, base.mpy:211-301).  bits: this lane's entries,
+// relative to lane a (LI: 16 deletions, then 16 additions); ent: the update
+// lanes' sites (+ bit 31: it deletes), bv0 their back-indices; t<j>: list
+// slot nr0 - j.  Everything an entry may need from an earlier one of the
+// block (the slot it wrote and the site it put there) stays in registers,
+// so no entry waits for memory; every change is written through in order.
+// A lane without an entry changes nothing.  Every lane takes part.
+struct FzBlock {
+    int nr0, ws[4], wv[4];
+};
+template <int I0, int N, bool LI>
+__device__ __forceinline__ void fz_replay(__amdgpu_buffer_rsrc_t rs, FzList &F, FzBlock &B, int &nr, unsigned &bits,
+                                          int a, int ent, int bv0, int t0, int t1, int t2, int t3)
 {
-    int st[RB], bv[RB];
-    bool act[RB], isd[RB];
+    int st[N], bv[N];
+    bool act[N], isd[N];
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
+    for (int i = 0; i < N; ++i) {
         act[i] = bits != 0;
         const int rel = __builtin_ctz(bits | 0x80000000u);
         const int src = (a + (LI ? rel & 15 : rel)) << 2;
@@ -191,68 +221,62 @@ __device__ __forceinline__ void fz_replay(FzList &F, int &nr, unsigned &bits, in
             st[i] &= 0x7FFFFFFF;
         bits &= bits - 1;
     }
-    const int nr0 = nr;
-    int cur = nr0;
-    int ws[RB], wv[RB];
+    int cur = nr;
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
+    for (int i = 0; i < N; ++i) {
         // the last slot's site and the deleted site's place, as the entries
         // before left them
         int moved = t0;
-        if (i > 0)
-            moved = nr0 - cur == 1 ? t1 : moved;
-        if (i > 1)
-            moved = nr0 - cur == 2 ? t2 : moved;
-        if (i > 2)
-            moved = nr0 - cur == 3 ? t3 : moved;
-#pragma unroll
-        for (int j = 0; j < i; ++j)
-            moved = ws[j] == cur ? wv[j] : moved;
+        if (I0 + i > 0)
+            moved = B.nr0 - cur == 1 ? t1 : moved;
+        if (I0 + i > 1)
+            moved = B.nr0 - cur == 2 ? t2 : moved;
+        if (I0 + i > 2)
+            moved = B.nr0 - cur == 3 ? t3 : moved;
         int mp = bv[i];
 #pragma unroll
-        for (int j = 0; j < i; ++j)
-            mp = wv[j] == st[i] ? ws[j] : mp;
+        for (int j = 0; j < I0 + i; ++j) {
+            moved = B.ws[j] == cur ? B.wv[j] : moved;
+            mp = B.wv[j] == st[i] ? B.ws[j] : mp;
+        }
         // (lists that match the lattice never fail here)
         const bool okd = (unsigned)(mp - 1) < (unsigned)cur;
         const bool del = act[i] && isd[i] && okd;
         const bool add = act[i] && !isd[i] && cur < F.V;
         F.err |= act[i] && !del && !add ? 1 : 0;
-        const bool mv = del && mp < cur;
+        const bool mv = del && mp < cur, put = add || mv;
         const int slot = del ? mp : cur + 1;
-        const int val = del ? (mv ? moved : 0) : st[i];
-        if (del || add) {
-            F.L.b(st[i]) = del ? 0 : slot;
-            F.L.s(slot) = val;
-        }
-        if (mv) {
-            F.L.b(moved) = mp;
-            F.L.s(cur) = 0;
-        }
-        const bool put = add || mv;
-        ws[i] = put ? slot : 0;
-        wv[i] = put ? val : 0;
-        F.patch = ws[i] == F.pk ? wv[i] : F.patch;
+        const int val = del ? moved : st[i];
+        // back[site], the slot, back[moved site]; slots past the end keep
+        // what they held
+        __builtin_amdgcn_raw_buffer_store_b32(del ? 0 : slot, rs,
+                                              del || add ? F.bo + ((unsigned)st[i] << 2) : FZ_NONE, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(val, rs, put ? F.so + ((unsigned)slot << 2) : FZ_NONE, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(slot, rs, mv ? F.bo + ((unsigned)moved << 2) : FZ_NONE, 0, 0);
+        B.ws[I0 + i] = put ? slot : 0;
+        B.wv[I0 + i] = put ? val : 0;
+        F.patch = put && slot == F.pk ? val : F.patch;
         cur = del ? cur - 1 : add ? cur + 1 : cur;
     }
     nr = cur;
 }
 
-// The left-to-right FP64 prefix over lanes (accumulate) for a long chain.
-// Lane l of L links from lane f on adds, at time t, the term of lane
-// l - (L - 1) + t, read from LDS at consecutive addresses; terms below lane f
-// read as zero (adding zero changes no bit), so every lane ends with its own
-// term after the last link.  One LDS read serves two links and a link is one
-// dependent addition, where the shifted form spends two shifts, a hazard
-// and the addition.  `tz`: 128 doubles, the first 64 zero.
+// The left-to-right FP64 prefix over lanes (accumulate).  Lane l of L links
+// from lane f on adds, at time t, the term of lane l - (L - 1) + t, read from
+// LDS at consecutive addresses; terms below lane f read as zero (adding zero
+// changes no bit), so every lane ends with its own term after the last link.
+// One LDS read serves two links and a link is one dependent addition (9
+// cycles), where the shifted form spends two shifts, their hazard and the
+// addition (about 40).  `tz`: 128 doubles, the first 64 zero.
 __device__ __forceinline__ double fz_chain(double *tz, double c, double acc, int P, int lane, int f)
 {
     constexpr int U = 8;
-    const int L = (P - f + U - 1) & ~(U - 1);
-    const double before = f > 0 ? readlane_d(acc, f - 1) : 0.0;
+    const int L = max(P - f + U - 1, U) & ~(U - 1);
+    const double before = readlane_d(acc, max(f, 1) - 1);
     tz[64 + lane] = lane >= f ? c : 0.0;
     wave_sync();
     const double *p = tz + (64 + lane - (L - 1));
-    double a = lane >= f ? before : acc;
+    double a = lane >= f ? (f > 0 ? before : 0.0) : acc;
     double v[U];
 #pragma unroll
     for (int k = 0; k < U; ++k)
@@ -299,11 +323,20 @@ __device__ __attribute__((noinline)) FzUni fz_uniforms(unsigned seed, unsigned s
     return {-log(uu[0]), uu[1], uu[2]};
 }
 
+// What a run keeps beside the steps.
+enum : int { FZ_PLAIN = 0, FZ_REC = 1, FZ_MSD = 2 };
+
 // do_kmc_steps for one replica per wave (proclist_generic_subroutines.mpy:
 // 1-44).  The launch guarantees: records for the model, at most 64
 // processes and two dimensions, lists matching the lattices, lattices in
-// LDS, no extent below 2 * fz_moff + 1 (no two offsets of the records meet).
-template <int BITS, int FORM, bool MSD>
+// LDS, no extent below 2 * fz_moff + 1 (no two offsets of the records meet),
+// rows of more than one site, V times the row below 2^32.
+//
+// A lone wave issues an instruction in 6 to 9 cycles, and a branch or a
+// divergent region costs 30 to 45: the loop has one pass per step with few
+// branches, conditions end in selects, and stops (no process possible, a
+// corrupted list) lower the limit the loop runs to.
+template <int BITS, int FORM, int MODE>
 __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *smem)
 {
     constexpr bool LI = FORM == FZ_LI;
@@ -318,33 +351,32 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
     const int r = wave_setup<1, BITS, true, false>(W, kp, smem);
     if (r < 0)
         return;
-    const int slot = blockIdx.x * kp.wpg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rslot = blockIdx.x * kp.wpg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = W.lane, P = W.P;
     const int *recs = kp.fz_recs;
     const int nch = FORM == FZ_4 ? kp.fz_nch : 1;
     double *tz = (double *)W.win;
-    unsigned *bm = (unsigned *)(tz + 128);             // FZ_LI: entries per process
+    unsigned *bm = (unsigned *)(tz + 128);             // FZ_LI: entries per process, then spare words
     tz[lane] = 0.0;
     if (LI)
         bm[lane] = 0;
     wave_sync();
-    const int st0 = kp.status[r];
+    int st = kp.status[r];
     long long n = kp.nsteps;
     if (kp.budget)
-        n = min(n, kp.budget[slot]);
-    if (st0 != ST_OK)
+        n = min(n, kp.budget[rslot]);
+    if (st != ST_OK)
         n = 0;
-    if (kp.srec)
+    if (MODE == FZ_REC)
         count_species<1, BITS>(W);
-    double t = kp.ktime[r], dt_last = kp.kdt[r];
-    int st = st0;
-    long long done = 0, drawn = 0;                     // steps done, uniforms used
-    int rec_left = kp.sample_every, rec_idx = 0;
+    double t = kp.ktime[r];
+    int rec_left = kp.sample_every + 1, rec_idx = 0;
     const unsigned row = (unsigned)W.V1 << 2;          // bytes of one list
     FzList F;
-    F.L.base = (char *)W.avail;
-    F.L.so = row * (unsigned)(lane < P ? lane : 0);
-    F.L.bo = row * (unsigned)(P + (lane < P ? lane : 0));
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((char *)W.avail - FZ_LEAD, 0, (int)(2u * P * row + FZ_LEAD), 0x00027000);
+    F.so = FZ_LEAD + row * (unsigned)(lane < P ? lane : 0);
+    F.bo = FZ_LEAD + row * (unsigned)(P + (lane < P ? lane : 0));
     F.V = W.d.V;
     F.pk = -1;
     F.patch = 0;
@@ -352,20 +384,62 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
     FzAt at;
     at.sX = W.d.sX;
     at.Y = W.d.Y;
-    const Magic mrow = make_magic(at.sX);
-    const unsigned in_lo = W.d.moff * W.d.spuck, in_w = at.sX - 2 * in_lo;
-    const unsigned in_y = W.d.dim >= 2 ? W.d.moff : 0, in_h = at.Y - 2 * in_y;
-    double lmlog = 0.0, lu1 = 0.0, lu2 = 0.0;
-    // the selected step: its terms, total, process, slot, site on the way
-    double acc = 0.0, c = 0.0, total = 0.0, mlog = 0.0;
-    int pick = 0, kk = 0, sv = 0;
-    int nr = W.nr[0], nrs = nr;                        // nrs: the counts acc belongs to
+    const unsigned mrow = make_magic(at.sX).m;         // (the launch: 1 < sX, V * sX < 2^32)
+    const unsigned in_lo = __builtin_amdgcn_readfirstlane(W.d.moff * W.d.spuck);
+    const unsigned in_y = __builtin_amdgcn_readfirstlane(W.d.dim >= 2 ? W.d.moff : 0);
+    const unsigned in_w = __builtin_amdgcn_readfirstlane(at.sX - 2 * in_lo);
+    const unsigned in_h = __builtin_amdgcn_readfirstlane(at.Y - 2 * in_y);
     const double rate = W.rate[0];
     double integ = W.integ[0];
+    int nr = W.nr[0];
+    double lmlog = 0.0, lu1 = 0.0, lu2 = 0.0;
+    double acc = 0.0;
+    int nrs = -1;                    // the counts acc belongs to (none yet)
+    int nrx = nr;                    // the counts after the step before
+    // the step before: its entries in this lane's list, its terms (none yet)
+    unsigned bits = 0, bo = 0;
+    int a = 0, ent = 0, bv = 0, t0 = 0, t1 = 0, t2 = 0, t3 = 0;
+    bool back = false, three = false;
+    double cc = 0.0, cmlog = 0.0, ctotal = 1.0;
+    int cpick = -1;
+    double total = 0.0;
+    int kk = 0;
     FzRec<FORM> q;
-    // selects step k (0-based in this run) after the counts nrx: accum_rates,
-    // process, slot; its site and records are requested, not waited for
-    auto select = [&](long long k, int nrx, bool anew) {
+#if KMCG_PHASES
+    for (int i = 0; i < 5; ++i)
+        W.tph[i] = 0;
+    W.nblk = W.napply = 0;
+    W.tmark = __builtin_amdgcn_s_memtime();
+#endif
+    auto finish = [&]() {
+        // the list updates of the step before
+        FzBlock B;
+        B.nr0 = nr;
+        fz_replay<0, 2, LI>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
+        if (three) {
+            fz_replay<2, 2, LI>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
+            while (__ballot(bits != 0)) {
+#if KMCG_PHASES
+                W.nblk += 1;
+#endif
+                // four more: the list tail and the back-indices read again,
+                // behind the stores of the block before
+                const int4v tl = __builtin_amdgcn_raw_buffer_load_b128(
+                    rs, bits ? F.so + ((unsigned)nr << 2) - 12 : FZ_NONE, 0, 0);
+                const int bn = __builtin_amdgcn_raw_buffer_load_b32(rs, back ? bo : FZ_NONE, 0, 0);
+                B.nr0 = nr;
+                fz_replay<0, 4, LI>(rs, F, B, nr, bits, a, ent, bn, tl.w, tl.z, tl.y, tl.x);
+            }
+        }
+#if KMCG_PHASES
+        W.napply += 1;
+        W.nblk += 1;
+#endif
+    };
+    long long k = 0;                 // the step being selected
+    long long limit = n;
+    while (n > 0) {
+        PH_MARK(W, 4);
         const int uj = (int)k & 63;
         if (uj == 0) {
             // uniforms of 64 steps at a time: lane i draws step k + i
@@ -375,224 +449,166 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
             lu1 = u.u1;
             lu2 = u.u2;
         }
-        c = (double)nrx * rate;
+        // ---- select step k: accum_rates, process, slot; its site and
+        // records are requested, not waited for
+        const double c = (double)nrx * rate;
         const unsigned long long ch = __ballot(nrx != nrs);
         nrs = nrx;
-        int f = ch ? __ffsll((long long)ch) - 1 : 64;
-        if (anew)
-            f = 0;
-        if (P - f > 6) {
+        const int f = ch ? __ffsll((long long)ch) - 1 : 64;
+        if (P > 2)
             acc = fz_chain(tz, c, acc, P, lane, f);
-        } else if (f < P) {
-            const double cs[1] = {c};
-            double as[1] = {acc};
-            const int fs[1] = {f};
-            accumulate<1>(cs, as, P, lane, fs);
-            acc = as[0];
-        }
+        else
+            acc = wave_shr1z(c) + c;         // one link
         total = readlane_d(acc, P - 1);
-        mlog = readlane_d(lmlog, uj);
-        if (total > 0.0) {
-            // interval_search_real (base.mpy:1234-1338): the first process
-            // whose prefix exceeds the value (no equal prefix lies left of
-            // it), past the end the leftmost of those equal to the last
-            const double value = readlane_d(lu1, uj) * total;
-            unsigned long long mk = __ballot(lane < P && value < acc);
-            if (!mk)
-                mk = __ballot(lane < P && acc == total);
-            pick = __ffsll((long long)mk) - 1;
-            const int nrp = readlane_i(nrx, pick);
-            kk = (int)(1.0 + readlane_d(lu2, uj) * (double)nrp);
-            kk = __builtin_amdgcn_readfirstlane(kk > nrp ? nrp : kk);
-            F.pk = lane == pick && kk > 0 ? kk : -1;
-            F.patch = 0;
-            sv = *(const int *)(F.L.base + (row * (unsigned)pick + ((unsigned)max(kk, 0) << 2)));
-            fz_load<FORM>(recs, pick * nch, lane, q);
+        // interval_search_real (base.mpy:1234-1338): the first process whose
+        // prefix exceeds the value (no equal prefix lies left of it), past
+        // the end the leftmost of those equal to the last
+        const double value = readlane_d(lu1, uj) * total;
+        const unsigned long long mk = __ballot(lane < P && (value < acc || acc == total));
+        const int pick = __ffsll((long long)mk) - 1;
+        const int nrp = readlane_i(nrx, pick);
+        kk = (int)(1.0 + readlane_d(lu2, uj) * (double)nrp);
+        kk = __builtin_amdgcn_readfirstlane(kk > nrp ? nrp : kk);
+        F.pk = lane == pick && kk > 0 ? kk : -1;
+        F.patch = 0;
+        const int sv = __builtin_amdgcn_raw_buffer_load_b32(
+            rs, FZ_LEAD + row * (unsigned)pick + ((unsigned)max(kk, 0) << 2), 0, 0);
+        fz_load<FORM>(recs, pick * nch, lane, q);
+        limit = total > 0.0 && kk > 0 ? limit : k;
+        PH_MARK(W, 0);
+        // ---- finish step k - 1: update_clocks, update_integ_rate (with the
+        // counts before it), its list updates
+        if (MODE != FZ_MSD) {
+            const double dt = cmlog / ctotal;
+            t = t + dt;
+            integ = integ + cc * dt;
+            W.pstat[0] += lane == cpick ? 1 : 0;
         }
-    };
-    if (n > 0) {
-        select(0, nr, true);
-        drawn = 0;
-    }
-#if KMCG_PHASES
-    for (int i = 0; i < 5; ++i)
-        W.tph[i] = 0;
-    W.nblk = W.napply = 0;
-    W.tmark = __builtin_amdgcn_s_memtime();
-#endif
-    while (done != n) {
-        if (!(total > 0.0)) {
-            st = ST_ABSORBING;
+        finish();
+        if (MODE == FZ_REC && --rec_left == 0) {
+            const FzCold kc = fz_cold();
+            W.integ[0] = integ;
+            write_record<1, BITS>(W, kp, rslot, rec_idx, t, cmlog / ctotal, kc->kstep[r] + k, ST_OK);
+            rec_left = kc->sample_every;
+            rec_idx += 1;
+        }
+        PH_MARK(W, 3);
+        if (k == limit || __ballot(F.err))
             break;
-        }
-        PH_MARK(W, 4);
-        // this step's site: read ahead, or just written by the last step
-        const int pv = readlane_i(F.patch, pick);
-        const int site = pv ? pv : __builtin_amdgcn_readfirstlane(sv);
+        // ---- step k: its site, read ahead or just written by the step before
+        const int pv = readlane_i(F.patch, pick), sr = __builtin_amdgcn_readfirstlane(sv);
+        const int site = pv ? pv : sr;
         PH_MARK(W, 1);
-        const int cpick = pick;
-        const double ctotal = total, cc = c, cmlog = mlog;
-        drawn = done + 1;
-        if (kk < 1) {                       // only a corrupted database gets here
-            st = ST_CORRUPT;
-            dt_last = cmlog / ctotal;
-            t = t + dt_last;
-            integ = integ + cc * dt_last;
-            break;
-        }
+        cc = c;
+        cmlog = readlane_d(lmlog, uj);
+        ctotal = total;
+        cpick = pick;
         at.s0 = site - 1;
-        at.y = divm(at.s0, mrow);
+        at.y = (int)__umulhi((unsigned)at.s0, mrow);
         at.rem = at.s0 - at.y * at.sX;
         const bool inside = (unsigned)at.rem - in_lo < in_w && (unsigned)at.y - in_y < in_h;
+        if (MODE == FZ_MSD) {
+            const double dt = cmlog / ctotal;
+            t = t + dt;
+            integ = integ + cc * dt;
+            W.pstat[0] += lane == pick ? 1 : 0;
+            if (kp.acf_pa)
+                acf_before<1, BITS>(W, kp, r, t, dt, pick, site);
+            else
+                msd_track<1, BITS>(W, kp, r, pick, site);
+        }
         const int nchp = FORM == FZ_4 ? __builtin_amdgcn_readfirstlane(bf_u(q.w[1], 16, 5)) : 1;
-        for (int ci = 0; ci < nchp; ++ci) {
+        for (int ci = 0; ; ++ci) {
             // evaluation; bits: this owner lane's entries, nd of them deletions
-            int s, ws, a, nd, ent;
-            unsigned bits, bo;
-            bool back;
+            FzSites<FORM> z;
+            z.template form<true>(at, q);
+            if (!inside)
+                z.template form<false>(at, q);
+            int nd;
+            a = bf_u(q.w[0], 7, 6);
             if constexpr (LI) {
                 int pd, pa;
-                if (inside)
-                    fz_eval_li<BITS, true>(W.lat.p, smem, at, q, s, ws, pd, pa);
-                else
-                    fz_eval_li<BITS, false>(W.lat.p, smem, at, q, s, ws, pd, pa);
+                z.template variants<BITS>(W.lat.p, smem, q, pd, pa);
                 const unsigned at1 = 1u << bf_u(q.w[0], 13, 4);
-                if (pd)
-                    atomicOr(&bm[pd - 1], at1);
-                if (pa)
-                    atomicOr(&bm[pa - 1], at1 << 16);
+                // (a lane without an entry has a spare word of its own)
+                atomicOr(&bm[pd ? pd - 1 : 64 + lane], at1);
+                atomicOr(&bm[pa ? pa - 1 : 64 + lane], at1 << 16);
                 wave_sync();
                 bits = bm[lane];
                 wave_sync();
                 bm[lane] = 0;
-                a = bf_u(q.w[0], 7, 6);
                 back = pd != 0;
-                bo = (__umul24(P - 1 + pd, (unsigned)W.V1) + (unsigned)s + 1u) << 2;
-                ent = s + 1;
+                bo = ((__umul24(P - 1 + pd, (unsigned)W.V1) + (unsigned)z.s) << 2) + (FZ_LEAD + 4);
+                ent = z.s + 1;
                 nd = __popc(bits & 0xFFFFu);
             } else {
-                bool ok;
-                if (inside)
-                    ok = fz_eval<BITS, FORM, true>(W.lat.p, at, q, s, ws);
-                else
-                    ok = fz_eval<BITS, FORM, false>(W.lat.p, at, q, s, ws);
+                const bool ok = z.template holds<BITS>(W.lat.p, q);
                 back = ok && q.w[0] < 0;
-                const unsigned long long mk = __ballot(ok), dk = __ballot(back);
-                bo = (__umul24(q.w[0] & 127, (unsigned)W.V1) + (unsigned)s + 1u) << 2;
-                a = bf_u(q.w[0], 7, 6);
+                const unsigned long long mo = __ballot(ok), mb = __ballot(back);
+                bo = ((__umul24(q.w[0] & 127, (unsigned)W.V1) + (unsigned)z.s) << 2) + (FZ_LEAD + 4);
                 const int len = bf_u(q.w[0], 13, 5);
-                bits = (unsigned)bf_u((int)(mk >> a), 0, len);
-                nd = __popc((unsigned)bf_u((int)(dk >> a), 0, len));
-                ent = (s + 1) | (q.w[0] & (int)0x80000000);
+                bits = (unsigned)bf_u((int)(mo >> a), 0, len);
+                nd = __popc((unsigned)bf_u((int)(mb >> a), 0, len));
+                ent = (z.s + 1) | (q.w[0] & (int)0x80000000);
             }
-            // back[site] of a deletion, the slots a deletion takes the last
-            // site from
-            int bv = 0;
-            if (back)
-                bv = *(const int *)(F.L.base + bo);
+            // back[site] of a deletion; the slots a deletion takes the last
+            // site from, read at once (the words before a list's first are
+            // another list's or the pool's leading words)
+            bv = __builtin_amdgcn_raw_buffer_load_b32(rs, back ? bo : FZ_NONE, 0, 0);
+            const int4v tl = __builtin_amdgcn_raw_buffer_load_b128(
+                rs, nd > 0 ? F.so + ((unsigned)nr << 2) - 12 : FZ_NONE, 0, 0);
+            t0 = tl.w;
+            t1 = tl.z;
+            t2 = tl.y;
+            t3 = tl.x;
             const int ne = __popc(bits);
-            const bool two = __ballot(ne > 1), three = __ballot(ne > 2), four = __ballot(ne > 3);
-            int t0 = 0, t1 = 0, t2 = 0, t3 = 0;
-            if (nd > 0)
-                t0 = F.L.s(nr);
-            if (two && nd > 1) {
-                t1 = F.L.s(max(nr - 1, 0));
-                if (nd > 2)
-                    t2 = F.L.s(max(nr - 2, 0));
-                if (nd > 3)
-                    t3 = F.L.s(max(nr - 3, 0));
-            }
-            const int w0 = q.w[0];
-            const bool lastc = ci == nchp - 1;
-            PH_MARK(W, 2);
-            if (lastc)
-                select(done + 1, nr + ne - 2 * nd, false);
-            else
-                fz_load<FORM>(recs, cpick * nch + ci + 1, lane, q);
-            PH_MARK(W, 0);
+            nrx = nr + ne - 2 * nd;
+            three = __ballot(ne > 2) != 0;
             // the writes (their old species are known); nothing of this
             // step reads a written site
-            const int so = bf_u(w0, 22, 4), sn = bf_u(w0, 26, 4);
-            if (so != sn) {
-                W.lat.xset(ws, so, sn);
-                if (W.track) {
-                    const int tt = ws - divm(ws, W.ms) * W.d.spuck;
-                    if (so < W.S)
-                        atomicAdd(&W.occ[so * W.d.spuck + tt], -1);
-                    if (sn < W.S)
-                        atomicAdd(&W.occ[sn * W.d.spuck + tt], 1);
-                }
+            const int so = bf_u(q.w[0], 22, 4), sn = bf_u(q.w[0], 26, 4);
+            fz_write<BITS>(W.lat.p, bm + 64 + lane, z.ws, so, sn);
+            if (MODE == FZ_REC && so != sn) {
+                const int tt = z.ws - divm(z.ws, W.ms) * W.d.spuck;
+                if (so < W.S)
+                    atomicAdd(&W.occ[so * W.d.spuck + tt], -1);
+                if (sn < W.S)
+                    atomicAdd(&W.occ[sn * W.d.spuck + tt], 1);
             }
             wave_sync();
-            if (lastc) {
-                // update_clocks, update_integ_rate with the counts before
-                const double dt = cmlog / ctotal;
-                t = t + dt;
-                dt_last = dt;
-                integ = integ + cc * dt;
-                W.pstat[0] += lane == cpick ? 1 : 0;
-                done += 1;
-                if (MSD) {
-                    if (kp.acf_pa)
-                        acf_before<1, BITS>(W, kp, r, t, dt, cpick, site);
-                    else
-                        msd_track<1, BITS>(W, kp, r, cpick, site);
-                }
-            }
-            // the list updates
-#if KMCG_PHASES
-            W.napply += 1;
-            W.nblk += 1;
-#endif
-            if (four) {
-                fz_replay<4, LI>(F, nr, bits, a, ent, bv, t0, t1, t2, t3);
-                while (__ballot(bits != 0)) {
-#if KMCG_PHASES
-                    W.nblk += 1;
-#endif
-                    // the next four: list tail and back-indices read again,
-                    // behind the stores of the block before
-                    const bool more = bits != 0;
-                    t0 = more ? F.L.s(nr) : 0;
-                    t1 = more ? F.L.s(max(nr - 1, 0)) : 0;
-                    t2 = more ? F.L.s(max(nr - 2, 0)) : 0;
-                    t3 = more ? F.L.s(max(nr - 3, 0)) : 0;
-                    if (back)
-                        bv = *(const int *)(F.L.base + bo);
-                    fz_replay<4, LI>(F, nr, bits, a, ent, bv, t0, t1, t2, t3);
-                }
-            } else if (three) {
-                fz_replay<3, LI>(F, nr, bits, a, ent, bv, t0, t1, t2, 0);
-            } else if (two) {
-                fz_replay<2, LI>(F, nr, bits, a, ent, bv, t0, t1, 0, 0);
-            } else {
-                fz_replay<1, LI>(F, nr, bits, a, ent, bv, t0, 0, 0, 0);
-            }
-            PH_MARK(W, 3);
+            if (ci == nchp - 1)
+                break;
+            fz_load<FORM>(recs, pick * nch + ci + 1, lane, q);
+            finish();
         }
-        if (MSD && kp.acf_pa && lane == 0)
+        if (MODE == FZ_MSD && kp.acf_pa && lane == 0)
             acf_after(kp, r);
-        if (__ballot(F.err)) {
-            st = LI ? ST_DEL_ABSENT : ST_CORRUPT;
-            break;
-        }
-        if (W.track && --rec_left == 0) {
-            const FzCold kc = fz_cold();
-            W.integ[0] = integ;
-            write_record<1, BITS>(W, kp, slot, rec_idx, t, dt_last, kc->kstep[r] + done, ST_OK);
-            rec_left = kc->sample_every;
-            rec_idx += 1;
+        k += 1;
+        PH_MARK(W, 2);
+    }
+    const FzCold kc = fz_cold();
+    double dt_last = k > 0 ? cmlog / ctotal : kc->kdt[r];
+    long long drawn = k;
+    if (__ballot(F.err)) {
+        st = LI ? ST_DEL_ABSENT : ST_CORRUPT;
+    } else if (k < n) {
+        st = ST_ABSORBING;
+        if (total > 0.0) {               // only a corrupted database gets here
+            st = ST_CORRUPT;
+            drawn += 1;
+            dt_last = readlane_d(lmlog, (int)k & 63) / total;
+            t = t + dt_last;
+            integ = integ + ((double)nrx * rate) * dt_last;
         }
     }
     W.nr[0] = nr;
     W.integ[0] = integ;
-    const FzCold kc = fz_cold();
-    steps_end<1, BITS, true>(W, kp, r, slot, t, dt_last, kc->kstep[r] + drawn, kc->rngctr[r] + drawn, st, done);
+    steps_end<1, BITS, true>(W, kp, r, rslot, t, dt_last, kc->kstep[r] + drawn, kc->rngctr[r] + drawn, st, k);
 }
 
-template <int BITS, int FORM, bool MSD>
+template <int BITS, int FORM, int MODE>
 __global__ __launch_bounds__(64 * MAX_WPG) __attribute__((amdgpu_waves_per_eu(4))) void kmc_steps_kernel_fz(KParams kp)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    fused_loop<BITS, FORM, MSD>(kp, smem);
+    fused_loop<BITS, FORM, MODE>(kp, smem);
 }
