@@ -1457,6 +1457,67 @@ __device__ __forceinline__ void acf_after(const KParams &kp, int r)
     }
 }
 
+// Species counts of a 2-bit lattice, SP site types per cell (1, 2 or 4, so
+// that a word's 16 sites keep their types), words i0, i0 + step, ...: three
+// masks and a population count per species and word instead of an LDS
+// atomic per site, which all meet on a few counters.
+template <int SP>
+__device__ __forceinline__ void count_words(const unsigned *w, int nw, int i0, int step, int (&cnt)[3 * SP])
+{
+#pragma unroll
+    for (int j = 0; j < 3 * SP; ++j)
+        cnt[j] = 0;
+    constexpr unsigned types[3] = {0x55555555u, 0x11111111u, 0x01010101u};
+    constexpr unsigned m0 = types[SP == 1 ? 0 : SP == 2 ? 1 : 2];
+    for (int i = i0; i < nw; i += step) {
+        const unsigned v = w[i];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned x = v ^ (0x55555555u * (unsigned)(q + 1));       // 00 where the species is q
+            const unsigned hit = ~(x | (x >> 1));
+#pragma unroll
+            for (int t = 0; t < SP; ++t)
+                cnt[q * SP + t] += __popc(hit & (m0 << (2 * t)));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 3 * SP; ++j)
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1)
+            cnt[j] += __shfl_xor(cnt[j], d);
+}
+
+// Adds this wave's share of a lattice's species counts (sites i0, i0 + step,
+// ... of V; words of a 2-bit lattice) to counts[S][spuck].
+template <int BITS, int SP>
+__device__ __forceinline__ void add_words(const unsigned char *lat, int V, int i0, int step, int S, int lane, int *counts)
+{
+    int cnt[3 * SP];
+    count_words<SP>((const unsigned *)lat, (V + 15) >> 4, i0, step, cnt);
+#pragma unroll
+    for (int j = 0; j < 3 * SP; ++j)
+        if (lane == j && j < S * SP)
+            atomicAdd(&counts[j], cnt[j]);
+}
+template <int BITS>
+__device__ __forceinline__ void add_species(const Lattice<BITS> &lat, int V, int i0, int step, int S, int spuck,
+                                            const Magic &ms, int lane, int *counts)
+{
+    if (BITS == 2 && spuck == 1) {
+        add_words<BITS, 1>(lat.p, V, i0, step, S, lane, counts);
+    } else if (BITS == 2 && spuck == 2) {
+        add_words<BITS, 2>(lat.p, V, i0, step, S, lane, counts);
+    } else if (BITS == 2 && spuck == 4) {
+        add_words<BITS, 4>(lat.p, V, i0, step, S, lane, counts);
+    } else {
+        for (int s = i0; s < V; s += step) {
+            const int q = lat.get(s);
+            if (q >= 0 && q < S)
+                atomicAdd(&counts[q * spuck + (s - divm(s, ms) * spuck)], 1);
+        }
+    }
+}
+
 // The species counts per site type of a run that records samples, kept up to
 // date by the writes from here on.
 template <int PPL, int BITS>
@@ -1467,11 +1528,7 @@ __device__ __forceinline__ void count_species(Wave<PPL, BITS> &W)
     for (int i = W.lane; i < no; i += 64)
         W.occ[i] = 0;
     wave_sync();
-    for (int s = W.lane; s < W.d.V; s += 64) {
-        const int q = W.lat.get(s);
-        if (q >= 0 && q < W.S)
-            atomicAdd(&W.occ[q * W.d.spuck + (s - divm(s, W.ms) * W.d.spuck)], 1);
-    }
+    add_species<BITS>(W.lat, W.d.V, W.lane, 64, W.S, W.d.spuck, W.ms, W.lane, W.occ);
     wave_sync();
 }
 
@@ -2001,11 +2058,7 @@ __global__ void kmc_occupation_kernel(KParams kp, double *out)
     __syncthreads();
     Lattice<BITS> lat;
     lat.p = kp.lat_pool + kp.lat_off[r];
-    for (int s = threadIdx.x; s < dd.w; s += blockDim.x) {
-        const int sp = lat.get(s);
-        if (sp >= 0 && sp < S)
-            atomicAdd(&counts[sp * spuck + s % spuck], 1);
-    }
+    add_species<BITS>(lat, dd.w, threadIdx.x, blockDim.x, S, spuck, make_magic(spuck), threadIdx.x & 63, counts);
     __syncthreads();
     const double cells = (double)dd.x * dd.y * dd.z;
     for (int i = threadIdx.x; i < S * spuck; i += blockDim.x)
@@ -2028,11 +2081,7 @@ __global__ __launch_bounds__(256) void kmc_sample_kernel(KParams kp, double *out
     __syncthreads();
     Lattice<BITS> lat;
     lat.p = kp.lat_pool + kp.lat_off[r];
-    for (int s = threadIdx.x; s < dd.w; s += blockDim.x) {
-        const int sp = lat.get(s);
-        if (sp >= 0 && sp < S)
-            atomicAdd(&counts[sp * spuck + s % spuck], 1);
-    }
+    add_species<BITS>(lat, dd.w, threadIdx.x, blockDim.x, S, spuck, make_magic(spuck), threadIdx.x & 63, counts);
     __syncthreads();
     double *rec = out + (long long)blockIdx.x * width;
     const double cells = (double)dd.x * dd.y * dd.z;
