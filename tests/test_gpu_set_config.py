@@ -1,0 +1,50 @@
+"""kmcg_set_config (the database rebuilt list by list) against the oracle's
+touchups one after the other: lists left by earlier steps and an earlier
+configuration, every backend, one and several layers, lattices whose lists
+fit LDS and one whose lists do not, a replica that has stopped."""
+import os
+
+import numpy as np
+import pytest
+
+from kmos_amd import workloads as W
+from kmos_amd.compiler import compile_model
+from kmos_amd.model import load_project
+from paritylib import GOLDEN, compare_state, oracle_replica, pdopd_project, random_config
+
+pytestmark = pytest.mark.gpu
+
+SMALL = [(8, 8), (9, 13), (16, 17), (31, 11)]
+CASES = [
+    ("quickstart", W.quickstart_project, "local_smart", [(1, 1), (5, 3), (215, 211)]),
+    ("zgb", W.zgb_project, "local_smart", SMALL), ("zgb_li", W.zgb_project, "lat_int", SMALL),
+    ("ruo2", W.ruo2_project, "local_smart", SMALL), ("ruo2_li", W.ruo2_project, "lat_int", SMALL),
+    ("pairwise", W.pairwise_project, "local_smart", SMALL), ("pairwise_li", W.pairwise_project, "lat_int", SMALL),
+    ("grid", lambda: load_project(os.path.join(GOLDEN, "2d_grid.xml")), "local_smart", SMALL),
+    ("pdopd", pdopd_project, "local_smart", [(4, 4), (8, 5)]), ("pdopd_li", pdopd_project, "lat_int", [(4, 4), (8, 5)]),
+]
+
+
+@pytest.mark.parametrize("name,factory,backend,sizes", CASES, ids=[c[0] for c in CASES])
+def test_set_config_matches_oracle(engine, oracle, name, factory, backend, sizes):
+    pt = factory()
+    cm = compile_model(pt, backend)
+    g = np.random.default_rng(23)
+    n = len(sizes)
+    rates = 10.0 ** g.uniform(-1, 3, (n, cm.nr_of_proc))
+    seeds = g.integers(1 << 31, size=n).astype(np.uint32)
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init(seeds, np.zeros(n, np.uint32))
+    b.set_rates(rates)
+    orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), 0, rates[i]) for i, s in enumerate(sizes)]
+    for rnd, steps in enumerate((200, 300, 50)):
+        configs = [random_config(pt, int(v), g) for v in b.volumes]
+        b.set_config(configs)
+        for i, o in enumerate(orcs):
+            o.set_config(configs[i])
+            compare_state(b, i, o, where="%s %s configuration %d" % (name, sizes[i], rnd))
+        b.run(steps)
+        for i, o in enumerate(orcs):
+            o.run(steps)
+            compare_state(b, i, o, where="%s %s steps %d" % (name, sizes[i], rnd))
+    b.close()
