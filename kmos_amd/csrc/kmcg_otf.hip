@@ -16,13 +16,13 @@
 // processes).  The lattice sits in LDS as one byte per site.  In HBM, per
 // replica and process, four rows of C entries (C = cells): the list
 // (cell + 1, 0 = empty), the inverse index (list position + 1 by cell),
-// the entry rates and their running sum in list order.  The running sum is
-// what makes the step exact and cheap: the reference's full re-summation
-// in list order equals the stored running sum as long as every entry from
-// the first changed position on is re-added, so a step re-adds only the
-// tail behind the smallest list position it changed (per owner lane,
-// sequential, in the same order as the reference's loop).  The site
-// search reads that running sum: 64-ary, two or three dependent rounds.
+// the entry rates and, after every 16th entry, their running sum in list
+// order.  The running sum is what makes the step exact and cheap: the
+// reference's full re-summation in list order equals the stored running sum
+// as long as every entry from the first changed position on is re-added, so
+// a step re-adds only the blocks from the smallest list position it changed
+// on (sequential, in the same order as the reference's loop).  The site
+// search reads those sums, then the 16 entries behind the one it finds.
 //
 // Rates.  gr_<proc>(cell) depends only on the bystander counts; the host
 // evaluates each process's expression for every count combination once per
@@ -50,9 +50,11 @@ struct OtfParams {
     const int *prog;                 // global copy of the program (W words)
     int off_owner, off_writes, off_byst, off_tbase, off_touch;
     int tab_lds;                     // 1: the replica's rate table is staged in LDS too
+    const int *fast;                 // otf_fast_kernel: its LDS words (FW), then the op records
+    int FW, off_fw, off_fb, off_ft;  // writes, bystanders, table bases within the LDS words
     const int *dims;                 // [n][4]: X, Y, Z, C
     const long long *lat_off;        // [n]: first site of the replica in `lat`
-    const long long *list_off;       // [n]: first entry of the replica's rows
+    const long long *list_off;       // [n]: first entry of the replica's rows (of otf_row(C) entries each)
     signed char *lat;
     int *sites, *back;
     double *rm, *pre;
@@ -139,122 +141,195 @@ __device__ __forceinline__ int otf_del(int *srow, int *brow, double *rrow, int &
     return changed;
 }
 
-// the running sum of a row from position `from` on (update_accum_rate's
-// order: left to right), one lane alone; returns the row's total
-__device__ __forceinline__ double otf_resum(const double *rrow, double *prow, int from, int n)
+// entries from one row to the next: whole checkpoint blocks
+constexpr int OTF_BLK = 16;
+__host__ __device__ inline long long otf_row(int C) { return (C + OTF_BLK - 1) & ~(long long)(OTF_BLK - 1); }
+
+// A row's running sum in list order (update_accum_rate, base_otf.f90:
+// 687-717), kept after every 16th entry only: chk[j] is the sum of the first
+// 16 (j + 1) entries.  Re-adds the entries from the block of position `from`
+// on and returns the row's total.  Every lane walks its own row: an entry is
+// one dependent addition, half a load and a sixteenth of a store, where rows
+// of 16 lanes shifting a carry spent three instructions and a hazard per
+// entry on four rows at a time.  Entries past the end are zero (adding zero
+// changes no bit).  AHEAD blocks are on their way at a time.
+template <int AHEAD>
+__device__ __forceinline__ double otf_resum(const double *rrow, double *chk, int from, int n)
 {
-    double a = from > 0 ? prow[from - 1] : 0.0;
-    int j = from;
-    for (; j + 8 <= n; j += 8) {
-        double v[8];
+    const int b0 = from >> 4, nb = (n + OTF_BLK - 1) >> 4;
+    double a = b0 > 0 ? chk[b0 - 1] : 0.0;
+    if (b0 >= nb)
+        return a;
+    typedef double double2w __attribute__((ext_vector_type(2), aligned(8)));
+    double2w v[AHEAD][8];
+    auto load = [&](double2w (&w)[8], int b) {
+        // past the last block: the last one again, not used
+        const double2w *s = (const double2w *)(rrow + OTF_BLK * min(b, nb - 1));
 #pragma unroll
         for (int k = 0; k < 8; ++k)
-            v[k] = rrow[j + k];
+            w[k] = s[k];
+    };
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            a = a + v[k];
-            prow[j + k] = a;
+    for (int j = 0; j < AHEAD; ++j)
+        load(v[j], b0 + j);
+    for (int b = b0;;) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                a = a + v[j][k].x;
+                a = a + v[j][k].y;
+            }
+            chk[b] = a;
+            if (++b >= nb)
+                return a;
+            load(v[j], b + AHEAD - 1);
         }
     }
-    for (; j < n; ++j) {
-        a = a + rrow[j];
-        prow[j] = a;
+}
+
+// otf_resum for all lists a step changed at once (whole wave; `want`, from,
+// n, rrow and chk per owner lane).  A lane that reads its own row alone takes
+// 16 of a line's 128 bytes at a time, and with ten rows and five blocks ahead
+// in eight waves per CU the lines outgrow the L1 cache: 35,000 to 50,000
+// cycles of a full chip's step against 16,000 on an empty one.  Here 16
+// lanes read a row's block (one line), four rows per load, OTF_DEEP blocks
+// ahead in registers; each block passes through LDS to the lane that adds
+// it up: 25,000 to 37,000 cycles on a full chip (33 -> 24 us per step), bound
+// by its additions and their LDS reads.  Up to OTF_ROWS lists at a time.
+// Returns the row's total where `want`.
+constexpr int OTF_ROWS = 12, OTF_DEEP = 6, OTF_STAGE = OTF_BLK + 2;   // (16-byte aligned, spread over the banks)
+
+__device__ __forceinline__ double otf_resum_wave(const double *rm, long long crow, double *chk, bool want, int from,
+                                                 int n, double tot, double *stage, int *ids, int lane)
+{
+    constexpr int SETS = OTF_ROWS / 4;
+    const int b0 = from >> 4, nb = (n + OTF_BLK - 1) >> 4;
+    // short tails only (rates that do not differ within a list): each lane
+    // its own
+    if (!__ballot(want && nb - b0 > 2))
+        return want ? otf_resum<2>(rm + lane * crow, chk, from, n) : tot;
+    double a = want && b0 > 0 ? chk[b0 - 1] : 0.0;
+    unsigned long long todo = __ballot(want && b0 < nb);
+    while (todo) {
+        // this group's lists: the first OTF_ROWS pending lanes
+        const int rank = __popcll(todo & ((1ull << lane) - 1ull));
+        const bool mine = ((todo >> lane) & 1) && rank < OTF_ROWS;
+        if (lane < OTF_ROWS)
+            ids[lane] = -1;
+        wave_sync();
+        if (mine)
+            ids[rank] = lane;
+        wave_sync();
+        const double *src[SETS];
+        int last[SETS];
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) {
+            const int id = ids[4 * i + (lane >> 4)];
+            const int f = __builtin_amdgcn_ds_bpermute(id << 2, b0), e = __builtin_amdgcn_ds_bpermute(id << 2, nb);
+            // (behind its last block a row reads that one again, unused)
+            last[i] = id >= 0 ? e - f - 1 : 0;
+            src[i] = rm + max(id, 0) * crow + (id >= 0 ? OTF_BLK * f : 0) + (lane & 15);
+        }
+        const int T = mine ? nb - b0 : 0;
+        double v[OTF_DEEP][SETS];
+#pragma unroll
+        for (int j = 0; j < OTF_DEEP; ++j)
+#pragma unroll
+            for (int i = 0; i < SETS; ++i)
+                v[j][i] = src[i][OTF_BLK * min(j, last[i])];
+        const double *my = stage + (mine ? rank : 0) * OTF_STAGE;
+        double sum = a;
+        for (int t0 = 0; __ballot(t0 < T); t0 += OTF_DEEP) {
+#pragma unroll
+            for (int j = 0; j < OTF_DEEP; ++j) {
+                const int t = t0 + j;
+#pragma unroll
+                for (int i = 0; i < SETS; ++i) {
+                    stage[(4 * i + (lane >> 4)) * OTF_STAGE + (lane & 15)] = v[j][i];
+                    v[j][i] = src[i][OTF_BLK * min(t + OTF_DEEP, last[i])];
+                }
+                wave_sync();
+                double w[OTF_BLK];
+#pragma unroll
+                for (int k = 0; k < OTF_BLK; ++k)
+                    w[k] = my[k];
+#pragma unroll
+                for (int k = 0; k < OTF_BLK; ++k)
+                    sum = sum + w[k];
+                if (t < T)
+                    chk[b0 + t] = a = sum;
+                wave_sync();
+            }
+        }
+        todo &= ~__ballot(mine);
     }
+    return want ? a : tot;
+}
+
+// The running sum of the first pos + 1 entries of a row.
+__device__ __forceinline__ double otf_prefix(const double *rrow, const double *chk, int pos)
+{
+    double a = pos >> 4 ? chk[(pos >> 4) - 1] : 0.0;
+    for (int j = pos & ~(OTF_BLK - 1); j <= pos; ++j)
+        a = a + rrow[j];
     return a;
 }
 
-// lane l receives v from lane l-1 of its row of 16 (DPP row_shr:1); the
-// first lane of each row receives 0
-__device__ __forceinline__ double row_shr1z(double v)
+// The cell of the first entry of a row of np entries whose running sum
+// exceeds vs (interval search of determine_procsite, base_otf.f90:1213-1278;
+// past the end the last entry, walked left over equal sums).  Uniform call:
+// 64-ary over the checkpoints, four of them per lane in the last round, then
+// the 16 entries behind the one found, added by every lane alike, their
+// cells read along with them.
+__device__ __forceinline__ int otf_pick(const int *srow, const double *rrow, const double *chk, int np, double vs,
+                                        int lane)
 {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x111, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x111, 0xF, 0xF, true);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
-// The pending list with the most entries to re-add (uniform; ties to the
-// lowest lane), taken off `pend`; -1 when none is left.
-__device__ __forceinline__ int otf_take_longest(unsigned long long &pend, int len)
-{
-    int best = -1, most = -1;
-    for (unsigned long long m = pend; m; m &= m - 1) {
-        const int l = __ffsll((long long)m) - 1;
-        const int v = readlane_i(len, l);
-        if (v > most) {
-            most = v;
-            best = l;
+    int lo = 0, hi = np >> 4;
+    while (hi - lo > 256) {
+        const int stride = (hi - lo + 63) >> 6;
+        const int at = lo + (lane + 1) * stride - 1;
+        const bool in = at < hi;
+        const double pv = in ? chk[at] : 0.0;
+        const unsigned long long mm = __ballot(in && pv > vs);
+        if (mm) {
+            const int k = __ffsll((long long)mm) - 1;
+            hi = lo + (k + 1) * stride - 1;
+            lo = lo + k * stride;
+        } else {
+            lo = lo + (int)__popcll(__ballot(in)) * stride;
         }
     }
-    if (best >= 0)
-        pend &= ~(1ull << best);
-    return best;
-}
-
-// The running sums of every list a step changed, re-added from its first
-// changed position to its end, four lists at a time (the longest four
-// first, so that lists of like length share a pass): each row of 16 lanes
-// walks one list in blocks of 16 entries (one coalesced read), and within
-// a block the sum is carried left to right through the row by 15 shifted
-// adds, so lane i ends with ((carry + r0) + r1) + ... + ri, the rounding of
-// update_accum_rate's loop.  `dirty` and `n` are per owner lane.
-__device__ __forceinline__ void otf_resum_rows(const double *rm, double *pre, long long base, int C, int lane,
-                                               bool want, int dirty, int n)
-{
-    unsigned long long dm = __ballot(want && dirty < n);
-    const int row = lane >> 4, i = lane & 15;
-    const int mylen = (want && dirty < n) ? n - dirty : 0;
-    while (dm) {
-        int qs[4];
+    double c4[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            qs[k] = otf_take_longest(dm, mylen);
-        int d4[4], n4[4];
+    for (int k = 0; k < 4; ++k)
+        c4[k] = lo + 4 * lane + k < hi ? chk[lo + 4 * lane + k] : 0.0;
+    int mine = 4;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            d4[k] = qs[k] >= 0 ? readlane_i(dirty, qs[k]) : 0;
-            n4[k] = qs[k] >= 0 ? readlane_i(n, qs[k]) : 0;
-        }
-        const int q = row == 0 ? qs[0] : (row == 1 ? qs[1] : (row == 2 ? qs[2] : qs[3]));
-        const int d = row == 0 ? d4[0] : (row == 1 ? d4[1] : (row == 2 ? d4[2] : d4[3]));
-        const int len = (row == 0 ? n4[0] : (row == 1 ? n4[1] : (row == 2 ? n4[2] : n4[3]))) - d;
-        const int maxlen = max(max(n4[0] - d4[0], n4[1] - d4[1]), max(n4[2] - d4[2], n4[3] - d4[3]));
-        const double *rr = rm + base + (long long)(q < 0 ? 0 : q) * C;
-        double *pr = pre + base + (long long)(q < 0 ? 0 : q) * C;
-        double carry = (q >= 0 && d > 0) ? pr[d - 1] : 0.0;
-        // eight blocks per trip, the next eight read while these are summed
-        constexpr int NB = 8;
-        double v[NB], vn[NB];
+    for (int k = 3; k >= 0; --k)
+        mine = lo + 4 * lane + k < hi && c4[k] > vs ? k : mine;
+    const unsigned long long mc = __ballot(mine < 4);
+    const int l0 = mc ? __ffsll((long long)mc) - 1 : 0;
+    const int blk = mc ? lo + 4 * l0 + readlane_i(mine, l0) : hi;
+    double a = blk > 0 ? chk[blk - 1] : 0.0;
+    const int mycell = lane < OTF_BLK && OTF_BLK * blk + lane < np ? srow[OTF_BLK * blk + lane] : 0;
+    double e[OTF_BLK];
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-            v[b] = (16 * b + i < len) ? rr[d + 16 * b + i] : 0.0;
-        for (int off = 0; off < maxlen; off += 16 * NB) {
+    for (int k = 0; k < OTF_BLK; ++k)
+        e[k] = OTF_BLK * blk + k < np ? rrow[OTF_BLK * blk + k] : 0.0;
+    int at = 0;
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int jn = off + 16 * (NB + b) + i;
-                vn[b] = (jn < len) ? rr[d + jn] : 0.0;
-            }
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int j = off + 16 * b;
-                if (j >= maxlen)
-                    break;
-                const double ce = (i == 0) ? carry + v[b] : v[b];
-                double a = ce;
-#pragma unroll
-                for (int k = 1; k < 16; ++k)
-                    a = row_shr1z(a) + ce;
-                if (j + i < len)
-                    pr[d + j + i] = a;
-                const double c0 = readlane_d(a, 15), c1 = readlane_d(a, 31), c2 = readlane_d(a, 47),
-                             c3 = readlane_d(a, 63);
-                carry = row == 0 ? c0 : (row == 1 ? c1 : (row == 2 ? c2 : c3));
-            }
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-                v[b] = vn[b];
-        }
+    for (int k = 0; k < OTF_BLK; ++k) {
+        a = a + e[k];
+        at += a > vs ? 0 : 1;
     }
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (OTF_BLK * blk + at < np)
+        return readlane_i(mycell, at) - 1;
+    int pos = np - 1;
+    while (pos > 0 && otf_prefix(rrow, chk, pos - 1) >= otf_prefix(rrow, chk, pos))
+        --pos;
+    return __builtin_amdgcn_readfirstlane(srow[pos]) - 1;
 }
 
 __device__ __forceinline__ bool otf_conds(const OtfParams &p, const OtfCell &g, const signed char *slat,
@@ -296,11 +371,11 @@ __global__ __launch_bounds__(64) void otf_setup_kernel(OtfParams p)
     if (lane >= p.P)
         return;
     const int q = lane;
-    const long long lo = p.list_off[r] + (long long)q * g.C;
+    const long long lo = p.list_off[r] + q * otf_row(g.C);
     int *srow = p.sites + lo;
     int *brow = p.back + lo;
     double *rrow = p.rm + lo;
-    double *prow = p.pre + lo;
+    double *prow = p.pre + lo / OTF_BLK;
     const double *tab = p.table + (long long)r * p.T;
     const int slot = r * p.P + q;
     int n = p.nsites[slot];
@@ -359,7 +434,7 @@ __global__ __launch_bounds__(64) void otf_setup_kernel(OtfParams p)
             }
         }
     }
-    otf_resum(rrow, prow, 0, n);
+    otf_resum<5>(rrow, prow, 0, n);
     p.nsites[slot] = n;
     p.runsum[slot] = run;
     if (p.mode == 0) {
@@ -407,14 +482,15 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
     const bool act = lane < P;
     const int q = act ? lane : 0;
     const long long base = p.list_off[r];
-    const long long lo = base + (long long)q * g.C;
+    const long long crow = otf_row(g.C);
+    const long long lo = base + q * crow;
     int *srow = p.sites + lo;
     int *brow = p.back + lo;
     double *rrow = p.rm + lo;
-    double *prow = p.pre + lo;
+    double *chk = p.pre + lo / OTF_BLK;
     const int slot = r * P + q;
     int n = act ? p.nsites[slot] : 0;
-    double tot = (act && n > 0) ? prow[n - 1] : 0.0;
+    double tot = (act && n > 0) ? otf_prefix(rrow, chk, n - 1) : 0.0;
     double integ = act ? p.integ[slot] : 0.0;
     double run = act ? p.runsum[slot] : 0.0;
     double my_acc = act ? p.accum[slot] : 0.0;
@@ -424,9 +500,17 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
     long long kstep = p.kmc_step[r];
     unsigned long long ctr = p.ctr[r];
     const unsigned seed = p.seed[r], stream = p.stream[r];
+    const unsigned long long ctr0 = ctr;
+    double lmlog = 0.0, lu1 = 0.0, lu2 = 0.0;
     for (long long s = 0; s < p.steps; ++s) {
-        double u[3];
-        step_uniforms(seed, stream, ctr, u);
+        // uniforms of 64 steps at a time: lane i draws step s + i
+        const int uj = (int)s & 63;
+        if (uj == 0) {
+            const FzUni un = fz_uniforms(seed, stream, ctr0 + (unsigned long long)s + lane);
+            lmlog = un.mlog;
+            lu1 = un.u1;
+            lu2 = un.u2;
+        }
         // update_accum_rate: accum(i) = accum(i-1) + sum of list i
         double acc = 0.0;
         for (int i = 0; i < P; ++i) {
@@ -443,7 +527,7 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
         }
         ctr += 1;
         // update_clocks, update_integ_rate
-        const double dt = -log(u[0]) / total;
+        const double dt = readlane_d(lmlog, uj) / total;
         t_step = dt;
         t = t + dt;
         kstep += 1;
@@ -451,44 +535,16 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
         // determine_procsite: the first process whose accum exceeds the
         // value (interval_search_real); past the end, the last one, walked
         // left over equal sums
-        const double v = u[1] * total;
+        const double v = readlane_d(lu1, uj) * total;
         const unsigned long long mp = __ballot(act && my_acc > v);
         int proc = mp ? __ffsll((long long)mp) - 1 : P - 1;
         if (!mp)
             while (proc > 0 && readlane_d(my_acc, proc - 1) >= readlane_d(my_acc, proc))
                 --proc;
         const int np = readlane_i(n, proc);
-        const double vs = u[2] * readlane_d(tot, proc);
-        const double *pp = p.pre + base + (long long)proc * g.C;
-        int lo_ = 0, hi_ = np;
-        while (hi_ - lo_ > 64) {
-            const int stride = (hi_ - lo_ + 63) >> 6;
-            const int at = lo_ + (lane + 1) * stride - 1;
-            const bool in = at < hi_;
-            const double pv = in ? pp[at] : 0.0;
-            const unsigned long long mm = __ballot(in && pv > vs);
-            if (mm) {
-                const int k = __ffsll((long long)mm) - 1;
-                hi_ = lo_ + (k + 1) * stride - 1;
-                lo_ = lo_ + k * stride;
-            } else {
-                lo_ = lo_ + (int)__popcll(__ballot(in)) * stride;
-            }
-        }
-        int pos;
-        {
-            const int at = lo_ + lane;
-            const bool in = at < hi_;
-            const double pv = in ? pp[at] : 0.0;
-            const unsigned long long mm = __ballot(in && pv > vs);
-            pos = mm ? lo_ + __ffsll((long long)mm) - 1 : hi_;
-        }
-        if (pos >= np) {
-            pos = np - 1;
-            while (pos > 0 && pp[pos - 1] >= pp[pos])
-                --pos;
-        }
-        const int cell = p.sites[base + (long long)proc * g.C + pos] - 1;
+        const double vs = readlane_d(lu2, uj) * readlane_d(tot, proc);
+        const int cell = otf_pick(p.sites + base + proc * crow, p.rm + base + proc * crow,
+                                  p.pre + (base + proc * crow) / OTF_BLK, np, vs, lane);
         int x, y, z;
         g.xyz(cell, x, y, z);
         if (lane == proc)
@@ -605,9 +661,10 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
                 w += 1 + ncond;
             }
         }
-        otf_resum_rows(p.rm, p.pre, base, g.C, lane, act, dirty, n);
-        if (dirty != 0x7fffffff)
-            tot = n > 0 ? prow[n - 1] : 0.0;
+        // (an entry deleted at the end leaves its block's checkpoint behind
+        // the last whole block: not read)
+        if (act && dirty != 0x7fffffff)
+            tot = otf_resum<5>(rrow, chk, min(dirty, n), n);
         if (__ballot(bad)) {
             st = KMCG_REPLICA_SPECIES_MISMATCH;
             break;
@@ -636,6 +693,315 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
     }
 }
 
+// The step loop with one lane per list operation (models and lattices
+// otf_fast_ok names; the others run otf_steps_kernel).
+//
+// A step of the intZGB model has 13 to 23 deletes, 40 to 62 rate updates and
+// 5 to 13 adds on ten lists.  An owner lane that walks its own ones waits for
+// two or three dependent reads per operation and looks its bystanders up one
+// by one (40,000 of a step's 80,000 cycles).  Here every operation of the
+// executed process is a lane (two rounds of 64): inverse index, old rate,
+// conditions and new rate of all of them are found at once, and the owner
+// lanes only apply what takes place, in the reference's order, from LDS.
+// Deletes precede updates and adds and name each (process, cell) once, so an
+// entry's place changes only by the moves of the deletes, which stay in
+// registers.
+//
+// Op records of an executed process (global memory, read while its cell is
+// searched): 64 owner words: first op | ops << 8 | deletes << 16 | updates << 24;
+// then 128 pairs: kind (0 delete, 1 none, 2 update, 3 add) | process << 2 |
+// same cell updated before << 8 | conditions << 9 | their LDS word << 16;
+// dx, dy, dz (8 bits each).
+constexpr int OTF_OPS = 128;
+constexpr int OTF_FREC = 64 + 2 * OTF_OPS;
+
+__global__ __launch_bounds__(64) void otf_fast_kernel(OtfParams p)
+{
+    extern __shared__ __align__(16) int otf_smem[];
+    const int r = p.rep_ids[blockIdx.x];
+    const int lane = threadIdx.x;
+    const int P = p.P;
+    const OtfCell g{p.dims[4 * r], p.dims[4 * r + 1], p.dims[4 * r + 2], p.dims[4 * r + 3]};
+    const int V = g.C * p.spuck;
+    // LDS: program words, rate table, the operations' results, lattice
+    int *prog = otf_smem;
+    double *tab = reinterpret_cast<double *>(otf_smem + ((p.FW + 1) & ~1));
+    double *eold = tab + p.T, *enew = eold + OTF_OPS;
+    int *ecell = reinterpret_cast<int *>(enew + OTF_OPS), *eback = ecell + OTF_OPS;
+    signed char *slat = reinterpret_cast<signed char *>(eback + OTF_OPS);
+    signed char *glat = p.lat + p.lat_off[r];
+    for (int i = lane; i < p.FW; i += 64)
+        prog[i] = p.fast[i];
+    for (int i = lane; i < p.T; i += 64)
+        tab[i] = p.table[(long long)r * p.T + i];
+    for (int i = lane; i < V; i += 64)
+        slat[i] = glat[i];
+    __syncthreads();
+    int st = p.status[r];
+    if (st != KMCG_REPLICA_OK)
+        return;
+    const int *recs = p.fast + p.FW;
+    const bool act = lane < P;
+    const int q = act ? lane : 0;
+    const long long base = p.list_off[r], crow = otf_row(g.C);
+    const long long lo = base + q * crow;
+    int *srow = p.sites + lo;
+    int *brow = p.back + lo;
+    double *rrow = p.rm + lo;
+    double *chk = p.pre + lo / OTF_BLK;
+    const int slot = r * P + q;
+    int n = act ? p.nsites[slot] : 0;
+    double tot = (act && n > 0) ? otf_prefix(rrow, chk, n - 1) : 0.0;
+    double integ = act ? p.integ[slot] : 0.0;
+    double run = act ? p.runsum[slot] : 0.0;
+    double my_acc = act ? p.accum[slot] : 0.0;
+    long long pstat = act ? p.procstat[slot] : 0;
+    double t = p.kmc_time[r];
+    double t_step = p.kmc_time_step[r];
+    const long long kstep0 = p.kmc_step[r];
+    const unsigned long long ctr0 = p.ctr[r];
+    const unsigned seed = p.seed[r], stream = p.stream[r];
+    double lmlog = 0.0, lu1 = 0.0, lu2 = 0.0;
+    long long s = 0;
+    for (; s < p.steps; ++s) {
+        // uniforms of 64 steps at a time: lane i draws step s + i
+        const int uj = (int)s & 63;
+        if (uj == 0) {
+            const FzUni un = fz_uniforms(seed, stream, ctr0 + (unsigned long long)s + lane);
+            lmlog = un.mlog;
+            lu1 = un.u1;
+            lu2 = un.u2;
+        }
+        // update_accum_rate: accum(i) = accum(i-1) + sum of list i
+        double acc = 0.0;
+        for (int i = 0; i < P; ++i) {
+            const double ti = readlane_d(tot, i);
+            acc = i == 0 ? ti : acc + ti;
+            if (lane == i)
+                my_acc = acc;
+        }
+        run = tot;
+        const double total = acc;
+        if (!(total > 0.0)) {
+            st = KMCG_REPLICA_ABSORBING;
+            break;
+        }
+        // update_clocks, update_integ_rate
+        const double dt = readlane_d(lmlog, uj) / total;
+        t_step = dt;
+        t = t + dt;
+        integ = integ + tot * dt;
+        // determine_procsite (the process: see otf_steps_kernel)
+        const double v = readlane_d(lu1, uj) * total;
+        const unsigned long long mp = __ballot(act && my_acc > v);
+        int proc = mp ? __ffsll((long long)mp) - 1 : P - 1;
+        if (!mp)
+            while (proc > 0 && readlane_d(my_acc, proc - 1) >= readlane_d(my_acc, proc))
+                --proc;
+        // its records are on their way during the search
+        const int *rec = recs + proc * OTF_FREC;
+        const int own = rec[lane];
+        const int2 op0 = ((const int2 *)(rec + 64))[lane], op1 = ((const int2 *)(rec + 64))[64 + lane];
+        const int np = readlane_i(n, proc);
+        const double vs = readlane_d(lu2, uj) * readlane_d(tot, proc);
+        const int cell = otf_pick(p.sites + base + proc * crow, p.rm + base + proc * crow,
+                                  p.pre + (base + proc * crow) / OTF_BLK, np, vs, lane);
+        int x, y, z;
+        g.xyz(cell, x, y, z);
+        if (lane == proc)
+            pstat += 1;
+        // every operation's cell and inverse index
+        int oc[2], ob[2], ocx[2], ocy[2], ocz[2], okind[2], oq[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int2 o = h ? op1 : op0;
+            okind[h] = o.x & 3;
+            oq[h] = (o.x >> 2) & 63;
+            ocx[h] = otf_wrap(x + sx8(o.y, 0), g.X);
+            ocy[h] = otf_wrap(y + sx8(o.y, 8), g.Y);
+            ocz[h] = otf_wrap(z + sx8(o.y, 16), g.Z);
+            oc[h] = g.idx(ocx[h], ocy[h], ocz[h]);
+            ob[h] = p.back[base + oq[h] * crow + oc[h]];
+        }
+        // lattice writes
+        const int wt = prog[p.off_fw + proc];
+        bool bad = false;
+        if (lane < (wt >> 16)) {
+            const int *ww = prog + (wt & 0xFFFF) + 2 * lane;
+            const int c = g.at(x, y, z, sx8(ww[0], 0), sx8(ww[0], 8), sx8(ww[0], 16));
+            const int site = p.spuck * c + ((ww[0] >> 24) & 0xFF);
+            bad = slat[site] != (ww[1] & 0xFFFF);
+            slat[site] = (signed char)(ww[1] >> 16);
+        }
+        __syncthreads();
+        // which take place, old and new rates
+        bool corrupt = false;
+        unsigned long long on[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int2 o = h ? op1 : op0;
+            const int nq = __builtin_amdgcn_ds_bpermute(oq[h] << 2, n);
+            const bool listed = okind[h] != 1 && okind[h] != 3 && ob[h] != 0;
+            const bool off = listed && (ob[h] < 0 || ob[h] > nq);
+            corrupt = corrupt || off;
+            bool take = listed && !off;
+            double old = 0.0, rate = 0.0;
+            if (take)
+                old = p.rm[base + oq[h] * crow + ob[h] - 1];
+            if (okind[h] == 3)
+                take = otf_conds(p, g, slat, prog + (int)((unsigned)o.x >> 16), (o.x >> 9) & 0x3F, x, y, z);
+            if (take && okind[h] >= 2) {
+                const int bt = prog[p.off_fb + oq[h]], nb = bt >> 16;
+                const int *b = prog + (bt & 0xFFFF);
+                int idx = prog[p.off_ft + oq[h]];
+                for (int k0 = 0; k0 < nb; k0 += 4) {
+                    int sw[4], sp[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        sw[k] = b[min(k0 + k, nb - 1) * (1 + p.S)];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        sp[k] = slat[p.spuck * g.at(ocx[h], ocy[h], ocz[h], sx8(sw[k], 0), sx8(sw[k], 8), sx8(sw[k], 16)) +
+                                     ((sw[k] >> 24) & 0xFF)];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k0 + k < nb && sp[k] >= 0 && sp[k] < p.S)
+                            idx += b[(k0 + k) * (1 + p.S) + 1 + sp[k]];
+                }
+                rate = tab[idx];
+            }
+            const int e = 64 * h + lane;
+            ecell[e] = oc[h];
+            eback[e] = ob[h];
+            eold[e] = (o.x >> 8) & 1 ? rate : old;      // updated before in this step: its new rate
+            enew[e] = rate;
+            on[h] = __ballot(take);
+        }
+        // this owner lane's run of operations
+        const int first = own & 0xFF, ndel = (own >> 16) & 0xFF, nupd = (own >> 24) & 0xFF;
+        unsigned bits;
+        {
+            const unsigned long long l0 = on[0] >> (first & 63), l1 = on[1] >> (first & 63);
+            const unsigned long long up = (first & 63) ? on[1] << (64 - (first & 63)) : 0ull;
+            bits = (unsigned)(first < 64 ? l0 | up : l1);
+            const int len = (own >> 8) & 0xFF;
+            bits = act ? bits & ((1u << len) - 1u) : 0u;
+        }
+        int dirty = 0x7fffffff;
+        __syncthreads();
+        // deletes (del_proc, base_otf.f90:221-282): the last entry moves
+        // into the freed place
+        unsigned db = bits & ((1u << ndel) - 1u);
+        {
+            const int n0 = n, nd = __popc(db);
+            int tc[4];
+            double tr[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                tc[i] = i < nd && n0 - 1 - i >= 0 ? srow[n0 - 1 - i] : 0;
+                tr[i] = i < nd && n0 - 1 - i >= 0 ? rrow[n0 - 1 - i] : 0.0;
+            }
+            int mvc[4] = {0, 0, 0, 0}, mvp[4] = {0, 0, 0, 0};
+            double mvr[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (db) {
+                    const int e = first + __builtin_ctz(db);
+                    db &= db - 1;
+                    const int c = ecell[e];
+                    int pos = eback[e] - 1;
+                    const double gone = eold[e];
+                    const int last = n - 1;
+                    int mv = tc[i];
+                    double mr = tr[i];
+#pragma unroll
+                    for (int j = 0; j < i; ++j) {
+                        pos = mvc[j] == c + 1 ? mvp[j] : pos;
+                        mr = mvc[j] && mvp[j] == last ? mvr[j] : mr;
+                        mv = mvc[j] && mvp[j] == last ? mvc[j] : mv;
+                    }
+                    run = run - gone;
+                    int changed = last;
+                    if (pos < last) {
+                        srow[pos] = mv;
+                        rrow[pos] = mr;
+                        brow[mv - 1] = pos + 1;
+                        if (mr != gone)
+                            changed = pos;
+                        mvc[i] = mv;
+                        mvp[i] = pos;
+                        mvr[i] = mr;
+                    }
+                    srow[last] = 0;
+                    rrow[last] = 0.0;
+                    brow[c] = 0;
+                    n = last;
+                    dirty = min(dirty, changed);
+                }
+            }
+            // rate updates, in program order
+            for (unsigned ub = (bits >> ndel) & ((1u << nupd) - 1u); ub; ub &= ub - 1) {
+                const int e = first + ndel + __builtin_ctz(ub);
+                const int c = ecell[e];
+                int pos = eback[e] - 1;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    pos = mvc[j] == c + 1 ? mvp[j] : pos;
+                const double old = eold[e], rate = enew[e];
+                run = run + rate - old;
+                rrow[pos] = rate;
+                if (rate != old)
+                    dirty = min(dirty, pos);
+            }
+        }
+        // adds, in program order
+        for (unsigned ab = bits >> (ndel + nupd); ab; ab &= ab - 1) {
+            const int e = first + ndel + nupd + __builtin_ctz(ab);
+            const int c = ecell[e];
+            const double rate = enew[e];
+            if (n >= g.C) {
+                corrupt = true;             // an add to a full list
+            } else {
+                srow[n] = c + 1;
+                brow[c] = n + 1;
+                rrow[n] = rate;
+                run = run + rate;
+                dirty = min(dirty, n);
+                n += 1;
+            }
+        }
+        tot = otf_resum_wave(p.rm + base, crow, chk, act && dirty != 0x7fffffff, min(dirty, n), n, tot, eold, ecell,
+                             lane);
+        if (__ballot(bad)) {
+            st = KMCG_REPLICA_SPECIES_MISMATCH;
+            s += 1;
+            break;
+        }
+        if (__ballot(corrupt)) {
+            st = KMCG_REPLICA_CORRUPT;
+            s += 1;
+            break;
+        }
+    }
+    __syncthreads();
+    for (int i = lane; i < V; i += 64)
+        glat[i] = slat[i];
+    if (act) {
+        p.nsites[slot] = n;
+        p.procstat[slot] = pstat;
+        p.integ[slot] = integ;
+        p.accum[slot] = my_acc;
+        p.runsum[slot] = run;
+    }
+    if (lane == 0) {
+        p.kmc_time[r] = t;
+        p.kmc_time_step[r] = t_step;
+        p.kmc_step[r] = kstep0 + s;
+        p.ctr[r] = ctr0 + (unsigned long long)s;
+        p.status[r] = st;
+    }
+}
+
 } // namespace
 
 // ===========================================================================
@@ -647,6 +1013,11 @@ struct kmcg_otf_model {
     int reach[3] = {0, 0, 0};        // largest |offset| per dimension
     std::vector<int> prog;           // the device program (see build)
     int off_owner = 0, off_writes = 0, off_byst = 0, off_tbase = 0, off_touch = 0;
+    // otf_fast_kernel's words (empty: not for this model): FW LDS words, then
+    // the op records; the largest offset of an operation per dimension
+    std::vector<int> fast;
+    int FW = 0, off_fw = 0, off_fb = 0, off_ft = 0;
+    int op_reach[3] = {0, 0, 0};
 };
 
 struct kmcg_otf_batch {
@@ -798,6 +1169,95 @@ int otf_op_word(int kind, int dx, int dy, int dz, int ncond)
 int otf_cond_word(int dx, int dy, int dz, int n1, int sp)
 {
     return (dx & 0x7F) | (dy & 0x7F) << 7 | (dz & 0x7F) << 14 | (n1 - 1) << 21 | sp << 26;
+}
+
+// The words of otf_fast_kernel.  Leaves m->fast empty for models it does not
+// take: more than 128 operations of one process or 31 on one list, more than
+// four deletes on one list, an update behind an add.
+void otf_build_fast(kmcg_otf_model *m, const std::vector<std::vector<std::vector<int>>> &own,
+                    const std::vector<std::vector<int>> &writes)
+{
+    const int P = m->P;
+    std::vector<int> w;
+    const std::vector<int> &g = m->prog;
+    m->off_fw = 0;
+    w.resize(P);
+    m->off_fb = (int)w.size();
+    w.resize(w.size() + P);
+    m->off_ft = (int)w.size();
+    w.insert(w.end(), g.begin() + m->off_tbase, g.begin() + m->off_tbase + P);
+    for (int p = 0; p < P; ++p) {
+        w[m->off_fw + p] = (int)w.size() | (int)(writes[p].size() / 2) << 16;
+        w.insert(w.end(), writes[p].begin(), writes[p].end());
+    }
+    for (int q = 0; q < P; ++q) {
+        const int bt = g[m->off_byst + q], nb = bt >> 16;
+        w[m->off_fb + q] = (int)w.size() | nb << 16;
+        w.insert(w.end(), g.begin() + (bt & 0xFFFF), g.begin() + (bt & 0xFFFF) + nb * (1 + m->S));
+    }
+    std::map<std::vector<int>, int> pool;                // condition lists already placed
+    std::vector<int> rec((size_t)P * OTF_FREC, 0);
+    int reach[3] = {0, 0, 0};
+    for (int p = 0; p < P; ++p) {
+        int *r = &rec[(size_t)p * OTF_FREC];
+        for (int j = 0; j < OTF_OPS; ++j)
+            r[64 + 2 * j] = 1;
+        int at = 0;
+        for (int q = 0; q < P; ++q) {
+            const std::vector<int> &ops = own[p][q];
+            const int first = at;
+            int nd = 0, nu = 0, na = 0;
+            std::vector<int> gone, seen;                 // cells deleted, updated
+            for (size_t i = 0; i < ops.size();) {
+                const int op = ops[i], kind = op & 3, ncond = (op >> 26) & 0x3F, cellw = (op >> 2) & 0xFFFFFF;
+                const std::vector<int> conds(ops.begin() + i + 1, ops.begin() + i + 1 + (kind == 3 ? ncond : 0));
+                i += 1 + conds.size();
+                for (int d = 0; d < 3; ++d)
+                    reach[d] = std::max(reach[d], std::abs((int)(signed char)((cellw >> (8 * d)) & 0xFF)));
+                const bool was = std::find(gone.begin(), gone.end(), cellw) != gone.end();
+                int dup = 0, cat = 0;
+                if (kind == 0) {
+                    if (nu || na)
+                        return;
+                    if (was)
+                        continue;                        // finds nothing the second time
+                    gone.push_back(cellw);
+                    nd += 1;
+                } else if (kind == 2) {
+                    if (na)
+                        return;
+                    if (was)
+                        continue;                        // its entry is deleted in this step
+                    dup = std::find(seen.begin(), seen.end(), cellw) != seen.end() ? 1 : 0;
+                    seen.push_back(cellw);
+                    nu += 1;
+                } else {
+                    na += 1;
+                    const auto it = pool.emplace(conds, (int)w.size());
+                    if (it.second)
+                        w.insert(w.end(), conds.begin(), conds.end());
+                    cat = it.first->second;
+                }
+                if (at >= OTF_OPS || cat > 65535)
+                    return;
+                r[64 + 2 * at] = kind | q << 2 | dup << 8 | (kind == 3 ? ncond : 0) << 9 | (int)((unsigned)cat << 16);
+                r[64 + 2 * at + 1] = cellw;
+                at += 1;
+            }
+            if (nd > 4 || nd + nu + na > 31)
+                return;
+            r[q] = first | (nd + nu + na) << 8 | nd << 16 | nu << 24;
+        }
+    }
+    if (w.size() > 65535)
+        return;
+    while (w.size() % 4)
+        w.push_back(0);
+    m->FW = (int)w.size();
+    w.insert(w.end(), rec.begin(), rec.end());
+    m->fast.swap(w);
+    for (int d = 0; d < 3; ++d)
+        m->op_reach[d] = reach[d];
 }
 
 int otf_build(kmcg_otf_model *m)
@@ -966,6 +1426,7 @@ int otf_build(kmcg_otf_model *m)
         return fail(KMCG_EUNSUPPORTED, "otf program too large for the engine (" + std::to_string(g.size()) +
                                        " words)");
     m->T = (int)T;
+    otf_build_fast(m, own, writes);
     return KMCG_OK;
 }
 
@@ -977,6 +1438,8 @@ OtfParams otf_params(kmcg_otf_batch *b, long long steps, int mode)
     p.prog = b->d_prog;
     p.off_owner = m->off_owner; p.off_writes = m->off_writes; p.off_byst = m->off_byst;
     p.off_tbase = m->off_tbase; p.off_touch = m->off_touch;
+    p.fast = b->d_prog + ((m->prog.size() + 3) & ~(size_t)3);
+    p.FW = m->FW; p.off_fw = m->off_fw; p.off_fb = m->off_fb; p.off_ft = m->off_ft;
     p.dims = b->d_dims; p.lat_off = b->d_lat_off; p.list_off = b->d_list_off;
     p.lat = b->d_lat; p.sites = b->d_sites; p.back = b->d_back; p.rm = b->d_rm; p.pre = b->d_pre;
     p.nsites = b->d_nsites; p.procstat = b->d_procstat; p.integ = b->d_integ; p.accum = b->d_accum;
@@ -1021,9 +1484,20 @@ int otf_launch(kmcg_otf_batch *b, int32_t r0, int32_t n, long long steps, int mo
     const size_t prog_bytes = (size_t)((p.W + 1) & ~1) * 4;
     const size_t tab_bytes = (size_t)b->m->T * 8;
     p.tab_lds = prog_bytes + tab_bytes + (size_t)b->maxV <= (size_t)OTF_LDS;
+    // one lane per operation: 41 -> 24 us per step on 2048 replicas of the
+    // intZGB model at 64x64 (RuO2, one 20x20 replica: 7.7 -> 5.2), and
+    // faster at every size measured.  It needs the table in LDS and extents
+    // on which no two offsets of the operations meet.
+    const size_t fast_bytes = (size_t)((b->m->FW + 1) & ~1) * 4 + tab_bytes + OTF_OPS * 24 + (size_t)b->maxV;
+    bool fast = mode < 0 && !b->m->fast.empty() && fast_bytes <= (size_t)OTF_LDS;
+    for (int i = 0; i < n && fast; ++i)
+        for (int d = 0; d < 3; ++d)
+            fast = fast && b->dims[4 * (r0 + i) + d] >= 2 * b->m->op_reach[d] + 1;
     if (timed)
         HIPCHK(hipEventRecord(b->ev0, b->stream));
-    if (mode < 0 && p.tab_lds)
+    if (fast)
+        hipLaunchKernelGGL(otf_fast_kernel, dim3(n), dim3(64), fast_bytes, b->stream, p);
+    else if (mode < 0 && p.tab_lds)
         hipLaunchKernelGGL(otf_steps_kernel<true>, dim3(n), dim3(64), prog_bytes + tab_bytes + b->maxV,
                            b->stream, p);
     else if (mode < 0)
@@ -1177,7 +1651,7 @@ int kmcg_otf_batch_create(const kmcg_otf_model *m, int32_t n, const int32_t *siz
         b->lat_off[r] = b->lat_total;
         b->lat_total += (long long)C * m->spuck;
         b->list_off[r] = b->list_total;
-        b->list_total += (long long)C * m->P;
+        b->list_total += otf_row(C) * m->P;
         b->maxV = std::max(b->maxV, C * m->spuck);
     }
     b->rates.assign((size_t)n * m->P, 0.0);
@@ -1190,8 +1664,11 @@ int kmcg_otf_batch_create(const kmcg_otf_model *m, int32_t n, const int32_t *siz
         hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess)
         return bail(KMCG_EHIP, "stream or event creation failed");
     const size_t P = m->P;
+    std::vector<int> progs(m->prog);                     // the program, then the fast kernel's words
+    progs.resize((progs.size() + 3) & ~(size_t)3, 0);
+    progs.insert(progs.end(), m->fast.begin(), m->fast.end());
     struct A { void **p; size_t bytes; } allocs[] = {
-        {(void **)&b->d_prog, m->prog.size() * sizeof(int)},
+        {(void **)&b->d_prog, progs.size() * sizeof(int)},
         {(void **)&b->d_dims, b->dims.size() * sizeof(int)},
         {(void **)&b->d_rep, (size_t)n * sizeof(int)},
         {(void **)&b->d_lat_off, (size_t)n * sizeof(long long)},
@@ -1200,7 +1677,7 @@ int kmcg_otf_batch_create(const kmcg_otf_model *m, int32_t n, const int32_t *siz
         {(void **)&b->d_sites, (size_t)b->list_total * sizeof(int)},
         {(void **)&b->d_back, (size_t)b->list_total * sizeof(int)},
         {(void **)&b->d_rm, (size_t)b->list_total * sizeof(double)},
-        {(void **)&b->d_pre, (size_t)b->list_total * sizeof(double)},
+        {(void **)&b->d_pre, (size_t)(b->list_total / OTF_BLK) * sizeof(double)},
         {(void **)&b->d_nsites, n * P * sizeof(int)},
         {(void **)&b->d_status, (size_t)n * sizeof(int)},
         {(void **)&b->d_integ, n * P * sizeof(double)},
@@ -1218,11 +1695,12 @@ int kmcg_otf_batch_create(const kmcg_otf_model *m, int32_t n, const int32_t *siz
     for (auto &a : allocs)
         if (hipMalloc(a.p, std::max(a.bytes, (size_t)8)) != hipSuccess)
             return bail(KMCG_ENOMEM, "device allocation failed for an otf batch");
-    if (hipMemcpy(b->d_prog, m->prog.data(), m->prog.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(b->d_prog, progs.data(), progs.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_dims, b->dims.data(), b->dims.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_lat_off, b->lat_off.data(), n * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_list_off, b->list_off.data(), n * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(b->d_nsites, 0, n * P * sizeof(int)) != hipSuccess ||
+        hipMemset(b->d_rm, 0, (size_t)b->list_total * sizeof(double)) != hipSuccess ||
         hipMemset(b->d_runsum, 0, n * P * sizeof(double)) != hipSuccess ||
         hipMemset(b->d_table, 0, (size_t)n * std::max(m->T, 1) * sizeof(double)) != hipSuccess ||
         hipMemset(b->d_status, 0xff, (size_t)n * sizeof(int)) != hipSuccess)
@@ -1382,8 +1860,9 @@ int kmcg_otf_get_avail(kmcg_otf_batch *b, int32_t r, int32_t *sites, int32_t *ba
         return rc;
     const kmcg_otf_model *m = b->m;
     const int P = m->P, C = b->dims[4 * r + 3], V = C * m->spuck;
-    std::vector<int> s((size_t)P * C), bk((size_t)P * C);
-    std::vector<double> rm((size_t)P * C), run(P);
+    const size_t R = (size_t)otf_row(C);
+    std::vector<int> s(P * R), bk(P * R);
+    std::vector<double> rm(P * R), run(P);
     if ((rc = otf_copy_out(b, s.data(), b->d_sites + b->list_off[r], s.size())) ||
         (rc = otf_copy_out(b, bk.data(), b->d_back + b->list_off[r], bk.size())) ||
         (rc = otf_copy_out(b, rm.data(), b->d_rm + b->list_off[r], rm.size())) ||
@@ -1398,10 +1877,10 @@ int kmcg_otf_get_avail(kmcg_otf_batch *b, int32_t r, int32_t *sites, int32_t *ba
             rates_matrix[(size_t)p * (V + 1) + i] = 0.0;
         }
         for (int i = 0; i < C; ++i) {
-            const int cell1 = s[(size_t)p * C + i];
+            const int cell1 = s[p * R + i];
             sites[(size_t)p * V + i] = cell1 ? (cell1 - 1) * m->spuck + 1 : 0;
-            back[(size_t)p * V + (size_t)i * m->spuck] = bk[(size_t)p * C + i];
-            rates_matrix[(size_t)p * (V + 1) + i] = rm[(size_t)p * C + i];
+            back[(size_t)p * V + (size_t)i * m->spuck] = bk[p * R + i];
+            rates_matrix[(size_t)p * (V + 1) + i] = rm[p * R + i];
         }
         rates_matrix[(size_t)p * (V + 1) + V] = run[p];
     }
