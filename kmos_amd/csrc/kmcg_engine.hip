@@ -2269,6 +2269,20 @@ __global__ __launch_bounds__(256) void kmc_sample_kernel(KParams kp, double *out
     }
 }
 
+// The scalars of one replica into pinned host memory (kmcg_get_scalars): one
+// launch and one wait where a copy each cost five.
+__global__ void kmc_scalars_kernel(KParams kp, int r, double *out)
+{
+    long long *o = (long long *)out;
+    if (threadIdx.x == 0) {
+        out[0] = kp.ktime[r];
+        out[1] = kp.kdt[r];
+        o[2] = kp.kstep[r];
+        o[3] = (long long)kp.rngctr[r];
+        o[4] = kp.status[r];
+    }
+}
+
 } // namespace
 
 // ===========================================================================
@@ -2363,10 +2377,10 @@ struct kmcg_batch {
     long long *executed = nullptr;
     long long *budget = nullptr;
     int *rep_ids = nullptr;
+    const int *run_ids = nullptr;       // the list of the last run
     int *out = nullptr;
     unsigned long long *phase = nullptr;   // phase counters (KMCG_PHASES builds)
     double *occ = nullptr;
-    double *samples = nullptr;
     // pinned staging of a run's replica list and budgets; one run in flight
     int *h_ids = nullptr;
     long long *h_budget = nullptr;
@@ -2376,7 +2390,11 @@ struct kmcg_batch {
     size_t srec_len = 0;                // doubles in each
     double *user_srec = nullptr;
     size_t n_srec = 0;
-    double *h_samples = nullptr;        // pinned staging of sample records
+    // sample records, pinned: the kernels write them there directly, without
+    // a copy; five words behind them for kmcg_get_scalars
+    double *h_samples = nullptr;
+    size_t samples_len = 0;
+    int *iota = nullptr;                // 0, 1, 2, ... on the device: replica lists without gaps
     double *user_samples = nullptr;     // where the records go at the sync
     size_t n_samples = 0;
     int n_last = 0;
@@ -3510,14 +3528,23 @@ int check_replica(kmcg_batch *b, int r)
 
 int settle(kmcg_batch *b);
 
+// first replica of a list without gaps (its place in b->iota), or -1
+int contiguous(const int32_t *ids, int n)
+{
+    for (int i = 1; i < n; ++i)
+        if (ids[i] != ids[0] + i)
+            return -1;
+    return ids[0];
+}
+
 // run the misc kernel for replicas [ids] synchronously
 int run_misc(kmcg_batch *b, const std::vector<int> &ids, int mode, int a0, int a1, int a2, int a3)
 {
     int rc = settle(b);
     if (rc)
         return rc;
-    HIPCHK(hipMemcpyAsync(b->rep_ids, ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
     KParams kp = make_params(b);
+    kp.rep_ids = b->iota + ids[0];                       // (consecutive replicas)
     const Shape s = launch_shape(b, ids.data(), (int)ids.size(), kp, MAX_WPG);
     kp.mode = mode;
     kp.arg0 = a0; kp.arg1 = a1; kp.arg2 = a2; kp.arg3 = a3;
@@ -3700,7 +3727,7 @@ void kmcg_batch_free(kmcg_batch *b)
     void *ptrs[] = {b->prog, b->dims, b->lat_off_d, b->avail_off_d, b->seed, b->strm, b->lat_pool,
                     b->avail_pool, b->nr, b->rates, b->integ, b->pstat, b->ktime, b->kdt, b->kstep,
                     b->rngctr, b->status, b->executed, b->budget, b->rep_ids, b->out, b->occ,
-                    b->samples, b->msd_hop, b->msd_d, b->msd_id, b->msd_site, b->msd_disp,
+                    b->msd_hop, b->msd_d, b->msd_id, b->msd_site, b->msd_disp,
                     b->msd_off_d, b->msd_ev, b->msd_evn, b->lists_ok, b->acf_pa, b->acf_po, b->acf_buf,
                     b->acf_pp, b->acf_bin, b->acf_cnt, b->acf_boff, b->acf_d, b->acf_i, b->phase};
     for (void *p : ptrs)
@@ -3785,7 +3812,8 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     BALLOC(b->prog, fz_at + m->fz.size());
     b->fz = b->prog + fz_at;
     b->lists_ok_h.assign(n, 0);
-    BALLOC(b->dims, n);
+    BALLOC(b->dims, n + (n + 3) / 4);            // then the list 0, 1, 2, ...
+    b->iota = (int *)(b->dims + n);
     BALLOC(b->lat_off_d, n);
     BALLOC(b->avail_off_d, n);
     BALLOC(b->seed, n);
@@ -3810,13 +3838,16 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     BALLOC(b->phase, (size_t)n * PHASE_W);
 #endif
     BALLOC(b->occ, (size_t)n * m->S * m->spuck);
-    BALLOC(b->samples, (size_t)n * (4 + m->S * m->spuck + 2 * P));
+    b->samples_len = (size_t)n * (4 + m->S * m->spuck + 2 * P);
     if (hipHostMalloc((void **)&b->h_ids, n * sizeof(int), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&b->h_budget, n * sizeof(long long), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&b->h_samples, (size_t)n * (4 + m->S * m->spuck + 2 * P) * sizeof(double),
-                      hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void **)&b->h_samples, (b->samples_len + 8) * sizeof(double), hipHostMallocDefault) !=
+            hipSuccess)
         return bail(fail(KMCG_ENOMEM, "pinned host allocation failed"));
 #undef BALLOC
+    dims.resize(n + (n + 3) / 4);
+    for (int i = 0; i < n; ++i)
+        ((int *)(dims.data() + n))[i] = i;
     auto H2D = [&](void *d, const void *h, size_t bytes) {
         return hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, b->stream) == hipSuccess;
     };
@@ -3824,7 +3855,7 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     progs.resize(fz_at, 0);
     progs.insert(progs.end(), m->fz.begin(), m->fz.end());
     if (!H2D(b->prog, progs.data(), progs.size() * sizeof(int)) ||
-        !H2D(b->dims, dims.data(), n * sizeof(int4)) ||
+        !H2D(b->dims, dims.data(), dims.size() * sizeof(int4)) ||
         !H2D(b->lat_off_d, b->lat_off.data(), n * sizeof(long long)) ||
         !H2D(b->avail_off_d, b->avail_off.data(), n * sizeof(long long)))
         return bail(fail(KMCG_EHIP, "copy to device failed"));
@@ -3869,31 +3900,52 @@ int kmcg_set_launch(kmcg_batch *b, int32_t lattice_in_lds, int32_t waves_per_gro
     return KMCG_OK;
 }
 
-static int pack_config(kmcg_batch *b, int r, const int8_t *config, std::vector<unsigned char> &packed)
+// The lattices of replicas [r0, r0+n) as the device holds them, one after the
+// other as in lat_pool: one copy sends them all.
+static int pack_configs(kmcg_batch *b, int r0, int n, const int8_t *config, std::vector<unsigned char> &packed)
 {
-    const int V = b->V[r];
-    for (int s = 0; s < V; ++s)
-        if (!b->m->species_ok(config[s]))
+    const long long base = b->lat_off[r0];
+    packed.assign((size_t)((r0 + n < b->n ? b->lat_off[r0 + n] : b->lat_total) - base), 0);
+    for (int r = r0; r < r0 + n; ++r) {
+        const int V = b->V[r];
+        unsigned char *out = packed.data() + (b->lat_off[r] - base);
+        // species 0..S-1, or S where it is the null species
+        const unsigned most = b->m->nullsp >= 0 ? b->m->S : b->m->S - 1;
+        unsigned bad = 0;
+        for (int s = 0; s < V; ++s)
+            bad |= (unsigned)((unsigned char)config[s] > most);
+        if (bad)
             return fail(KMCG_EINVAL, "configuration holds an unknown species");
-    packed.assign(lattice_bytes(V, b->bits), 0);
-    if (b->bits == 8) {
-        for (int s = 0; s < V; ++s)
-            packed[s] = (unsigned char)config[s];
-    } else {
-        for (int s = 0; s < V; ++s)
-            packed[(s * 2) >> 3] |= (unsigned char)(((config[s] + 1) & 3) << ((s * 2) & 7));
+        if (b->bits == 8) {
+            memcpy(out, config, V);
+        } else {
+            // four sites a byte: their low bits meet in the top byte of one
+            // product (4.3 million sites: 5 ms one by one)
+            int s = 0;
+            for (; s + 4 <= V; s += 4) {
+                uint32_t x;
+                memcpy(&x, config + s, 4);
+                out[s >> 2] = (unsigned char)(((x + 0x01010101u) * 0x01041040u) >> 24);
+            }
+            for (; s < V; ++s)
+                out[s >> 2] |= (unsigned char)((config[s] + 1) << ((s & 3) * 2));
+        }
+        config += V;
     }
     return KMCG_OK;
 }
 
 namespace {
 // mark replicas [r0, r0+n) as having lists that do (1) or may not (0) match
-// their lattices
+// their lattices, behind the batch's queued work, and wait for both
 int set_lists_ok(kmcg_batch *b, int r0, int n, int v)
 {
-    std::vector<int> f(n, v);
-    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)v);
-    return copy_in(b, b->lists_ok + r0, f.data(), (size_t)n);
+    HIPCHK(hipSetDevice(b->device));
+    HIPCHK(hipMemsetD32Async((hipDeviceptr_t)(b->lists_ok + r0), v, n, b->stream));
+    const int rc = settle(b);
+    if (!rc)
+        std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)v);
+    return rc;
 }
 } // namespace
 
@@ -3907,16 +3959,11 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
         return rc0;
     // every configuration is checked before any replica is touched, so a
     // rejected call leaves all replicas as they were
-    std::vector<std::vector<unsigned char>> packed;   // alive until the stream is synchronised
+    std::vector<unsigned char> packed;       // alive until the stream is synchronised
     if (configs) {
-        long long off = 0;
-        packed.resize(n);
-        for (int i = 0; i < n; ++i) {
-            const int rc = pack_config(b, r0 + i, configs + off, packed[i]);
-            if (rc)
-                return rc;
-            off += b->V[r0 + i];
-        }
+        const int rc = pack_configs(b, r0, n, configs, packed);
+        if (rc)
+            return rc;
     }
     const long long P = b->m->P;
     std::vector<unsigned> st(n, 0u);
@@ -3935,15 +3982,11 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
     const long long a0 = b->avail_off[r0];
     const long long a1 = (r0 + n < b->n) ? b->avail_off[r0 + n] : b->avail_total;
     HIPCHK(hipMemsetAsync(b->avail_pool + a0, 0, (a1 - a0) * sizeof(int), b->stream));
-    std::vector<int> ids(n);
-    for (int i = 0; i < n; ++i)
-        ids[i] = r0 + i;
-    HIPCHK(hipMemcpyAsync(b->rep_ids, ids.data(), n * sizeof(int), hipMemcpyHostToDevice, b->stream));
     KParams kp = make_params(b);
+    kp.rep_ids = b->iota + r0;
     if (configs) {
-        for (int i = 0; i < n; ++i)
-            HIPCHK(hipMemcpyAsync(b->lat_pool + b->lat_off[r0 + i], packed[i].data(), packed[i].size(),
-                                  hipMemcpyHostToDevice, b->stream));
+        HIPCHK(hipMemcpyAsync(b->lat_pool + b->lat_off[r0], packed.data(), packed.size(), hipMemcpyHostToDevice,
+                              b->stream));
     } else if (b->bits == 2) {
         hipLaunchKernelGGL((kmc_fill_default_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp);
     } else {
@@ -3957,7 +4000,6 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
     else
         hipLaunchKernelGGL((kmc_init_lists_kernel<8>), grid, dim3(256), 0, b->stream, kp);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(b->stream));
     return set_lists_ok(b, r0, n, 1);
 }
 
@@ -4021,29 +4063,20 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
         return fail(KMCG_EINVAL, "bad replica range");
     // every configuration is checked before any lattice is replaced, so a
     // rejected call leaves all replicas as they were
-    long long off = 0;
-    std::vector<int> ids(n);
-    std::vector<std::vector<unsigned char>> packed(n);
-    for (int i = 0; i < n; ++i) {
-        const int rc = pack_config(b, r0 + i, config + off, packed[i]);
-        if (rc)
-            return rc;
-        off += b->V[r0 + i];
-        ids[i] = r0 + i;
-    }
-    int rc = settle(b);
-    if (rc)
+    std::vector<unsigned char> packed;
+    int rc = pack_configs(b, r0, n, config, packed);
+    if (rc || (rc = settle(b)))
         return rc;
+    HIPCHK(hipMemcpyAsync(b->lat_pool + b->lat_off[r0], packed.data(), packed.size(), hipMemcpyHostToDevice, b->stream));
+    std::vector<int> ids(n);
     long long cells = 0;
     for (int i = 0; i < n; ++i) {
-        const int r = r0 + i;
-        cells = std::max(cells, (long long)b->X[r] * b->Y[r] * b->Z[r]);
-        HIPCHK(hipMemcpyAsync(b->lat_pool + b->lat_off[r], packed[i].data(), packed[i].size(), hipMemcpyHostToDevice,
-                              b->stream));
+        ids[i] = r0 + i;
+        cells = std::max(cells, (long long)b->X[r0 + i] * b->Y[r0 + i] * b->Z[r0 + i]);
     }
     if (b->m->adjust_lists) {
-        HIPCHK(hipMemcpyAsync(b->rep_ids, ids.data(), n * sizeof(int), hipMemcpyHostToDevice, b->stream));
         KParams kp = make_params(b);
+        kp.rep_ids = b->iota + r0;
         kp.arg0 = b->m->off_init;
         const dim3 grid((unsigned)(n * b->m->P));
         // the list and its inverse index in LDS while both fit
@@ -4058,7 +4091,6 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
         else
             hipLaunchKernelGGL((kmc_adjust_lists_kernel<8, false>), grid, dim3(256), 0, b->stream, kp);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(b->stream));
         return set_lists_ok(b, r0, n, 1);
     }
     rc = run_misc(b, ids, MODE_ADJUST, 0, 0, 0, 0);
@@ -4083,10 +4115,15 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     int rc = settle(b);      // the staging buffers belong to one run at a time
     if (rc)
         return rc;
-    memcpy(b->h_ids, replicas, n * sizeof(int));
+    const int first = contiguous(replicas, n);           // no list to send then
+    if (first < 0)
+        memcpy(b->h_ids, replicas, n * sizeof(int));
     if (budget)
         memcpy(b->h_budget, budget, n * sizeof(long long));
     KParams kp = make_params(b);
+    if (first >= 0)
+        kp.rep_ids = b->iota + first;
+    b->run_ids = kp.rep_ids;
     const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg, true);
     kp.nsteps = steps;
     kp.budget = budget ? b->budget : nullptr;
@@ -4138,7 +4175,9 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     // the stream work of the run; `timed` brackets the kernel with the
     // batch's events (not inside a graph: a replay is timed as a whole)
     auto enqueue = [&](bool timed) -> hipError_t {
-        hipError_t e = hipMemcpyAsync(b->rep_ids, b->h_ids, n * sizeof(int), hipMemcpyHostToDevice, b->stream);
+        hipError_t e = hipSuccess;
+        if (first < 0)
+            e = hipMemcpyAsync(b->rep_ids, b->h_ids, n * sizeof(int), hipMemcpyHostToDevice, b->stream);
         if (e == hipSuccess && budget)
             e = hipMemcpyAsync(b->budget, b->h_budget, n * sizeof(long long), hipMemcpyHostToDevice, b->stream);
         if (e == hipSuccess && timed)
@@ -4237,17 +4276,15 @@ int kmcg_run_sampled(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t 
     int rc = kmcg_run(b, replicas, n, steps, budget);
     if (rc)
         return rc;
-    // the run left the replica list in rep_ids; the records follow it on the
-    // same stream
+    // the records follow the run on the same stream
     const int width = 4 + b->m->S * b->m->spuck + 2 * b->m->P;
     KParams kp = make_params(b);
+    kp.rep_ids = b->run_ids;
     if (b->bits == 2)
-        hipLaunchKernelGGL((kmc_sample_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp, b->samples, width);
+        hipLaunchKernelGGL((kmc_sample_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp, b->h_samples, width);
     else
-        hipLaunchKernelGGL((kmc_sample_kernel<8>), dim3(n), dim3(256), 0, b->stream, kp, b->samples, width);
+        hipLaunchKernelGGL((kmc_sample_kernel<8>), dim3(n), dim3(256), 0, b->stream, kp, b->h_samples, width);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(b->h_samples, b->samples, (size_t)n * width * sizeof(double), hipMemcpyDeviceToHost,
-                          b->stream));
     b->user_samples = samples;
     b->n_samples = (size_t)n * width;
     return KMCG_OK;
@@ -4382,11 +4419,15 @@ int kmcg_get_scalars(kmcg_batch *b, int32_t r, double *time2, int64_t *step2, in
     int rc = check_replica(b, r);
     if (rc)
         return rc;
-    if ((rc = copy_out(b, time2, b->ktime + r, 1)) || (rc = copy_out(b, time2 + 1, b->kdt + r, 1)) ||
-        (rc = copy_out(b, (long long *)step2, b->kstep + r, 1)) ||
-        (rc = copy_out(b, (unsigned long long *)(step2 + 1), b->rngctr + r, 1)) ||
-        (rc = copy_out(b, status, b->status + r, 1)))
+    if ((rc = settle(b)))
         return rc;
+    double *o = b->h_samples + b->samples_len;           // five words behind the records
+    hipLaunchKernelGGL(kmc_scalars_kernel, dim3(1), dim3(64), 0, b->stream, make_params(b), r, o);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(b->stream));
+    memcpy(time2, o, 2 * sizeof(double));
+    memcpy(step2, o + 2, 2 * sizeof(int64_t));
+    *status = (int32_t)((const long long *)o)[4];
     return KMCG_OK;
 }
 
@@ -4963,7 +5004,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
         if (integ_rates && !std::isfinite(integ_rates[p]))
             return fail(KMCG_EINVAL, "set_state: integ_rates must be finite");
     std::vector<unsigned char> packed;
-    if ((rc = pack_config(b, r, lattice, packed)))
+    if ((rc = pack_configs(b, r, 1, lattice, packed)))
         return rc;
     const std::vector<double> ig = integ_rates ? std::vector<double>(integ_rates, integ_rates + P)
                                                : std::vector<double>(P, 0.0);
@@ -4988,11 +5029,8 @@ int kmcg_get_occupation(kmcg_batch *b, int32_t r0, int32_t n, double *out)
     if (b->m->S * b->m->spuck > 8 * 32)
         return fail(KMCG_EUNSUPPORTED, "too many species x sites for occupation");
     HIPCHK(hipSetDevice(b->device));
-    std::vector<int> ids(n);
-    for (int i = 0; i < n; ++i)
-        ids[i] = r0 + i;
-    HIPCHK(hipMemcpyAsync(b->rep_ids, ids.data(), n * sizeof(int), hipMemcpyHostToDevice, b->stream));
     KParams kp = make_params(b);
+    kp.rep_ids = b->iota + r0;
     if (b->bits == 2)
         hipLaunchKernelGGL((kmc_occupation_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp, b->occ);
     else
@@ -5023,16 +5061,24 @@ int kmcg_sample(kmcg_batch *b, const int32_t *replicas, int32_t n, double *out)
             return fail(KMCG_EINVAL, "replica index out of range");
     if (b->m->S * b->m->spuck > 8 * 32)
         return fail(KMCG_EUNSUPPORTED, "too many species x sites for occupation");
-    HIPCHK(hipSetDevice(b->device));
+    const int rc = settle(b);
+    if (rc)
+        return rc;
     const int width = 4 + b->m->S * b->m->spuck + 2 * b->m->P;
-    HIPCHK(hipMemcpyAsync(b->rep_ids, replicas, n * sizeof(int), hipMemcpyHostToDevice, b->stream));
     KParams kp = make_params(b);
-    if (b->bits == 2)
-        hipLaunchKernelGGL((kmc_sample_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp, b->samples, width);
+    const int first = contiguous(replicas, n);
+    if (first >= 0)
+        kp.rep_ids = b->iota + first;
     else
-        hipLaunchKernelGGL((kmc_sample_kernel<8>), dim3(n), dim3(256), 0, b->stream, kp, b->samples, width);
+        HIPCHK(hipMemcpyAsync(b->rep_ids, replicas, n * sizeof(int), hipMemcpyHostToDevice, b->stream));
+    if (b->bits == 2)
+        hipLaunchKernelGGL((kmc_sample_kernel<2>), dim3(n), dim3(256), 0, b->stream, kp, b->h_samples, width);
+    else
+        hipLaunchKernelGGL((kmc_sample_kernel<8>), dim3(n), dim3(256), 0, b->stream, kp, b->h_samples, width);
     HIPCHK(hipGetLastError());
-    return copy_out(b, out, b->samples, (size_t)n * width);
+    HIPCHK(hipStreamSynchronize(b->stream));
+    memcpy(out, b->h_samples, (size_t)n * width * sizeof(double));
+    return KMCG_OK;
 }
 
 } // extern "C"

@@ -70,11 +70,38 @@ struct OtfParams {
     const int *rep_ids;
     long long steps;
     int mode;
+    // the replicas' read-back words in pinned host memory, written by every
+    // kernel that changes them: OTF_OUT(P) words of 8 bytes each (integ[P],
+    // accum[P], procstat[P], list sizes[P], kmc_time, kmc_time_step, kmc_step,
+    // status)
+    double *out;
 };
+constexpr int OTF_OUT(int P) { return 4 * P + 4; }
 
 __device__ __forceinline__ int otf_wrap(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
 __device__ __forceinline__ int sx8(int w, int sh) { return (int)(signed char)((w >> sh) & 0xFF); }
 __device__ __forceinline__ int sx7(int w, int sh) { return (((w >> sh) & 0x7F) ^ 0x40) - 0x40; }
+
+// The read-back words of replica r from its owner lanes (act: lane < P).
+__device__ __forceinline__ void otf_export(const OtfParams &p, int r, int lane, bool act, double integ, double accum,
+                                           long long pstat, int n)
+{
+    double *o = p.out + (long long)r * (4 * p.P + 4);
+    if (act) {
+        o[lane] = integ;
+        o[p.P + lane] = accum;
+        ((long long *)o)[2 * p.P + lane] = pstat;
+        ((long long *)o)[3 * p.P + lane] = n;
+    }
+}
+__device__ __forceinline__ void otf_export_clock(const OtfParams &p, int r, double t, double dt, long long step, int st)
+{
+    double *o = p.out + (long long)r * (4 * p.P + 4) + 4 * p.P;
+    o[0] = t;
+    o[1] = dt;
+    ((long long *)o)[2] = step;
+    ((long long *)o)[3] = st;
+}
 
 struct OtfCell {
     int X, Y, Z, C;
@@ -449,6 +476,10 @@ __global__ __launch_bounds__(64) void otf_setup_kernel(OtfParams p)
             p.status[r] = KMCG_REPLICA_OK;
         }
     }
+    otf_export(p, r, lane, true, p.integ[slot], p.accum[slot], p.procstat[slot], n);
+    wave_sync();
+    if (q == 0)
+        otf_export_clock(p, r, p.kmc_time[r], p.kmc_time_step[r], p.kmc_step[r], p.status[r]);
 }
 
 // do_kmc_steps for `steps` steps (fewer when the replica stops).  LDS holds
@@ -684,7 +715,9 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
         p.accum[slot] = my_acc;
         p.runsum[slot] = run;
     }
+    otf_export(p, r, lane, act, integ, my_acc, pstat, n);
     if (lane == 0) {
+        otf_export_clock(p, r, t, t_step, kstep, st);
         p.kmc_time[r] = t;
         p.kmc_time_step[r] = t_step;
         p.kmc_step[r] = kstep;
@@ -993,7 +1026,9 @@ __global__ __launch_bounds__(64) void otf_fast_kernel(OtfParams p)
         p.accum[slot] = my_acc;
         p.runsum[slot] = run;
     }
+    otf_export(p, r, lane, act, integ, my_acc, pstat, n);
     if (lane == 0) {
+        otf_export_clock(p, r, t, t_step, kstep0 + s, st);
         p.kmc_time[r] = t;
         p.kmc_time_step[r] = t_step;
         p.kmc_step[r] = kstep0 + s;
@@ -1040,6 +1075,9 @@ struct kmcg_otf_batch {
     unsigned long long *d_ctr = nullptr;
     unsigned *d_seed = nullptr, *d_stream = nullptr;
     std::vector<double> rates, userpar;  // per replica, as last set
+    double *h_out = nullptr;             // OtfParams::out
+    const long long *out(int r) const { return (const long long *)h_out + (size_t)r * OTF_OUT(m->P); }
+    int status(int r) const { return (int)out(r)[4 * m->P + 3]; }
 };
 
 namespace {
@@ -1446,7 +1484,7 @@ OtfParams otf_params(kmcg_otf_batch *b, long long steps, int mode)
     p.runsum = b->d_runsum; p.table = b->d_table; p.kmc_time = b->d_time; p.kmc_time_step = b->d_dt;
     p.kmc_step = b->d_step;
     p.ctr = b->d_ctr; p.seed = b->d_seed; p.stream = b->d_stream; p.status = b->d_status;
-    p.rep_ids = b->d_rep; p.steps = steps; p.mode = mode;
+    p.rep_ids = b->d_rep; p.steps = steps; p.mode = mode; p.out = b->h_out;
     return p;
 }
 
@@ -1470,15 +1508,12 @@ int otf_range(const kmcg_otf_batch *b, int32_t r0, int32_t n)
 
 int otf_launch(kmcg_otf_batch *b, int32_t r0, int32_t n, long long steps, int mode, bool timed)
 {
-    std::vector<int> ids(n);
-    for (int i = 0; i < n; ++i)
-        ids[i] = r0 + i;
     HIPCHK(hipSetDevice(b->device));
     int rc = otf_sync(b);
     if (rc)
         return rc;
-    HIPCHK(hipMemcpyAsync(b->d_rep, ids.data(), n * sizeof(int), hipMemcpyHostToDevice, b->stream));
     OtfParams p = otf_params(b, steps, mode);
+    p.rep_ids = b->d_rep + r0;               // 0, 1, 2, ... since the batch was created
     // the steps kernel stages the program (and, when it fits, the rate
     // table) in LDS ahead of the lattice
     const size_t prog_bytes = (size_t)((p.W + 1) & ~1) * 4;
@@ -1609,6 +1644,8 @@ void kmcg_otf_batch_free(kmcg_otf_batch *b)
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
+    if (b->h_out)
+        (void)hipHostFree(b->h_out);
     if (b->ev0)
         (void)hipEventDestroy(b->ev0);
     if (b->ev1)
@@ -1695,8 +1732,17 @@ int kmcg_otf_batch_create(const kmcg_otf_model *m, int32_t n, const int32_t *siz
     for (auto &a : allocs)
         if (hipMalloc(a.p, std::max(a.bytes, (size_t)8)) != hipSuccess)
             return bail(KMCG_ENOMEM, "device allocation failed for an otf batch");
+    if (hipHostMalloc((void **)&b->h_out, (size_t)n * OTF_OUT(m->P) * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        return bail(KMCG_ENOMEM, "pinned host allocation failed for an otf batch");
+    memset(b->h_out, 0, (size_t)n * OTF_OUT(m->P) * sizeof(double));
+    for (int r = 0; r < n; ++r)
+        ((long long *)b->h_out)[(size_t)(r + 1) * OTF_OUT(m->P) - 1] = -1;     // not initialised
+    std::vector<int> iota(n);
+    for (int r = 0; r < n; ++r)
+        iota[r] = r;
     if (hipMemcpy(b->d_prog, progs.data(), progs.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_dims, b->dims.data(), b->dims.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(b->d_rep, iota.data(), n * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_lat_off, b->lat_off.data(), n * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_list_off, b->list_off.data(), n * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(b->d_nsites, 0, n * P * sizeof(int)) != hipSuccess ||
@@ -1748,9 +1794,7 @@ int kmcg_otf_set_params(kmcg_otf_batch *b, int32_t r0, int32_t n, const double *
         b->userpar.swap(old_u);
         return rc;
     }
-    int status0 = 0;
-    HIPCHK(hipMemcpy(&status0, b->d_status + r0, sizeof(int), hipMemcpyDeviceToHost));
-    if (status0 == -1)
+    if (b->status(r0) == -1)
         return KMCG_OK;                   // not initialised yet: init builds the lists
     if ((rc = otf_launch(b, r0, n, 0, 2, false)))
         return rc;
@@ -1770,11 +1814,10 @@ int kmcg_otf_set_config(kmcg_otf_batch *b, int32_t r0, int32_t n, const int8_t *
     for (long long i = 0; i < total; ++i)
         if (config[i] < 0 || config[i] >= b->m->S)
             return fail(KMCG_EINVAL, "species ids must be 0..S-1");
-    std::vector<int> st(n);
-    if ((rc = otf_copy_out(b, st.data(), b->d_status + r0, n)))
+    if ((rc = otf_sync(b)))
         return rc;
     for (int i = 0; i < n; ++i)
-        if (st[i] == -1)
+        if (b->status(r0 + i) == -1)
             return fail(KMCG_EINVAL, "set_config before init");
     HIPCHK(hipMemcpy(b->d_lat + b->lat_off[r0], config, total, hipMemcpyHostToDevice));
     if ((rc = otf_launch(b, r0, n, 0, 1, false)))
@@ -1789,11 +1832,10 @@ int kmcg_otf_run(kmcg_otf_batch *b, int32_t r0, int32_t n, int64_t steps)
         return rc;
     if (steps < 0)
         return fail(KMCG_EINVAL, "steps must be non-negative");
-    std::vector<int> st(n);
-    if ((rc = otf_copy_out(b, st.data(), b->d_status + r0, n)))
+    if ((rc = otf_sync(b)))
         return rc;
     for (int i = 0; i < n; ++i)
-        if (st[i] == -1)
+        if (b->status(r0 + i) == -1)
             return fail(KMCG_EINVAL, "run before init");
     return otf_launch(b, r0, n, steps, -1, true);
 }
@@ -1820,13 +1862,16 @@ int kmcg_otf_get_scalars(kmcg_otf_batch *b, int32_t r, double *kmc_time, double 
     int rc = otf_range(b, r, 1);
     if (rc)
         return rc;
-    if ((rc = otf_copy_out(b, kmc_time, b->d_time + r, 1)) || (rc = otf_copy_out(b, kmc_time_step, b->d_dt + r, 1)))
+    // (the read-back words are written by the kernels that change them: a
+    // getter costs no copy of its own, 15 us each)
+    if ((rc = otf_sync(b)))
         return rc;
-    long long s = 0;
-    if ((rc = otf_copy_out(b, &s, b->d_step + r, 1)))
-        return rc;
-    *kmc_step = s;
-    return otf_copy_out(b, (int *)status, b->d_status + r, 1);
+    const long long *o = b->out(r) + 4 * b->m->P;
+    memcpy(kmc_time, o, 8);
+    memcpy(kmc_time_step, o + 1, 8);
+    *kmc_step = o[2];
+    *status = (int32_t)o[3];
+    return KMCG_OK;
 }
 
 int kmcg_otf_get_lattice(kmcg_otf_batch *b, int32_t r, int8_t *out)
@@ -1844,13 +1889,16 @@ int kmcg_otf_get_counters(kmcg_otf_batch *b, int32_t r, int32_t *nr_of_sites, in
     if (rc)
         return rc;
     const size_t P = b->m->P;
-    if ((rc = otf_copy_out(b, (int *)nr_of_sites, b->d_nsites + r * P, P)))
+    if ((rc = otf_sync(b)))
         return rc;
-    if ((rc = otf_copy_out(b, (long long *)procstat, b->d_procstat + r * P, P)))
-        return rc;
-    if ((rc = otf_copy_out(b, integ, b->d_integ + r * P, P)))
-        return rc;
-    return otf_copy_out(b, accum, b->d_accum + r * P, P);
+    const long long *o = b->out(r);
+    memcpy(integ, o, P * 8);
+    memcpy(accum, o + P, P * 8);
+    for (size_t p = 0; p < P; ++p) {
+        procstat[p] = o[2 * P + p];
+        nr_of_sites[p] = (int32_t)o[3 * P + p];
+    }
+    return KMCG_OK;
 }
 
 int kmcg_otf_get_avail(kmcg_otf_batch *b, int32_t r, int32_t *sites, int32_t *back, double *rates_matrix)
