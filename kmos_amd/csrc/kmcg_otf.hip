@@ -227,15 +227,22 @@ __device__ __forceinline__ double otf_resum(const double *rrow, double *chk, int
 // Returns the row's total where `want`.
 constexpr int OTF_ROWS = 12, OTF_DEEP = 6, OTF_STAGE = OTF_BLK + 2;   // (16-byte aligned, spread over the banks)
 
-__device__ __forceinline__ double otf_resum_wave(const double *rm, long long crow, double *chk, bool want, int from,
-                                                 int n, double tot, double *stage, int *ids, int lane)
+__device__ __forceinline__ double otf_resum_wave(const double *rm, double *pre, long long crow, int P, bool want,
+                                                 int from, int n, double tot, double *stage, int *ids, int lane)
 {
     constexpr int SETS = OTF_ROWS / 4;
     const int b0 = from >> 4, nb = (n + OTF_BLK - 1) >> 4;
     // short tails only (rates that do not differ within a list): each lane
     // its own
     if (!__ballot(want && nb - b0 > 2))
-        return want ? otf_resum<2>(rm + lane * crow, chk, from, n) : tot;
+        return want ? otf_resum<2>(rm + lane * crow, pre + lane * (crow / OTF_BLK), from, n) : tot;
+    // the checkpoints through a buffer descriptor: lanes past their last
+    // block store outside it, without a branch
+    typedef int int2v __attribute__((ext_vector_type(2)));
+    const int crow_chk = (int)(crow / OTF_BLK);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(pre, 0, P * crow_chk * 8, 0x00027000);
+    const double *chk = pre + (want ? lane : 0) * crow_chk;
+    const unsigned at0 = (unsigned)((want ? lane : 0) * crow_chk + b0) * 8u;
     double a = want && b0 > 0 ? chk[b0 - 1] : 0.0;
     unsigned long long todo = __ballot(want && b0 < nb);
     while (todo) {
@@ -248,7 +255,8 @@ __device__ __forceinline__ double otf_resum_wave(const double *rm, long long cro
         if (mine)
             ids[rank] = lane;
         wave_sync();
-        const double *src[SETS];
+        const char *rows = (const char *)rm;             // (a replica's rows: below 4 GiB)
+        unsigned src[SETS];
         int last[SETS];
 #pragma unroll
         for (int i = 0; i < SETS; ++i) {
@@ -256,7 +264,7 @@ __device__ __forceinline__ double otf_resum_wave(const double *rm, long long cro
             const int f = __builtin_amdgcn_ds_bpermute(id << 2, b0), e = __builtin_amdgcn_ds_bpermute(id << 2, nb);
             // (behind its last block a row reads that one again, unused)
             last[i] = id >= 0 ? e - f - 1 : 0;
-            src[i] = rm + max(id, 0) * crow + (id >= 0 ? OTF_BLK * f : 0) + (lane & 15);
+            src[i] = (unsigned)(max(id, 0) * (int)crow + (id >= 0 ? OTF_BLK * f : 0) + (lane & 15)) * 8u;
         }
         const int T = mine ? nb - b0 : 0;
         double v[OTF_DEEP][SETS];
@@ -264,7 +272,7 @@ __device__ __forceinline__ double otf_resum_wave(const double *rm, long long cro
         for (int j = 0; j < OTF_DEEP; ++j)
 #pragma unroll
             for (int i = 0; i < SETS; ++i)
-                v[j][i] = src[i][OTF_BLK * min(j, last[i])];
+                v[j][i] = *(const double *)(rows + (src[i] + 8u * OTF_BLK * (unsigned)min(j, last[i])));
         const double *my = stage + (mine ? rank : 0) * OTF_STAGE;
         double sum = a;
         for (int t0 = 0; __ballot(t0 < T); t0 += OTF_DEEP) {
@@ -274,7 +282,8 @@ __device__ __forceinline__ double otf_resum_wave(const double *rm, long long cro
 #pragma unroll
                 for (int i = 0; i < SETS; ++i) {
                     stage[(4 * i + (lane >> 4)) * OTF_STAGE + (lane & 15)] = v[j][i];
-                    v[j][i] = src[i][OTF_BLK * min(t + OTF_DEEP, last[i])];
+                    v[j][i] = *(const double *)(rows +
+                                                (src[i] + 8u * OTF_BLK * (unsigned)min(t + OTF_DEEP, last[i])));
                 }
                 wave_sync();
                 double w[OTF_BLK];
@@ -284,8 +293,13 @@ __device__ __forceinline__ double otf_resum_wave(const double *rm, long long cro
 #pragma unroll
                 for (int k = 0; k < OTF_BLK; ++k)
                     sum = sum + w[k];
-                if (t < T)
-                    chk[b0 + t] = a = sum;
+                union {
+                    double d;
+                    int2v v;
+                } out;
+                out.d = sum;
+                __builtin_amdgcn_raw_buffer_store_b64(out.v, rs, t < T ? at0 + 8u * (unsigned)t : FZ_NONE, 0, 0);
+                a = t < T ? sum : a;
                 wave_sync();
             }
         }
@@ -1003,8 +1017,8 @@ __global__ __launch_bounds__(64) void otf_fast_kernel(OtfParams p)
                 n += 1;
             }
         }
-        tot = otf_resum_wave(p.rm + base, crow, chk, act && dirty != 0x7fffffff, min(dirty, n), n, tot, eold, ecell,
-                             lane);
+        tot = otf_resum_wave(p.rm + base, p.pre + base / OTF_BLK, crow, P, act && dirty != 0x7fffffff, min(dirty, n), n,
+                             tot, eold, ecell, lane);
         if (__ballot(bad)) {
             st = KMCG_REPLICA_SPECIES_MISMATCH;
             s += 1;
