@@ -125,6 +125,7 @@ struct KParams {
                                    // bit 1: a lat_int group's segments post in one pass
     int off_seg, off_proc, off_touch, off_nli, off_nlitab;
     const int *fz_recs;            // records of the fused step loop (kmcg_fused.hip)
+    int resume;                    // the generic loop behind a fused run: the steps it left
     int fz_nch;                    // chunks of 64 records per process
     int fz_tab_off;                // lat_int: word offset of the groups' tables behind the records
     double *srec;                  // in-loop sample records (or null)

@@ -1557,7 +1557,7 @@ __device__ __forceinline__ void steps_end(Wave<PPL, BITS> &W, const KParams &kp,
         kp.kstep[r] = ks;
         kp.rngctr[r] = ctr;
         kp.status[r] = st;
-        kp.executed[slot] = done;
+        kp.executed[slot] = (kp.resume ? kp.executed[slot] : 0) + done;
         if (kp.budget)
             kp.budget[slot] -= done;
     }
@@ -1580,10 +1580,14 @@ __device__ __forceinline__ void steps_loop(const KParams &kp, unsigned char *sme
     const int st0 = kp.status[r];
     W.chk = kp.lists_ok && kp.lists_ok[r] && W.local_smart;
     long long n = kp.nsteps;
+    const long long before = kp.resume ? kp.executed[slot] : 0;    // steps a fused run left off at
+    n -= before;
     if (kp.budget)
         n = min(n, kp.budget[slot]);
     if (st0 != ST_OK)
         n = 0;
+    if (kp.resume && n <= 0)
+        return;
     if (kp.srec)
         count_species<PPL, BITS>(W);
     double t = kp.ktime[r], dt_last = kp.kdt[r];
@@ -2483,12 +2487,13 @@ int fz_word(const kmcg_model *m, const Coord &c, int n0)
     return ((c[0] * m->spuck + c[3] - n0) & 0xFFFF) | (int)((unsigned)c[1] << 16);
 }
 
-// A single-layer local_smart model: per process the list updates of its
-// routines as one list, with every condition on a site whose species the
-// process's own conditions fix resolved here.  Not taken: more than 64
-// processes, three dimensions, several layers (their lists only promise that
-// registered processes hold), a write or a deletion whose conditions are
-// not known, more than four open conditions of one update.
+// A local_smart model: per process the list updates of its routines as one
+// list, with every condition on a site whose species the process's own
+// conditions fix resolved here.  Several layers: a write may name a site no
+// condition does; its old species is taken for known and checked before the
+// step.  Not taken: more than 64 processes, three dimensions, (one layer) such
+// a write, a deletion whose conditions are not known, more than four open
+// conditions of one update.
 void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector<std::vector<int>> &proc_items,
                  const std::vector<std::vector<int>> &pconds, const std::vector<bool> &have)
 {
@@ -2498,11 +2503,12 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
         Coord at;
         std::vector<std::pair<Coord, int>> conds;
     };
-    if (m->backend != 0 || m->nullsp >= 0 || m->P > 64 || m->spuck > 32 || m->dim > 2)
+    if (m->backend != 0 || m->P > 64 || m->spuck > 32 || m->dim > 2)
         return;
+    const bool layers = m->nullsp >= 0;
     const int code = m->lattice_bits() == 2 ? 1 : 0;     // species code of the records
     std::vector<std::vector<Up>> ups(m->P);
-    std::vector<std::map<Coord, std::pair<int, int>>> writes(m->P);    // old, new
+    std::vector<std::map<Coord, std::array<int, 3>>> writes(m->P);      // old, new, check the old one
     std::vector<int> n0(m->P, 1);                        // executing site type
     std::vector<std::pair<Coord, int>> held(m->P);       // a condition that always holds
     size_t maxc = 0, most = 0;
@@ -2531,14 +2537,24 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
                 return;
             auto shift = [&](int dx, int dy, int dz, int n) { return Coord{it[1] + dx, it[2] + dy, it[3] + dz, n}; };
             const Coord wc = shift(sg.writes[0], sg.writes[1], sg.writes[2], sg.writes[3]);
-            const auto kn = known.find(wc);
+            auto kn = known.find(wc);
+            int check = 0;
+            if (kn == known.end() && layers) {
+                // (its routine's only old species)
+                int old = 0;
+                while (old < 15 && sg.writes[4] != 1 << old)
+                    ++old;
+                kn = known.emplace(wc, old).first;
+                check = 1;
+                reach(wc);
+            }
             if (kn == known.end() || sg.writes[4] != 1 << kn->second)
                 return;                                  // the write's old species is open
             bool written = false;
             const size_t seg0 = list.size();
             auto do_write = [&]() {
-                const auto w = writes[p - 1].emplace(wc, std::make_pair(kn->second, sg.writes[5]));
-                w.first->second.second = sg.writes[5];
+                const auto w = writes[p - 1].emplace(wc, std::array<int, 3>{kn->second, sg.writes[5], check});
+                w.first->second[1] = sg.writes[5];
                 kn->second = sg.writes[5];
                 written = true;
             };
@@ -2580,9 +2596,9 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
             return;
     }
     const int nch = std::max(1, (int)((most + 63) / 64));
-    const int form = maxc <= 1 && nch == 1 ? FZ_1 : FZ_4;
+    const int form = layers ? FZ_M : maxc <= 1 && nch == 1 ? FZ_1 : FZ_4;
     const int rw = form == FZ_1 ? 4 : 8;
-    if (maxc > 4 || nch > 31 || mo > 31 || (size_t)m->P * nch * 64 * rw > (size_t)1 << 20)
+    if (maxc > 4 || nch > 31 || (layers && nch > 1) || mo > 31 || (size_t)m->P * nch * 64 * rw > (size_t)1 << 20)
         return;
     std::vector<int> fz((size_t)m->P * nch * 64 * rw, 0);
     for (int p = 0; p < m->P; ++p) {
@@ -2630,7 +2646,7 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
                 if (ch == own_ch - 1 && l < (int)writes[p].size()) {
                     auto w = writes[p].begin();
                     std::advance(w, l);
-                    q[0] |= w->second.first << 22 | w->second.second << 26;
+                    q[0] |= w->second[0] << 22 | w->second[1] << 26 | w->second[2] << 30;
                     q[rw - 1] = fz_word(m, w->first, n0[p]);
                 }
             }
@@ -3387,7 +3403,8 @@ struct Shape {
     size_t lds;
 };
 
-Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wpg, bool steps = false)
+// steps: a step launch (2: one that records samples or tracks particles).
+Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wpg, int steps = 0)
 {
     long long maxlb = 0;
     for (int i = 0; i < n; ++i)
@@ -3419,7 +3436,7 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
     // offsets of the records meet (extents of 2 * reach + 1 and more), the
     // lattice fits LDS, and no other form was asked for
     const size_t fz_wave = (size_t)maxlb + (64 * WIN + occ) * sizeof(int);
-    s.fz = steps && !b->m->fz.empty() && b->ov_mode == -1 && b->lds_mode != 0 &&
+    s.fz = steps && !b->m->fz.empty() && (steps == 1 || b->m->fz_form != FZ_M) && b->ov_mode == -1 && b->lds_mode != 0 &&
            (size_t)b->m->fz_tab_bytes + fz_wave <= (size_t)b->max_lds;
     const int least = 2 * b->m->fz_moff + 1;
     for (int i = 0; i < n && s.fz; ++i) {
@@ -3467,6 +3484,7 @@ hipError_t launch_t(bool steps, const Shape &s, hipStream_t st, const KParams &k
             FZ_LAUNCH(FZ_4, FZ_PLAIN)
             FZ_LAUNCH(FZ_4, FZ_REC)
             FZ_LAUNCH(FZ_4, FZ_MSD)
+            FZ_LAUNCH(FZ_M, FZ_PLAIN)
             FZ_LAUNCH(FZ_LI, FZ_PLAIN)
             FZ_LAUNCH(FZ_LI, FZ_REC)
             FZ_LAUNCH(FZ_LI, FZ_MSD)
@@ -4124,9 +4142,21 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     if (first >= 0)
         kp.rep_ids = b->iota + first;
     b->run_ids = kp.rep_ids;
-    const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg, true);
+    const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg, records || track ? 2 : 1);
     kp.nsteps = steps;
     kp.budget = budget ? b->budget : nullptr;
+    // behind a fused run that may stop short of a step it cannot take: the
+    // generic loop for what is left
+    const bool tail = s.fz && s.fz_form == FZ_M;
+    KParams kt = make_params(b);
+    Shape st{};
+    if (tail) {
+        kt.rep_ids = kp.rep_ids;
+        st = launch_shape(b, replicas, n, kt, b->max_wpg);
+        kt.nsteps = steps;
+        kt.budget = kp.budget;
+        kt.resume = 1;
+    }
     if (track & 4) {
         kp.acf_pa = b->acf_pa;
         kp.acf_po = b->acf_po;
@@ -4184,6 +4214,8 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
             e = hipEventRecord(b->ev0, b->stream);
         if (e == hipSuccess)
             e = launch(b, true, s, kp);
+        if (e == hipSuccess && tail)
+            e = launch(b, true, st, kt);
         if (e == hipSuccess && timed)
             e = hipEventRecord(b->ev1, b->stream);
         if (e == hipSuccess && budget)

@@ -49,6 +49,14 @@
 //   FZ_1 (one condition):  site, condition site, write site
 //   FZ_4 (four, chunks):   four condition codes | chunks << 16, site, four
 //                          condition sites, write site
+//   FZ_M (several layers): as FZ_4.  The lists of several local_smart layers
+//                          promise only that registered processes hold: a
+//                          deletion that finds no entry is none (the next
+//                          step is then selected again), and a write whose
+//                          old species no condition names (word 0, bit 30)
+//                          looks before the step; where it fails the run
+//                          stops short and the generic loop behind it
+//                          finishes it.
 //   FZ_LI (lat_int):       cell, byte offsets of the two lookups (before |
 //                          after << 16), four open sites, write site
 // site word: (dx * spuck + n - n_exec) | dy << 16, signed halves, from the
@@ -57,14 +65,15 @@
 // a lane without an open condition tests a site the process knows, a lane
 // without an update has code 15, which no site holds.
 
-enum : int { FZ_1 = 1, FZ_LI = 2, FZ_4 = 4 };
+enum : int { FZ_1 = 1, FZ_LI = 2, FZ_M = 3, FZ_4 = 4 };
+__host__ __device__ constexpr bool fz_wide(int form) { return form == FZ_4 || form == FZ_M; }
 
 template <int FORM>
 struct FzRec {
     static constexpr int RW = FORM == FZ_1 ? 4 : 8;
     int w[RW];
     __device__ __forceinline__ int write_site() const { return w[RW - 1]; }
-    __device__ __forceinline__ int site() const { return FORM == FZ_4 ? w[2] : w[1]; }
+    __device__ __forceinline__ int site() const { return fz_wide(FORM) ? w[2] : w[1]; }
 };
 
 __device__ __forceinline__ int bf_s(int v, int off, int w) { return __builtin_amdgcn_sbfe(v, off, w); }
@@ -203,10 +212,11 @@ struct FzList {
 struct FzBlock {
     int nr0, ws[4], wv[4];
 };
-template <int I0, int N, bool LI>
+template <int I0, int N, int FORM>
 __device__ __forceinline__ void fz_replay(__amdgpu_buffer_rsrc_t rs, FzList &F, FzBlock &B, int &nr, unsigned &bits,
                                           int a, int ent, int bv0, int t0, int t1, int t2, int t3)
 {
+    constexpr bool LI = FORM == FZ_LI;
     int st[N], bv[N];
     bool act[N], isd[N];
 #pragma unroll
@@ -243,7 +253,7 @@ __device__ __forceinline__ void fz_replay(__amdgpu_buffer_rsrc_t rs, FzList &F, 
         const bool okd = (unsigned)(mp - 1) < (unsigned)cur;
         const bool del = act[i] && isd[i] && okd;
         const bool add = act[i] && !isd[i] && cur < F.V;
-        F.err |= act[i] && !del && !add ? 1 : 0;
+        F.err |= act[i] && !del && !add && !(FORM == FZ_M && isd[i] && mp == 0) ? 1 : 0;
         const bool mv = del && mp < cur, put = add || mv;
         const int slot = del ? mp : cur + 1;
         const int val = del ? moved : st[i];
@@ -354,7 +364,7 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
     const int rslot = blockIdx.x * kp.wpg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = W.lane, P = W.P;
     const int *recs = kp.fz_recs;
-    const int nch = FORM == FZ_4 ? kp.fz_nch : 1;
+    const int nch = fz_wide(FORM) ? kp.fz_nch : 1;
     double *tz = (double *)W.win;
     unsigned *bm = (unsigned *)(tz + 128);             // FZ_LI: entries per process, then spare words
     tz[lane] = 0.0;
@@ -404,6 +414,8 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
     int cpick = -1;
     double total = 0.0;
     int kk = 0;
+    bool bail = false;               // FZ_M: step k is left to the generic loop
+    double dt_done = 0.0;            // FZ_M: the last finished step's duration
     FzRec<FORM> q;
 #if KMCG_PHASES
     for (int i = 0; i < 5; ++i)
@@ -415,9 +427,9 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
         // the list updates of the step before
         FzBlock B;
         B.nr0 = nr;
-        fz_replay<0, 2, LI>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
+        fz_replay<0, 2, FORM>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
         if (three) {
-            fz_replay<2, 2, LI>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
+            fz_replay<2, 2, FORM>(rs, F, B, nr, bits, a, ent, bv, t0, t1, t2, t3);
             while (__ballot(bits != 0)) {
 #if KMCG_PHASES
                 W.nblk += 1;
@@ -428,7 +440,7 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
                     rs, bits ? F.so + ((unsigned)nr << 2) - 12 : FZ_NONE, 0, 0);
                 const int bn = __builtin_amdgcn_raw_buffer_load_b32(rs, back ? bo : FZ_NONE, 0, 0);
                 B.nr0 = nr;
-                fz_replay<0, 4, LI>(rs, F, B, nr, bits, a, ent, bn, tl.w, tl.z, tl.y, tl.x);
+                fz_replay<0, 4, FORM>(rs, F, B, nr, bits, a, ent, bn, tl.w, tl.z, tl.y, tl.x);
             }
         }
 #if KMCG_PHASES
@@ -480,11 +492,25 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
         // counts before it), its list updates
         if (MODE != FZ_MSD) {
             const double dt = cmlog / ctotal;
+            if (FORM == FZ_M)
+                dt_done = cpick >= 0 ? dt : dt_done;
             t = t + dt;
             integ = integ + cc * dt;
             W.pstat[0] += lane == cpick ? 1 : 0;
         }
         finish();
+        if (FORM == FZ_M && __ballot(nr != nrs)) {
+            // a deletion found no entry: step k selected again from the
+            // counts there are, nothing of step k - 1 left to do
+            nrx = nr;
+            bits = 0;
+            back = three = false;
+            cc = cmlog = 0.0;
+            ctotal = 1.0;
+            cpick = -1;
+            limit = n;
+            continue;
+        }
         if (MODE == FZ_REC && --rec_left == 0) {
             const FzCold kc = fz_cold();
             W.integ[0] = integ;
@@ -517,7 +543,7 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
             else
                 msd_track<1, BITS>(W, kp, r, pick, site);
         }
-        const int nchp = FORM == FZ_4 ? __builtin_amdgcn_readfirstlane(bf_u(q.w[1], 16, 5)) : 1;
+        const int nchp = fz_wide(FORM) ? __builtin_amdgcn_readfirstlane(bf_u(q.w[1], 16, 5)) : 1;
         for (int ci = 0; ; ++ci) {
             // evaluation; bits: this owner lane's entries, nd of them deletions
             FzSites<FORM> z;
@@ -525,6 +551,13 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
             if (!inside)
                 z.template form<false>(at, q);
             int nd;
+            if (FORM == FZ_M) {
+                const int want = bf_u(q.w[0], 22, 4) + (BITS == 2 ? 1 : 0);
+                if (__ballot(((q.w[0] >> 30) & 1) && fz_code<BITS>(W.lat.p, z.ws) != want)) {
+                    bail = true;
+                    break;
+                }
+            }
             a = bf_u(q.w[0], 7, 6);
             if constexpr (LI) {
                 int pd, pa;
@@ -583,15 +616,17 @@ __device__ __forceinline__ void fused_loop(const KParams &kp, unsigned char *sme
         }
         if (MODE == FZ_MSD && kp.acf_pa && lane == 0)
             acf_after(kp, r);
+        if (FORM == FZ_M && bail)
+            break;
         k += 1;
         PH_MARK(W, 2);
     }
     const FzCold kc = fz_cold();
-    double dt_last = k > 0 ? cmlog / ctotal : kc->kdt[r];
+    double dt_last = k > 0 ? (FORM == FZ_M ? dt_done : cmlog / ctotal) : kc->kdt[r];
     long long drawn = k;
     if (__ballot(F.err)) {
         st = LI ? ST_DEL_ABSENT : ST_CORRUPT;
-    } else if (k < n) {
+    } else if (k < n && !bail) {
         st = ST_ABSORBING;
         if (total > 0.0) {               // only a corrupted database gets here
             st = ST_CORRUPT;
