@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from kmos_amd import workloads as W
+from kmos_amd.acf import displacement_table
 from kmos_amd.compiler import compile_model
 from kmos_amd.model import load_project
 from paritylib import compare_state, oracle_replica, pdopd_project, random_config
@@ -84,4 +85,47 @@ def test_layers_stop_where_the_oracle_stops(engine, oracle):
                 assert left[i] == limits[i] - (o.kmc_step - before)
     stops = b.scalars_all()[2]
     assert (stops == 2).any() and (stops == 0).any()
+    b.close()
+
+
+@pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
+def test_moves_match_oracle(engine, oracle, backend):
+    """Particle moves, written one step after their hop: launches that end
+    on a hop, particles without a number (adsorbed after the start), a
+    trajectory that fills up inside a launch, a stopped replica."""
+    pt = W.pairwise_project()
+    cm = compile_model(pt, backend)
+    hops, disp = displacement_table(cm)
+    R = Records(cm)
+    assert R.have
+    m = 2 * R.reach + 1
+    sizes = [(m, m), (m, m + 3), (31, 17), (64, 33)]
+    g = np.random.default_rng(23)
+    n = len(sizes)
+    rates = 10.0 ** g.uniform(-1, 3, (n, cm.nr_of_proc))
+    rates[0] = 0.0
+    ids = pt.species_ids()
+    seeds = g.integers(1 << 31, size=n).astype(np.uint32)
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init(seeds, np.arange(n, dtype=np.uint32))
+    b.set_rates(rates)
+    configs = [np.where(g.random(int(v)) < 0.4, ids["A"], ids["empty"]).astype(np.int8) for v in b.volumes]
+    b.set_config(configs)
+    b.msd_init(ids["A"], hops, disp)
+    b.msd_trajectory(300)
+    orcs = []
+    for i, s in enumerate(sizes):
+        o = oracle_replica(oracle, cm, s, int(seeds[i]), i, rates[i], configs[i])
+        o.msd_init(ids["A"], hops, disp)
+        o.msd_trajectory(300)
+        orcs.append(o)
+    for steps in (1, 2, 61, 1, 140, 395):
+        b.run_displacement(steps, traj_on=True)
+        for i, o in enumerate(orcs):
+            o.run_displacement(steps, traj_on=True)
+            got, want = b.msd_state(i), o.msd_state()
+            for key in ("nr_of_ions", "site_arr", "id_arr", "displacement", "events"):
+                np.testing.assert_array_equal(got[key], want[key], err_msg="%s %s" % (sizes[i], key))
+            compare_state(b, i, o, where="%s %s" % (backend, sizes[i]))
+    assert b.scalars(0)[4] == 1
     b.close()
