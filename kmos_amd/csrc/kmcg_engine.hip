@@ -2511,6 +2511,7 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
     std::vector<std::map<Coord, std::array<int, 3>>> writes(m->P);      // old, new, check the old one
     std::vector<int> n0(m->P, 1);                        // executing site type
     std::vector<std::pair<Coord, int>> held(m->P);       // a condition that always holds
+    std::vector<std::pair<Coord, int>> open;             // an update's conditions on other sites
     size_t maxc = 0, most = 0;
     int mo = 0;
     auto reach = [&](const Coord &c) {
@@ -2521,14 +2522,19 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
         n0[p - 1] = m->blob[m->blob[9] + 3 * (p - 1)];
         if (!have[p] || pconds[p].empty())
             return;
-        std::map<Coord, int> known;
+        std::vector<std::pair<Coord, int>> known;        // a handful: searched in order
+        auto find = [&known](const Coord &at) {
+            return std::find_if(known.begin(), known.end(),
+                                [&at](const std::pair<Coord, int> &k) { return k.first == at; });
+        };
         for (size_t c = 0; c + 5 <= pconds[p].size(); c += 5) {
             const Coord at = {pconds[p][c], pconds[p][c + 1], pconds[p][c + 2], pconds[p][c + 3]};
-            if (!known.emplace(at, pconds[p][c + 4]).second)
+            if (find(at) != known.end())
                 return;                                  // two conditions on one site
+            known.emplace_back(at, pconds[p][c + 4]);
             reach(at);
         }
-        held[p - 1] = *known.begin();
+        held[p - 1] = *std::min_element(known.begin(), known.end());
         std::vector<Up> &list = ups[p - 1];
         for (size_t i = 0; i < proc_items[p - 1].size(); i += 4) {
             const int *it = &proc_items[p - 1][i];
@@ -2537,14 +2543,14 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
                 return;
             auto shift = [&](int dx, int dy, int dz, int n) { return Coord{it[1] + dx, it[2] + dy, it[3] + dz, n}; };
             const Coord wc = shift(sg.writes[0], sg.writes[1], sg.writes[2], sg.writes[3]);
-            auto kn = known.find(wc);
+            auto kn = find(wc);
             int check = 0;
             if (kn == known.end() && layers) {
                 // (its routine's only old species)
                 int old = 0;
                 while (old < 15 && sg.writes[4] != 1 << old)
                     ++old;
-                kn = known.emplace(wc, old).first;
+                kn = known.insert(known.end(), {wc, old});
                 check = 1;
                 reach(wc);
             }
@@ -2564,19 +2570,20 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
                     do_write();          // additions follow the deletions and see the write
                 if (del && (written || op.conds.empty()))
                     return;
-                Up u{op.arg, del, shift(op.dx, op.dy, op.dz, op.n), {}};
                 bool can = true;
+                open.clear();
                 for (size_t c = 0; c + 5 <= op.conds.size() && can; c += 5) {
                     const Coord at = shift(op.conds[c], op.conds[c + 1], op.conds[c + 2], op.conds[c + 3]);
                     const std::pair<Coord, int> cd = {at, op.conds[c + 4]};
-                    const auto k = known.find(at);
+                    const auto k = find(at);
                     if (k != known.end())
                         can = k->second == cd.second;
-                    else if (std::find(u.conds.begin(), u.conds.end(), cd) == u.conds.end())
-                        u.conds.push_back(cd);
+                    else if (std::find(open.begin(), open.end(), cd) == open.end())
+                        open.push_back(cd);
                 }
                 if (!can)
                     continue;
+                const Up u{op.arg, del, shift(op.dx, op.dy, op.dz, op.n), open};
                 // one routine names an update once
                 for (size_t v = seg0; v < list.size(); ++v)
                     if (list[v].proc == u.proc && list[v].del == u.del && list[v].at == u.at)
@@ -2605,20 +2612,19 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
         const std::vector<Up> &list = ups[p];
         const int own_ch = std::max(1, (int)((list.size() + 63) / 64));
         const int heldw = fz_word(m, held[p].first, n0[p]), heldc = held[p].second + code;
-        for (int ch = 0; ch < nch; ++ch)
+        for (int ch = 0; ch < nch; ++ch) {
+            // the run of process l + 1 in this chunk
+            int first[64] = {}, len[64] = {};
+            for (int j = 0; j < 64 && 64 * ch + j < (int)list.size(); ++j) {
+                const int o = list[64 * ch + j].proc - 1;
+                if (!len[o]++)
+                    first[o] = j;
+                if (len[o] > 31)
+                    return;
+            }
             for (int l = 0; l < 64; ++l) {
                 int *q = &fz[(((size_t)p * nch + ch) * 64 + l) * rw];
-                // the run of process l + 1 in this chunk
-                int first = 0, len = 0;
-                for (int j = 0; j < 64 && 64 * ch + j < (int)list.size(); ++j)
-                    if (list[64 * ch + j].proc == l + 1) {
-                        if (!len)
-                            first = j;
-                        ++len;
-                    }
-                if (len > 31)
-                    return;
-                q[0] = first << 7 | len << 13;
+                q[0] = first[l] << 7 | len[l] << 13;
                 const bool up = 64 * ch + l < (int)list.size();
                 int codes[4] = {heldc, heldc, heldc, heldc}, sites[4] = {heldw, heldw, heldw, heldw};
                 if (up) {
@@ -2650,6 +2656,7 @@ void build_fused(kmcg_model *m, const std::vector<SegH> &segs, const std::vector
                     q[rw - 1] = fz_word(m, w->first, n0[p]);
                 }
             }
+        }
     }
     m->fz.swap(fz);
     m->fz_form = form;
