@@ -377,8 +377,8 @@ def tracking_leg(engine, K, steps=20000, warm=20000):
     model compiled for local_smart (49 processes, hops in four directions),
     512 replicas of 256^2; after `warm` steps the A particles are numbered
     (msd_init) and K launches of `steps` steps are timed, through
-    do_kmc_steps_displacement and do_kmc_steps respectively, the plain form
-    (no overlapped select) in both runs."""
+    do_kmc_steps_displacement and do_kmc_steps respectively, in the form
+    the launch chooses."""
     from kmos_amd import acf
     wl = W.pairwise()
     cm = compile_model(wl.project, "local_smart")
@@ -389,7 +389,6 @@ def tracking_leg(engine, K, steps=20000, warm=20000):
            "kmc_steps_per_launch": wl.n * steps, "launches": K}
     for mode in ("plain", "tracking"):
         b = make_batch(engine, model, wl)
-        b.set_overlap(0)
         b.run(warm)
         if mode == "tracking":
             b.msd_init(trace, hops, disp)
