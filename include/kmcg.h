@@ -67,14 +67,15 @@ void kmcg_model_free(kmcg_model *m);
 int kmcg_model_info(const kmcg_model *m, int32_t *info5);
 /* The step kernel's forms this model can run: *li = 1 when a lat_int
  * group's two segments are posted in one pass (kmc_steps_kernel_li: every
- * nli group tabulated, at most 64 processes).  No counterpart in the
+ * nli group tabulated, at most 64 processes).  The fused loop (below) takes
+ * its place in runs it is sound for.  No counterpart in the
  * reference (a profiling aid). */
 int kmcg_model_forms(const kmcg_model *m, int32_t *li);
 
 /* The fused step loop's records (per process the list updates of its
  * routines as one flat list; layout in kmos_amd/csrc/kmcg_fused.hip): info6
  * = words in all (0: the model has none), form (1 one open condition, 4
- * four, 2 lat_int), chunks of 64 records per process, largest offset, word
+ * four, 3 several layers, 2 lat_int), chunks of 64 records per process, largest offset, word
  * offset and bytes of the lat_int tables; `words` may be NULL.  No
  * counterpart in the reference (a test aid). */
 int kmcg_model_fused(const kmcg_model *m, int32_t *info6, int32_t *words);
@@ -131,10 +132,11 @@ int kmcg_sync(kmcg_batch *b);
 int kmcg_set_launch(kmcg_batch *b, int32_t lattice_in_lds, int32_t waves_per_group);
 /* Step kernel form for kmcg_run with one process slot per lane (P <= 64)
  * and no tracking: 1 = the next step's accumulate and search run while the
- * replay's HBM reads are in flight, 0 = after them, -1 = automatic (on for
- * local_smart models of more than 16 processes in runs of at most 8
- * replicas per compute unit).  Both forms
- * give identical trajectories.  No counterpart in the reference (a launch
+ * replay's HBM reads are in flight, 0 = after them, -1 = automatic (the
+ * fused loop, which does so by itself, where the model has its records and
+ * every replica's lists follow its lattice; elsewhere on for local_smart
+ * models of more than 16 processes in runs of at most 8 replicas per compute
+ * unit).  All forms give identical trajectories.  No counterpart in the reference (a launch
  * setting of the batched engine). */
 int kmcg_set_overlap(kmcg_batch *b, int32_t mode);
 /* Runs through HIP graphs (1) or direct launches (0, the default).  With

@@ -3438,7 +3438,7 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
            (b->ov_mode == -1 && b->m->backend == 0 && b->m->P > 16 && (long long)n <= 8LL * b->n_cu);
     size_t shared = prog;
     // the fused step loop, faster than the others at every size measured
-    // (1.5 to 2.6 times, one replica of 20x20 to 4096 of 128x128), wherever
+    // (1.7 to 3.3 times, one replica of 20x20 to 4096 of 128x128), wherever
     // it is sound: the lists of every replica follow its lattice, no two
     // offsets of the records meet (extents of 2 * reach + 1 and more), the
     // lattice fits LDS, and no other form was asked for

@@ -1,5 +1,6 @@
-// kmcg_fused.hip -- the fused step loop (one layer of local_smart processes,
-// or lat_int with every group tabulated; one or two dimensions).
+// kmcg_fused.hip -- the fused step loop (local_smart processes on one or
+// several layers, or one layer of lat_int with every group tabulated; one or
+// two dimensions).
 //
 // Included by kmcg_engine.hip (device part, inside its namespace).
 //
@@ -34,10 +35,12 @@
 // register.
 //
 // Measured against the generic loops, per 1000 steps: ZGB 4096 x 128x128
-// 5.41 -> 2.38 ms, RuO2 mix of 2048 5.42 -> 2.65 ms, RuO2 lat_int, 300 odd
-// lattices 5.91 -> 1.79 ms, pairwise lat_int 512 x 256x256 4.48 -> 1.85 ms
-// (kernel); one RuO2 64x64 trajectory 3.8 -> 1.24 us per step; tracking on
-// the pairwise model (264 updates in five chunks) 14.1 -> 6.5 us per step.
+// 5.42 -> 2.22 ms, RuO2 mix of 2048 5.42 -> 2.60 ms, RuO2 lat_int, 300 odd
+// lattices 5.95 -> 1.79 ms, pairwise lat_int 512 x 256x256 4.48 -> 1.85 ms
+// (kernel, the first steps after an empty lattice), Pd oxide on two layers
+// (25 sites per cell) 4.54 -> 1.62 ms; one RuO2 64x64 trajectory 3.8 -> 1.24
+// us per step; the pairwise model as local_smart (264 updates in five
+// chunks) with moves tracked 14.1 -> 4.5 us per step.
 //
 // Record of one lane (RW words, 64 lanes per chunk, the chunks of a process
 // in turn):
