@@ -108,7 +108,8 @@ struct KParams {
     long long *kstep;
     unsigned long long *rngctr;
     int *status;
-    const int *lists_ok;           // per replica: lists match the lattice (or null)
+    int *lists_ok;                 // per replica: lists match the lattice
+    int *out_ok;                   // misc kernel: the same for each replica of the launch, pinned
     long long *executed;
     long long *budget;             // optional, per launch slot
     int *out;                      // misc kernel outputs

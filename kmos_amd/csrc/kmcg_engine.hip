@@ -1557,6 +1557,8 @@ __device__ __forceinline__ void steps_end(Wave<PPL, BITS> &W, const KParams &kp,
         kp.kstep[r] = ks;
         kp.rngctr[r] = ctr;
         kp.status[r] = st;
+        if (st != ST_OK && st != ST_ABSORBING)
+            kp.lists_ok[r] = 0;
         kp.executed[slot] = (kp.resume ? kp.executed[slot] : 0) + done;
         if (kp.budget)
             kp.budget[slot] -= done;
@@ -1837,8 +1839,29 @@ __global__ __launch_bounds__(64 * MAX_WPG) void kmc_misc_kernel(KParams kp)
         }
     }
     wave_store<PPL, BITS, LDS_LAT>(W, kp, r, changed);
-    if (lane == 0)
+    if (lane == 0) {
         kp.status[r] = st;
+        // Whether the lists follow the lattice from here on (the fused loop
+        // writes without a look at it).  Touchups of every site make them
+        // follow.  A stop may leave entries behind, also an earlier one:
+        // MODE_ADJUST passes a stopped replica by, its lattice replaced
+        // already.  The search of the next step changes neither.
+        int ok = kp.lists_ok[r];
+        if (kp.mode != MODE_NEXT_STEP)
+            ok = st == ST_OK && (ok || kp.mode == MODE_INIT || kp.mode == MODE_ADJUST);
+        kp.lists_ok[r] = ok;
+        kp.out_ok[blockIdx.x * kp.wpg + (threadIdx.x >> 6)] = ok;
+    }
+}
+
+// After a call that rebuilt the lists of replicas [r0, r0+n): they follow
+// the lattice but for a replica that is stopped, whose lists were left as
+// they were.  `out` (pinned): the same for the host.
+__global__ void kmc_mark_lists_kernel(KParams kp, int r0, int n, int *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        kp.lists_ok[r0 + i] = out[i] = kp.status[r0 + i] == ST_OK;
 }
 
 // default species of every site (initialize_state); site defaults are the
@@ -2417,9 +2440,12 @@ struct kmcg_batch {
     bool use_graph = false;
     std::vector<Captured> graphs;     // oldest first, at most MAX_GRAPHS
     // 1 per replica whose lists match its lattice (set by kmcg_init and
-    // kmcg_set_config, cleared by kmcg_replace_species and kmcg_set_state)
+    // kmcg_set_config where the replica is not stopped, cleared by
+    // kmcg_replace_species, kmcg_set_state and every stop on an error)
     int *lists_ok = nullptr;
-    std::vector<unsigned char> lists_ok_h;   // the same on the host
+    // the same on the host (a stop inside a run is taken over by the call
+    // that lets the replica go on: until then it takes no step)
+    std::vector<unsigned char> lists_ok_h;
     // displacement tracking (kmcg_msd_*): allocated by the first kmcg_msd_init
     int *msd_hop = nullptr;
     double *msd_d = nullptr;
@@ -3573,8 +3599,11 @@ int run_misc(kmcg_batch *b, const std::vector<int> &ids, int mode, int a0, int a
     const Shape s = launch_shape(b, ids.data(), (int)ids.size(), kp, MAX_WPG);
     kp.mode = mode;
     kp.arg0 = a0; kp.arg1 = a1; kp.arg2 = a2; kp.arg3 = a3;
+    kp.out_ok = b->h_ids;                                // (no run is in flight)
     HIPCHK(launch(b, false, s, kp));
     HIPCHK(hipStreamSynchronize(b->stream));
+    for (size_t i = 0; i < ids.size(); ++i)
+        b->lists_ok_h[ids[i]] = (unsigned char)b->h_ids[i];
     return KMCG_OK;
 }
 
@@ -3961,15 +3990,26 @@ static int pack_configs(kmcg_batch *b, int r0, int n, const int8_t *config, std:
 }
 
 namespace {
-// mark replicas [r0, r0+n) as having lists that do (1) or may not (0) match
-// their lattices, behind the batch's queued work, and wait for both
-int set_lists_ok(kmcg_batch *b, int r0, int n, int v)
+// replicas [r0, r0+n): their lists may no longer match their lattices.
+// Called before the first change, so that an error halfway leaves no mark.
+int clear_lists_ok(kmcg_batch *b, int r0, int n)
 {
     HIPCHK(hipSetDevice(b->device));
-    HIPCHK(hipMemsetD32Async((hipDeviceptr_t)(b->lists_ok + r0), v, n, b->stream));
+    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)0);
+    HIPCHK(hipMemsetD32Async((hipDeviceptr_t)(b->lists_ok + r0), 0, n, b->stream));
+    return settle(b);
+}
+
+// their lists were rebuilt, by work that is queued on the batch's stream:
+// marks them behind it and waits (kmc_mark_lists_kernel)
+int mark_lists_ok(kmcg_batch *b, int r0, int n)
+{
+    hipLaunchKernelGGL(kmc_mark_lists_kernel, dim3((n + 255) / 256), dim3(256), 0, b->stream, make_params(b), r0, n,
+                       b->h_ids);
+    HIPCHK(hipGetLastError());
     const int rc = settle(b);
-    if (!rc)
-        std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)v);
+    for (int i = 0; i < n && !rc; ++i)
+        b->lists_ok_h[r0 + i] = (unsigned char)b->h_ids[i];
     return rc;
 }
 } // namespace
@@ -3991,6 +4031,7 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
             return rc;
     }
     const long long P = b->m->P;
+    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)0);
     std::vector<unsigned> st(n, 0u);
     if (streams)
         st.assign(streams, streams + n);
@@ -4025,7 +4066,7 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
     else
         hipLaunchKernelGGL((kmc_init_lists_kernel<8>), grid, dim3(256), 0, b->stream, kp);
     HIPCHK(hipGetLastError());
-    return set_lists_ok(b, r0, n, 1);
+    return mark_lists_ok(b, r0, n);
 }
 
 int kmcg_check_lists(kmcg_batch *b, int32_t r0, int32_t n, int32_t *bad)
@@ -4092,6 +4133,7 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
     int rc = pack_configs(b, r0, n, config, packed);
     if (rc || (rc = settle(b)))
         return rc;
+    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)0);
     HIPCHK(hipMemcpyAsync(b->lat_pool + b->lat_off[r0], packed.data(), packed.size(), hipMemcpyHostToDevice, b->stream));
     std::vector<int> ids(n);
     long long cells = 0;
@@ -4116,10 +4158,9 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
         else
             hipLaunchKernelGGL((kmc_adjust_lists_kernel<8, false>), grid, dim3(256), 0, b->stream, kp);
         HIPCHK(hipGetLastError());
-        return set_lists_ok(b, r0, n, 1);
+        return mark_lists_ok(b, r0, n);
     }
-    rc = run_misc(b, ids, MODE_ADJUST, 0, 0, 0, 0);
-    return rc ? rc : set_lists_ok(b, r0, n, 1);
+    return run_misc(b, ids, MODE_ADJUST, 0, 0, 0, 0);
 }
 
 // track: bit 0 displacement tracking, bit 1 trajectory, bit 2 ACF bins
@@ -4436,7 +4477,7 @@ int kmcg_replace_species(kmcg_batch *b, int32_t r, int32_t site, int32_t old_sp,
     if (lat[site - 1] != old_sp)
         return fail(KMCG_EINVAL, "replace_species: site holds another species");
     // the lists no longer follow the lattice until the next set_config
-    if ((rc = set_lists_ok(b, r, 1, 0)))
+    if ((rc = clear_lists_ok(b, r, 1)))
         return rc;
     const long long s = site - 1;
     const long long byte = b->bits == 8 ? s : (s * 2) >> 3;
@@ -5048,7 +5089,9 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
     const std::vector<double> ig = integ_rates ? std::vector<double>(integ_rates, integ_rates + P)
                                                : std::vector<double>(P, 0.0);
     const int running = 0;
-    if ((rc = copy_in(b, b->lat_pool + b->lat_off[r], packed.data(), packed.size())) ||
+    // (a restored state is not checked against its lattice)
+    if ((rc = clear_lists_ok(b, r, 1)) ||
+        (rc = copy_in(b, b->lat_pool + b->lat_off[r], packed.data(), packed.size())) ||
         (rc = copy_in(b, b->avail_pool + b->avail_off[r], blk.data(), blk.size())) ||
         (rc = copy_in(b, b->nr + r * P, (const int *)nr_of_sites, (size_t)P)) ||
         (rc = copy_in(b, b->pstat + r * P, (const long long *)procstat, (size_t)P)) ||
@@ -5058,7 +5101,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
         (rc = copy_in(b, b->rngctr + r, (const unsigned long long *)(step2 + 1), 1)) ||
         (rc = copy_in(b, b->status + r, &running, 1)))
         return rc;
-    return set_lists_ok(b, r, 1, 0);      // a restored state is not checked against its lattice
+    return KMCG_OK;
 }
 
 int kmcg_get_occupation(kmcg_batch *b, int32_t r0, int32_t n, double *out)

@@ -1,0 +1,77 @@
+"""A stopped replica keeps its lists when set_config replaces its lattice.
+touchup and run_proc_nr let it go on; the lists then name processes whose
+conditions do not hold, and the run has to stop at the first of them whose
+write finds another species, as the oracle does, and must not write there.
+
+local_smart: in the oracle's state.  lat_int: at the oracle's step with a
+stop status (the deletion of an entry that is not registered is undefined in
+the reference, and the engine applies a step's deletions after its writes)."""
+import numpy as np
+import pytest
+
+from kmos_amd import workloads as W
+from kmos_amd.compiler import compile_model
+from paritylib import compare_state, oracle_replica
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("way", ["touchup", "run_proc_nr"])
+@pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
+def test_new_lattice_of_a_stopped_replica(engine, oracle, backend, way):
+    pt = W.zgb_project()
+    cm = compile_model(pt, backend)
+    sid = pt.species_ids()
+    sizes = [(12, 16), (9, 18)]
+    seeds = np.array([5, 6], np.uint32)
+    rates = np.tile([5.0, 1.0, 1.0, 1.0, 1.0, 0.5, 0.5], (2, 1))
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init(seeds)
+    b.set_rates(rates)
+    orcs = [oracle_replica(oracle, cm, s, int(seeds[r]), 0, rates[r]) for r, s in enumerate(sizes)]
+    b.run(40)
+    b.set_rates(0.0 * rates)
+    b.run(1)
+    for o in orcs:
+        o.run(40)
+        o.set_rates(0.0 * rates[0])
+        o.run(1)
+    assert list(b.scalars_all()[2]) == [1, 1] and all(o.status == 1 for o in orcs)
+    # other species in the lower rows, the upper ones as they are
+    g = np.random.default_rng(2)
+    before = [b.avail(r) for r in range(2)]
+    configs = []
+    for r, (X, Y) in enumerate(sizes):
+        lat = b.lattice(r).copy()
+        lat[:X * (Y // 2)] = g.integers(0, cm.nr_of_species, X * (Y // 2))
+        configs.append(lat)
+    b.set_config(configs)
+    b.set_rates(rates)
+    for r, o in enumerate(orcs):
+        st = o.get_state(rates[r])
+        st["lattice"] = configs[r]
+        o.set_state(st)
+        for got, kept in zip(b.avail(r), before[r]):
+            np.testing.assert_array_equal(got, kept)
+        X, Y = sizes[r]
+        if way == "touchup":
+            b.touchup(r, 1, Y - 4, 0, 1)
+            o.touchup(1, Y - 4, 0, 1)
+        else:
+            # CO adsorbs on an empty site far from the rows that changed
+            x = int(np.nonzero(configs[r].reshape(Y, X)[Y - 4] == sid["empty"])[0][0])
+            proc = cm.process_names.index("CO_adsorption") + 1
+            b.run_proc_nr(r, proc, (Y - 4) * X + x + 1)
+            o.run_proc_nr(proc, (Y - 4) * X + x + 1)
+        compare_state(b, r, o, where="%s replica %d" % (way, r))
+        assert o.status == 0
+    b.run(300)
+    for r, o in enumerate(orcs):
+        o.run(300)
+        assert o.status != 0
+        if backend == "local_smart":
+            compare_state(b, r, o, where="%s replica %d after its stop" % (way, r))
+        else:
+            _, _, ks, ctr, st = b.scalars(r)
+            assert st in (2, 3) and ks == o.kmc_step and ctr == o.rng_ctr, (st, ks, o.kmc_step)
+    b.close()
