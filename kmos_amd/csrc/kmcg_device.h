@@ -163,6 +163,10 @@ struct KParams {
 
 constexpr int PHASE_W = 8;
 
+// KParams::lists_ok of a replica with a list found corrupt, until
+// kmc_mark_lists_kernel has stopped it
+constexpr int LISTS_CORRUPT = -1;
+
 constexpr int MSD_HOP_W = 9;
 
 // ---- helpers --------------------------------------------------------------

@@ -1856,12 +1856,18 @@ __global__ __launch_bounds__(64 * MAX_WPG) void kmc_misc_kernel(KParams kp)
 
 // After a call that rebuilt the lists of replicas [r0, r0+n): they follow
 // the lattice but for a replica that is stopped, whose lists were left as
-// they were.  `out` (pinned): the same for the host.
+// they were, and one with a list found corrupt (LISTS_CORRUPT, left by the
+// workgroups that met it), which stops here, when no workgroup reads the
+// status any more.  `out` (pinned): the same for the host.
 __global__ void kmc_mark_lists_kernel(KParams kp, int r0, int n, int *out)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        kp.lists_ok[r0 + i] = out[i] = kp.status[r0 + i] == ST_OK;
+    if (i >= n)
+        return;
+    const int r = r0 + i;
+    if (kp.lists_ok[r] == LISTS_CORRUPT)
+        kp.status[r] = ST_CORRUPT;
+    kp.lists_ok[r] = out[i] = kp.status[r] == ST_OK;
 }
 
 // default species of every site (initialize_state); site defaults are the
@@ -2057,27 +2063,28 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
     const int *cd = prog + cbase + (int)((unsigned)w1 >> 21);
     int n = kp.nr[(long long)r * P + p];
     const int n0 = n;
-    if (n < 0 || n > ncell) {                    // a replica that was never initialised
+    if (n < 0 || n > ncell) {                    // no list of this process
         if (threadIdx.x == 0)
-            kp.status[r] = ST_CORRUPT;
+            kp.lists_ok[r] = LISTS_CORRUPT;
         return;
     }
     if (threadIdx.x == 0)
         count = 0;
     __syncthreads();
-    // in LDS: list[1..ncell] of cells, then the slot of every cell
+    // in LDS: list[1..ncell] of cells, then the slot of every cell.  Every
+    // entry that will be followed is a site of this process.
     unsigned short *list = adj, *slot = adj + ncell + 1;
-    if (INLDS) {
+    if (INLDS)
         for (int c = threadIdx.x; c < ncell; c += 256)
             slot[c] = (unsigned short)bp[kp.spuck * c + n_exec];
-        for (int k = threadIdx.x + 1; k <= n; k += 256) {
-            const int c = (sp[k] - n_exec) / kp.spuck;
-            if (c < 0 || c >= ncell)
-                count = -1;
+    for (int k = threadIdx.x + 1; k <= n; k += 256) {
+        const int at = sp[k] - n_exec, c = at / kp.spuck;
+        if (at < 0 || c >= ncell || at != c * kp.spuck)
+            count = -1;
+        if (INLDS)
             list[k] = (unsigned short)c;
-        }
-        __syncthreads();
     }
+    __syncthreads();
     for (int t = 0; t < ncell; t += 256) {
         const int i = t + threadIdx.x;
         bool en = false, reg = false;
@@ -2112,9 +2119,10 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
             const int m = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
             for (int j = 0; j < m; ++j) {
                 const int e = ev[j], cell = e >> 2;
-                // (an inverse index that points outside the list)
                 const int at0 = e & 2 ? (INLDS ? (int)slot[cell] : bp[kp.spuck * cell + n_exec]) : 1;
-                if (at0 < 1 || ((e & 2) && at0 > n)) {
+                // an inverse index that points outside the list, or an
+                // addition to a full one
+                if (at0 < 1 || ((e & 2) && at0 > n) || (e == (cell << 2 | 1) && n >= ncell)) {
                     count = -1;
                     break;
                 }
@@ -2150,7 +2158,7 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
     }
     if (count < 0) {
         if (threadIdx.x == 0)
-            kp.status[r] = ST_CORRUPT;
+            kp.lists_ok[r] = LISTS_CORRUPT;
         return;
     }
     if (threadIdx.x == 0)
@@ -3916,6 +3924,7 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     if (hipMemsetAsync(b->rates, 0, n * P * sizeof(double), b->stream) != hipSuccess ||
         hipMemsetAsync(b->status, 0, n * sizeof(int), b->stream) != hipSuccess ||
         hipMemsetAsync(b->lists_ok, 0, n * sizeof(int), b->stream) != hipSuccess ||
+        hipMemsetAsync(b->nr, 0, n * P * sizeof(int), b->stream) != hipSuccess ||
         hipMemsetAsync(b->avail_pool, 0, b->avail_total * sizeof(int), b->stream) != hipSuccess ||
         hipMemsetAsync(b->lat_pool, 0, b->lat_total, b->stream) != hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)

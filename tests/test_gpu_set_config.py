@@ -48,3 +48,52 @@ def test_set_config_matches_oracle(engine, oracle, name, factory, backend, sizes
             o.run(steps)
             compare_state(b, i, o, where="%s %s steps %d" % (name, sizes[i], rnd))
     b.close()
+
+
+@pytest.mark.parametrize("name,factory,backend,sizes", [
+    ("quickstart", W.quickstart_project, "local_smart", [(5, 3), (16, 17), (215, 211)]),
+    ("ruo2", W.ruo2_project, "local_smart", [(9, 13), (16, 17)]),
+    ("zgb_li", W.zgb_project, "lat_int", [(9, 13), (16, 17)]),
+], ids=["quickstart", "ruo2", "zgb_li"])
+def test_set_config_before_init(engine, oracle, name, factory, backend, sizes):
+    """Replicas that were never initialised have empty lists, whatever the
+    memory they lie in held: a configuration builds the lists from nothing."""
+    pt = factory()
+    cm = compile_model(pt, backend)
+    g = np.random.default_rng(29)
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    configs = [random_config(pt, int(v), g) for v in b.volumes]
+    b.set_config(configs)
+    for i, s in enumerate(sizes):
+        o = oracle.Oracle(cm.to_blob(), s)
+        o.set_config(configs[i])
+        assert b.scalars(i)[4] == 0
+        np.testing.assert_array_equal(b.lattice(i), o.lattice())
+        np.testing.assert_array_equal(b.nr_of_sites(i), o.nr_of_sites())
+        for got, want in zip(b.avail(i), o.avail()):
+            np.testing.assert_array_equal(got, want)
+    assert (b.check_lists() == 0).all()
+    b.close()
+
+
+def test_set_config_fills_and_empties_lists(engine, oracle):
+    """Every cell in one list, none, every one again: an addition to a list
+    one short of full, with the list in LDS and in memory."""
+    pt = W.quickstart_project()
+    cm = compile_model(pt, "local_smart")
+    ids = pt.species_ids()
+    sizes = [(1, 1), (5, 3), (16, 16), (215, 211)]
+    rates = np.full((len(sizes), 2), 3.0)
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init(np.arange(len(sizes), dtype=np.uint32))
+    b.set_rates(rates)
+    orcs = [oracle_replica(oracle, cm, s, i, 0, rates[i]) for i, s in enumerate(sizes)]
+    for species in ("CO", "empty", "CO", "CO", "empty"):
+        configs = [np.full(int(v), ids[species], np.int8) for v in b.volumes]
+        b.set_config(configs)
+        b.run(1)
+        for i, o in enumerate(orcs):
+            o.set_config(configs[i])
+            o.run(1)
+            compare_state(b, i, o, where="%s %s" % (species, sizes[i]))
+    b.close()
