@@ -2018,7 +2018,8 @@ __global__ __launch_bounds__(256) void kmc_init_lists_kernel(KParams kp)
 }
 
 // _adjust_database after a new lattice (kmos/run/__init__.py:1439-1457),
-// one workgroup per (replica, process).  The touchups, x outermost, visit
+// one workgroup of 256 threads per (replica, process), for whole lists (each
+// site once, of the process's own type).  The touchups, x outermost, visit
 // every site once; a visit deletes the site's entry of each process anchored
 // there, then adds it if its conditions hold.  The lists of different
 // processes do not meet, and whether a site is registered when it is visited
@@ -2454,6 +2455,12 @@ struct kmcg_batch {
     // the same on the host (a stop inside a run is taken over by the call
     // that lets the replica go on: until then it takes no step)
     std::vector<unsigned char> lists_ok_h;
+    // 1 per replica whose lists hold each site once, and sites of the
+    // process's own type only, whatever the lattice says.  Steps on lists
+    // that do not follow the lattice lose it (an addition may find its entry
+    // in the list), a restored state may come without it, kmcg_init gives it
+    // back.
+    std::vector<unsigned char> lists_whole_h;
     // displacement tracking (kmcg_msd_*): allocated by the first kmcg_msd_init
     int *msd_hop = nullptr;
     double *msd_d = nullptr;
@@ -3874,6 +3881,7 @@ int kmcg_batch_create(const kmcg_model *m, int32_t n, const int32_t *sizes, int3
     BALLOC(b->prog, fz_at + m->fz.size());
     b->fz = b->prog + fz_at;
     b->lists_ok_h.assign(n, 0);
+    b->lists_whole_h.assign(n, 1);               // (empty)
     BALLOC(b->dims, n + (n + 3) / 4);            // then the list 0, 1, 2, ...
     b->iota = (int *)(b->dims + n);
     BALLOC(b->lat_off_d, n);
@@ -4075,7 +4083,10 @@ int kmcg_init(kmcg_batch *b, int32_t r0, int32_t n, const uint32_t *seeds, const
     else
         hipLaunchKernelGGL((kmc_init_lists_kernel<8>), grid, dim3(256), 0, b->stream, kp);
     HIPCHK(hipGetLastError());
-    return mark_lists_ok(b, r0, n);
+    rc0 = mark_lists_ok(b, r0, n);
+    if (!rc0)
+        std::fill(b->lists_whole_h.begin() + r0, b->lists_whole_h.begin() + r0 + n, (unsigned char)1);
+    return rc0;
 }
 
 int kmcg_check_lists(kmcg_batch *b, int32_t r0, int32_t n, int32_t *bad)
@@ -4150,7 +4161,8 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
         ids[i] = r0 + i;
         cells = std::max(cells, (long long)b->X[r0 + i] * b->Y[r0 + i] * b->Z[r0 + i]);
     }
-    if (b->m->adjust_lists) {
+    const bool whole = !memchr(&b->lists_whole_h[r0], 0, n);
+    if (b->m->adjust_lists && whole) {
         KParams kp = make_params(b);
         kp.rep_ids = b->iota + r0;
         kp.arg0 = b->m->off_init;
@@ -4169,7 +4181,13 @@ int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config)
         HIPCHK(hipGetLastError());
         return mark_lists_ok(b, r0, n);
     }
-    return run_misc(b, ids, MODE_ADJUST, 0, 0, 0, 0);
+    // one touchup after the other.  A site's second entry stays (the inverse
+    // index names the other one): such lists follow no lattice.
+    rc = run_misc(b, ids, MODE_ADJUST, 0, 0, 0, 0);
+    for (int i = r0; i < r0 + n && !rc && !whole; ++i)
+        if (!b->lists_whole_h[i])
+            rc = clear_lists_ok(b, i, 1);
+    return rc;
 }
 
 // track: bit 0 displacement tracking, bit 1 trajectory, bit 2 ACF bins
@@ -4190,6 +4208,8 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     int rc = settle(b);      // the staging buffers belong to one run at a time
     if (rc)
         return rc;
+    for (int i = 0; i < n; ++i)
+        b->lists_whole_h[replicas[i]] &= b->lists_ok_h[replicas[i]];
     const int first = contiguous(replicas, n);           // no list to send then
     if (first < 0)
         memcpy(b->h_ids, replicas, n * sizeof(int));
@@ -4457,6 +4477,7 @@ int kmcg_run_proc_nr(kmcg_batch *b, int32_t r, int32_t proc, int32_t site)
         return rc;
     if (proc < 1 || proc > b->m->P || site < 1 || site > b->V[r])
         return fail(KMCG_EINVAL, "process or site out of range");
+    b->lists_whole_h[r] &= b->lists_ok_h[r];
     return run_misc(b, {r}, MODE_RUN_PROC, proc, site, 0, 0);
 }
 
@@ -5068,8 +5089,11 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
     // every list index and site the kernels will follow is checked here:
     // an inconsistent list would send add_proc/del_proc out of the row
     std::vector<int> blk(2 * P * V1, 0);
+    bool whole = true;
     for (long long p = 0; p < P; ++p) {
         const long long nr = nr_of_sites[p];
+        // the process's own site type
+        const int n0 = b->m->backend == 0 ? b->m->blob[b->m->blob[9] + 3 * p] : 1;
         if (nr < 0 || nr > V)
             return fail(KMCG_EINVAL, "set_state: nr_of_sites out of range");
         const int32_t *sp = sites + p * V, *bp = back + p * V;
@@ -5079,6 +5103,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
             if (i <= nr) {
                 if (s < 1 || s > V || bp[s - 1] != i)
                     return fail(KMCG_EINVAL, "set_state: avail_sites and avail_sites_back disagree");
+                whole &= (s - n0) % b->m->spuck == 0;
             } else if (s != 0) {
                 return fail(KMCG_EINVAL, "set_state: avail_sites holds entries beyond nr_of_sites");
             }
@@ -5099,6 +5124,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
                                                : std::vector<double>(P, 0.0);
     const int running = 0;
     // (a restored state is not checked against its lattice)
+    b->lists_whole_h[r] = 0;
     if ((rc = clear_lists_ok(b, r, 1)) ||
         (rc = copy_in(b, b->lat_pool + b->lat_off[r], packed.data(), packed.size())) ||
         (rc = copy_in(b, b->avail_pool + b->avail_off[r], blk.data(), blk.size())) ||
@@ -5110,6 +5136,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
         (rc = copy_in(b, b->rngctr + r, (const unsigned long long *)(step2 + 1), 1)) ||
         (rc = copy_in(b, b->status + r, &running, 1)))
         return rc;
+    b->lists_whole_h[r] = whole;
     return KMCG_OK;
 }
 

@@ -75,3 +75,78 @@ def test_new_lattice_of_a_stopped_replica(engine, oracle, backend, way):
             _, _, ks, ctr, st = b.scalars(r)
             assert st in (2, 3) and ks == o.kmc_step and ctr == o.rng_ctr, (st, ks, o.kmc_step)
     b.close()
+
+
+def test_entries_listed_twice(engine, oracle):
+    """A step on a database that replace_species left stale adds entries that
+    are listed already.  set_config takes one of the two away, as the oracle
+    does; the run then stops where a step finds that the other does not
+    hold."""
+    pt = W.zgb_project()
+    cm = compile_model(pt, "local_smart")
+    sid = pt.species_ids()
+    X, Y = 12, 10
+    rates = np.array([[0.5, 1.0, 1.0, 1.0, 1.0, 5.0, 5.0]])
+    g = np.random.default_rng(4)
+    lat = g.choice([sid["O"], sid["empty"]], size=X * Y).astype(np.int8)
+    rows = lat.reshape(Y, X)
+    rows[3, 2:6] = [sid["empty"], sid["empty"], sid["O"], sid["empty"]]
+    rows[2, 3] = rows[4, 3] = sid["empty"]
+    b = engine.Batch(engine.Model(cm), [(X, Y, 1)])
+    b.init([5], [0])
+    b.set_rates(rates)
+    b.set_config([lat])
+    o = oracle_replica(oracle, cm, (X, Y), 5, 0, rates[0], lat)
+    site, proc = 3 * X + 3 + 1, cm.process_names.index("CO_oxidation1") + 1
+    b.replace_species(0, site, sid["empty"], sid["CO"])
+    oracle.lib().orc_replace_species(o.h, site, sid["empty"], sid["CO"])
+    b.run_proc_nr(0, proc, site)
+    o.run_proc_nr(proc, site)
+    compare_state(b, 0, o, where="after the step")
+    sites, _ = o.avail()
+    listed = [s[:n] for s, n in zip(sites, o.nr_of_sites())]
+    assert any(np.unique(s).size < s.size for s in listed)
+    new = g.integers(0, cm.nr_of_species, X * Y).astype(np.int8)
+    b.set_config([new])
+    o.set_config(new)
+    compare_state(b, 0, o, where="after set_config")
+    b.run(400)
+    o.run(400)
+    assert o.status == 2
+    compare_state(b, 0, o, where="after the run")
+    b.close()
+
+
+def test_restored_entries_of_another_site_type(engine, oracle):
+    """set_state takes lists as they are given, a site of a type that the
+    process never runs on among them; set_config leaves what the oracle's
+    touchups leave."""
+    pt = W.ruo2_project()
+    cm = compile_model(pt, "local_smart")
+    g = np.random.default_rng(8)
+    size = (7, 6)
+    rates = 10.0 ** g.uniform(-1, 3, (1, cm.nr_of_proc))
+    b = engine.Batch(engine.Model(cm), [size + (1,)])
+    b.init([5], [0])
+    b.set_rates(rates)
+    b.run(60)
+    o = oracle_replica(oracle, cm, size, 5, 0, rates[0])
+    o.run(60)
+    st = o.get_state(rates[0])
+    p = int(np.argmax(st["nr_of_sites"]))
+    k = int(st["nr_of_sites"][p])
+    other = int(st["avail_sites"][p, 0]) + (1 if st["avail_sites"][p, 0] % 2 else -1)
+    st["avail_sites"][p, k] = other
+    st["avail_sites_back"][p, other - 1] = k + 1
+    st["nr_of_sites"][p] = k + 1
+    b.set_state(0, st)
+    o.set_state(st)
+    compare_state(b, 0, o, where="restored")
+    new = g.integers(0, cm.nr_of_species, int(b.volumes[0])).astype(np.int8)
+    b.set_config([new])
+    o.set_config(new)
+    compare_state(b, 0, o, where="after set_config")
+    b.run(200)
+    o.run(200)
+    compare_state(b, 0, o, where="after the run")
+    b.close()
