@@ -152,6 +152,10 @@ int kmcg_set_graph(kmcg_batch *b, int32_t enable);
 /* Milliseconds the last kmcg_run took on the device (HIP events around the
  * kernel on the batch's stream). */
 int kmcg_last_run_ms(kmcg_batch *b, float *ms);
+/* The step loop the last run took: 0 a generic one, else the form of the
+ * fused loop's records (info6[1] of kmcg_model_fused).  No counterpart in
+ * the reference (a test aid). */
+int kmcg_last_form(const kmcg_batch *b, int32_t *form);
 /* Phase profile of the step loop, for replicas r0..r0+n-1: out[n][8] holds
  * the shader-clock ticks each replica's wave spent selecting (accumulate,
  * clock, search), reading its site, posting the process's ops, replaying

@@ -71,6 +71,10 @@ int kmcg_otf_sync(kmcg_otf_batch *b);
 /* Kernel time of the last kmcg_otf_run, in milliseconds (HIP events on the
  * batch's stream). */
 int kmcg_otf_last_run_ms(kmcg_otf_batch *b, float *ms);
+/* The step loop of the last kmcg_otf_run: 1 with one lane per list
+ * operation, 0 the general one.  No counterpart in the reference (a test
+ * aid). */
+int kmcg_otf_last_form(const kmcg_otf_batch *b, int32_t *form);
 
 /* base.get_kmc_time, get_kmc_time_step, get_kmc_step and the replica's
  * status. */

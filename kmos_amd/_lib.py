@@ -29,6 +29,7 @@ SIGNATURES = [
     ("kmcg_model_info", _i32, [_vp, _vp]),
     ("kmcg_model_forms", _i32, [_vp, _vp]),
     ("kmcg_model_fused", _i32, [_vp, _vp, _vp]),
+    ("kmcg_last_form", _i32, [_vp, _vp]),
     ("kmcg_batch_footprint", _i32, [_vp, _i32, _vp, _vp]),
     ("kmcg_batch_create", _i32, [_vp, _i32, _vp, _i32, _vp]),
     ("kmcg_batch_free", None, [_vp]),
@@ -87,6 +88,7 @@ SIGNATURES = [
     ("kmcg_otf_set_config", _i32, [_vp, _i32, _i32, _vp]),
     ("kmcg_otf_run", _i32, [_vp, _i32, _i32, _i64]),
     ("kmcg_otf_sync", _i32, [_vp]),
+    ("kmcg_otf_last_form", _i32, [_vp, _vp]),
     ("kmcg_otf_last_run_ms", _i32, [_vp, _vp]),
     ("kmcg_otf_get_scalars", _i32, [_vp, _i32, _vp, _vp, _vp, _vp]),
     ("kmcg_otf_get_lattice", _i32, [_vp, _i32, _vp]),

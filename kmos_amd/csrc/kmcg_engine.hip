@@ -2372,7 +2372,7 @@ struct kmcg_model {
     bool adjust_lists = false;   // _adjust_database list by list (kmc_adjust_lists_kernel)
     // the fused step loop's records (kmcg_fused.hip; empty: not for this model)
     std::vector<int> fz;
-    int fz_form = 0;     // FZ_1, FZ_4 or FZ_LI
+    int fz_form = 0;     // FZ_1, FZ_4, FZ_M or FZ_LI
     int fz_nch = 1;      // chunks of 64 records per process
     int fz_moff = 0;     // largest offset component of the records
     int fz_tab_off = 0, fz_tab_bytes = 0;    // FZ_LI: the groups' tables behind the records
@@ -2418,6 +2418,7 @@ struct kmcg_batch {
     long long *budget = nullptr;
     int *rep_ids = nullptr;
     const int *run_ids = nullptr;       // the list of the last run
+    int last_form = 0;                  // the step loop it took (kmcg_last_form)
     int *out = nullptr;
     unsigned long long *phase = nullptr;   // phase counters (KMCG_PHASES builds)
     double *occ = nullptr;
@@ -3483,10 +3484,11 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
            (b->ov_mode == -1 && b->m->backend == 0 && b->m->P > 16 && (long long)n <= 8LL * b->n_cu);
     size_t shared = prog;
     // the fused step loop, faster than the others at every size measured
-    // (1.7 to 3.3 times, one replica of 20x20 to 4096 of 128x128), wherever
+    // (1.6 to 3.3 times, one replica of 20x20 to 4096 of 128x128), wherever
     // it is sound: the lists of every replica follow its lattice, no two
     // offsets of the records meet (extents of 2 * reach + 1 and more), the
-    // lattice fits LDS, and no other form was asked for
+    // lattice fits LDS, and no other form was asked for.  One replica it
+    // cannot take sends the whole launch to the generic loops.
     const size_t fz_wave = (size_t)maxlb + (64 * WIN + occ) * sizeof(int);
     s.fz = steps && !b->m->fz.empty() && (steps == 1 || b->m->fz_form != FZ_M) && b->ov_mode == -1 && b->lds_mode != 0 &&
            (size_t)b->m->fz_tab_bytes + fz_wave <= (size_t)b->max_lds;
@@ -3749,6 +3751,14 @@ int kmcg_model_fused(const kmcg_model *m, int32_t *info6, int32_t *words)
     info6[4] = m->fz_tab_off; info6[5] = m->fz_tab_bytes;
     if (words && !m->fz.empty())
         memcpy(words, m->fz.data(), m->fz.size() * sizeof(int));
+    return KMCG_OK;
+}
+
+int kmcg_last_form(const kmcg_batch *b, int32_t *form)
+{
+    if (!b || !form)
+        return fail(KMCG_EINVAL, "null argument");
+    *form = b->last_form;
     return KMCG_OK;
 }
 
@@ -4224,6 +4234,7 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
         kp.rep_ids = b->iota + first;
     b->run_ids = kp.rep_ids;
     const Shape s = launch_shape(b, replicas, n, kp, b->max_wpg, records || track ? 2 : 1);
+    b->last_form = s.fz_form;
     kp.nsteps = steps;
     kp.budget = budget ? b->budget : nullptr;
     // behind a fused run that may stop short of a step it cannot take: the

@@ -1090,6 +1090,7 @@ struct kmcg_otf_batch {
     unsigned *d_seed = nullptr, *d_stream = nullptr;
     std::vector<double> rates, userpar;  // per replica, as last set
     double *h_out = nullptr;             // OtfParams::out
+    int last_form = 0;                   // kmcg_otf_last_form
     const long long *out(int r) const { return (const long long *)h_out + (size_t)r * OTF_OUT(m->P); }
     int status(int r) const { return (int)out(r)[4 * m->P + 3]; }
 };
@@ -1542,6 +1543,8 @@ int otf_launch(kmcg_otf_batch *b, int32_t r0, int32_t n, long long steps, int mo
     for (int i = 0; i < n && fast; ++i)
         for (int d = 0; d < 3; ++d)
             fast = fast && b->dims[4 * (r0 + i) + d] >= 2 * b->m->op_reach[d] + 1;
+    if (mode < 0)
+        b->last_form = fast;
     if (timed)
         HIPCHK(hipEventRecord(b->ev0, b->stream));
     if (fast)
@@ -1859,6 +1862,14 @@ int kmcg_otf_sync(kmcg_otf_batch *b)
     if (!b)
         return fail(KMCG_EINVAL, "null batch");
     return otf_sync(b);
+}
+
+int kmcg_otf_last_form(const kmcg_otf_batch *b, int32_t *form)
+{
+    if (!b || !form)
+        return fail(KMCG_EINVAL, "null argument");
+    *form = b->last_form;
+    return KMCG_OK;
 }
 
 int kmcg_otf_last_run_ms(kmcg_otf_batch *b, float *ms)

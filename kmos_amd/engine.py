@@ -200,6 +200,13 @@ class Batch:
         _lib.check(_lib.load().kmcg_last_run_ms(self.h, ctypes.byref(v)))
         return float(v.value)
 
+    def last_form(self) -> int:
+        """The step loop the last run took: 0 a generic one, else the form
+        of the fused loop's records."""
+        v = ctypes.c_int32(0)
+        _lib.check(_lib.load().kmcg_last_form(self.h, ctypes.byref(v)))
+        return int(v.value)
+
     def phase_profile(self, r0: int = 0, n: Optional[int] = None) -> np.ndarray:
         """Step-loop phase counters of replicas r0.. ([n][8]: ticks in
         select, site read, post, replay, rest; steps), cleared after the

@@ -128,6 +128,13 @@ class OtfBatch:
         _lib.check(_lib.load().kmcg_otf_last_run_ms(self.h, ctypes.byref(ms)))
         return ms.value
 
+    def last_form(self) -> int:
+        """The step loop the last run took: 1 with one lane per list
+        operation, 0 the general one."""
+        v = ctypes.c_int32(0)
+        _lib.check(_lib.load().kmcg_otf_last_form(self.h, ctypes.byref(v)))
+        return int(v.value)
+
     # ---- state ---------------------------------------------------------------
     def scalars(self, r: int):
         """(kmc_time, kmc_step, status name)"""

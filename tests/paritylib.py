@@ -45,6 +45,39 @@ def pdopd_project():
     return load_project(model_file("pdopd.xml"))
 
 
+def four_species_project(bystanders=False):
+    """One layer with four species, so that the engine holds a byte per site:
+    ZGB with a third adsorbate that hops and leaves in pairs.  With
+    `bystanders`, CO leaves in 16 processes that name two neighbours, so that
+    an update keeps two conditions open."""
+    import itertools
+
+    from kmos_amd.model import CondAct, Coord, Layer, Process, Project, Site
+    species = ["CO", "N", "O", "empty"]
+    pt = Project(model_name="four_species", model_dimension=2, species=species, default_species="empty",
+                 layers=[Layer("sc", [Site("site", (0.5, 0.5, 0.5))])], default_layer="sc", substrate_layer="sc")
+
+    def s(sp, off=(0, 0, 0)):
+        return CondAct(sp, Coord(name="site", offset=off, layer="sc"))
+
+    pairs = [(1, 0, 0), (0, 1, 0)]
+    around = pairs + [(-1, 0, 0), (0, -1, 0)]
+    procs = [Process("%s_adsorption" % sp, "1.", [s("empty")], [s(sp)]) for sp in ("CO", "N")]
+    for i, d in enumerate(pairs):
+        procs.append(Process("O2_adsorption%d" % i, "1.", [s("empty"), s("empty", d)], [s("O"), s("O", d)]))
+        procs.append(Process("N2_desorption%d" % i, "1.", [s("N"), s("N", d)], [s("empty"), s("empty", d)]))
+    for i, d in enumerate(around):
+        procs.append(Process("CO_oxidation%d" % i, "1.", [s("CO"), s("O", d)], [s("empty"), s("empty", d)]))
+        procs.append(Process("N_hop%d" % i, "1.", [s("N"), s("empty", d)], [s("empty"), s("N", d)]))
+    sides = list(itertools.product(species, species)) if bystanders else [None]
+    for i, side in enumerate(sides):
+        near = [s(side[0], (1, 0, 0)), s(side[1], (-1, 0, 0))] if side else []
+        procs.append(Process("CO_desorption%d" % i, "1.", [s("CO")] + near, [s("empty")]))
+    pt.processes = procs
+    pt.validate()
+    return pt
+
+
 def oracle_replica(pyoracle, cm, size, seed, stream, rates, config=None):
     o = pyoracle.Oracle(cm.to_blob(), size)
     o.init(seed, stream)

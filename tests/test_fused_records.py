@@ -18,7 +18,7 @@ import pytest
 from kmos_amd import _lib, workloads as W
 from kmos_amd.compiler import compile_model
 from kmos_amd.model import load_project
-from paritylib import pdopd_project, random_config
+from paritylib import four_species_project, pdopd_project, random_config
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 FORM_1, FORM_LI, FORM_M, FORM_4 = 1, 2, 3, 4
@@ -137,6 +137,9 @@ MODELS = [
     ("ab_ini_li", _golden("ab_model.ini"), "lat_int", FORM_LI), ("ruo2_li", W.ruo2_project, "lat_int", FORM_LI),
     ("grid_li", _golden("2d_grid.xml"), "lat_int", FORM_LI), ("pdopd", pdopd_project, "local_smart", FORM_M),
     ("pairwise_li", W.pairwise_project, "lat_int", FORM_LI),
+    # a byte per site on one layer
+    ("four", four_species_project, "local_smart", FORM_1), ("four_li", four_species_project, "lat_int", FORM_LI),
+    ("four_wide", lambda: four_species_project(True), "local_smart", FORM_4),
 ]
 
 

@@ -29,10 +29,11 @@ def _compare_msd(b, r, o, where):
     np.testing.assert_array_equal(g["events"], c["events"], err_msg=where)
 
 
+@pytest.mark.parametrize("overlap", [-1, 0], ids=["fused", "generic"])
 @pytest.mark.parametrize("with_adsorption,backend", [(False, "local_smart"), (True, "local_smart"),
                                                      (False, "lat_int"), (True, "lat_int")])
-def test_tracking_matches_oracle(engine, oracle, with_adsorption, backend):
-    print("case adsorption=%s %s" % (with_adsorption, backend), flush=True)
+def test_tracking_matches_oracle(engine, oracle, with_adsorption, backend, overlap):
+    print("case adsorption=%s %s overlap %d" % (with_adsorption, backend, overlap), flush=True)
     cm = compile_model(hop_project(with_adsorption), backend)
     hops, disp = displacement_table(cm)
     P = cm.nr_of_proc
@@ -49,6 +50,7 @@ def test_tracking_matches_oracle(engine, oracle, with_adsorption, backend):
     b.set_config(configs)
     b.msd_init(ion, hops, disp)
     b.msd_trajectory(2500)
+    b.set_overlap(overlap)
     orcs = []
     for r, s in enumerate(sizes):
         o = oracle_replica(oracle, cm, s, int(seeds[r]), 0, rates[r], configs[r])
@@ -60,6 +62,7 @@ def test_tracking_matches_oracle(engine, oracle, with_adsorption, backend):
     done = 0
     for chunk in (1, 999, 1500):
         b.run_displacement(chunk, traj_on=True)
+        assert (b.last_form() != 0) == (overlap != 0)
         for o in orcs:
             o.run_displacement(chunk, traj_on=True)
         done += chunk
@@ -135,9 +138,10 @@ def _compare_acf(b, r, o, where):
         assert g[k] == c[k], "%s %s: %s vs %s" % (where, k, g[k], c[k])
 
 
+@pytest.mark.parametrize("overlap", [-1, 0], ids=["fused", "generic"])
 @pytest.mark.parametrize("with_adsorption,backend", [(False, "local_smart"), (True, "local_smart"),
                                                      (True, "lat_int")])
-def test_acf_matches_oracle(engine, oracle, with_adsorption, backend):
+def test_acf_matches_oracle(engine, oracle, with_adsorption, backend, overlap):
     """Two property types, bins short enough for several wraps and steps
     that spill into the extended bins, ragged sizes in one batch."""
     print("case acf adsorption=%s %s" % (with_adsorption, backend), flush=True)
@@ -175,6 +179,7 @@ def test_acf_matches_oracle(engine, oracle, with_adsorption, backend):
         b.acf_set_properties(bad, 3.0 * pp)
     b.acf_init(ion, hops)
     b.msd_trajectory(3000)
+    b.set_overlap(overlap)
     orcs = []
     for r, s in enumerate(sizes):
         o = oracle_replica(oracle, cm, s, int(seeds[r]), 0, rates[r], configs[r])
@@ -188,6 +193,7 @@ def test_acf_matches_oracle(engine, oracle, with_adsorption, backend):
     done = 0
     for chunk in (1, 1999, 1000):
         b.run_acf(chunk, traj_on=True)
+        assert (b.last_form() != 0) == (overlap != 0)
         for o in orcs:
             o.run_acf(chunk, traj_on=True)
         done += chunk

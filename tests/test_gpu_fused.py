@@ -11,8 +11,8 @@ from kmos_amd import workloads as W
 from kmos_amd.acf import displacement_table
 from kmos_amd.compiler import compile_model
 from kmos_amd.model import load_project
-from paritylib import compare_state, oracle_replica, pdopd_project, random_config
-from test_fused_records import GOLDEN, Records
+from paritylib import compare_state, four_species_project, oracle_replica, pdopd_project, random_config
+from test_fused_records import FORM_M, GOLDEN, Records
 
 pytestmark = pytest.mark.gpu
 
@@ -24,20 +24,32 @@ CASES = [
     ("pdopd", pdopd_project, "local_smart"),        # several layers
     ("zgb_li", W.zgb_project, "lat_int"), ("ruo2_li", W.ruo2_project, "lat_int"),
     ("pairwise_li", W.pairwise_project, "lat_int"),
+    # a byte per site on one layer
+    ("four", four_species_project, "local_smart"), ("four_li", four_species_project, "lat_int"),
+    ("four_wide", lambda: four_species_project(True), "local_smart"),
 ]
+# each with the fused loop, with one lattice below its extents (where the
+# model runs on such a one) and with the generic loop asked for
+WAYS = [c + (way,) for c in CASES for way in ("fused", "below_the_extent", "generic")
+        if way != "below_the_extent" or c[0] != "pdopd"]
 
 
-@pytest.mark.parametrize("small", [False, True], ids=["fused", "below_the_extent"])
-@pytest.mark.parametrize("name,factory,backend", CASES, ids=[c[0] for c in CASES])
-def test_edges_match_oracle(engine, oracle, name, factory, backend, small):
+def least_extent(cm, R):
+    """The smallest lattice side the fused loop takes: no two offsets of the
+    records meet, and a row has more than one site."""
+    return max(2 * R.reach + 1, 1 if cm.spuck > 1 else 2)
+
+
+@pytest.mark.parametrize("name,factory,backend,way", WAYS, ids=["%s-%s" % (c[0], c[3]) for c in WAYS])
+def test_edges_match_oracle(engine, oracle, name, factory, backend, way):
     pt = factory()
     cm = compile_model(pt, backend)
     R = Records(cm)
     assert R.have
-    m = 2 * R.reach + 1
+    m = least_extent(cm, R)
     sizes = [(m, m), (m, m + 3), (m + 4, m), (31, 17), (64, 33)]
-    if small and R.reach > 1:
-        sizes.append((m - 1, m + 2))       # its offsets meet: the whole launch runs the generic loop
+    if way == "below_the_extent":
+        sizes.append((m - 1, m + 2))       # the whole launch runs the generic loop
     g = np.random.default_rng(17)
     n = len(sizes)
     rates = 10.0 ** g.uniform(-1, 3, (n, cm.nr_of_proc))
@@ -46,11 +58,14 @@ def test_edges_match_oracle(engine, oracle, name, factory, backend, small):
     b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
     b.init(seeds, np.arange(n, dtype=np.uint32))
     b.set_rates(rates)
+    if way == "generic":
+        b.set_overlap(0)
     configs = [random_config(pt, int(v), g) for v in b.volumes]
     b.set_config(configs)
     orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), i, rates[i], configs[i]) for i, s in enumerate(sizes)]
     for steps in (1, 2, 61, 1, 140, 795):
         b.run(steps)
+        assert b.last_form() == (R.form if way == "fused" else 0)
         for i, o in enumerate(orcs):
             o.run(steps)
             compare_state(b, i, o, where="%s %s" % (name, sizes[i]))
@@ -77,6 +92,7 @@ def test_layers_stop_where_the_oracle_stops(engine, oracle):
     orcs = [oracle_replica(oracle, cm, s, i, 0, rates[i], configs[i]) for i, s in enumerate(sizes)]
     for steps, limits in ((100, None), (400, 150 + 10 * np.arange(n)), (900, None)):
         left = b.run(steps, budget=limits)
+        assert b.last_form() == FORM_M
         for i, o in enumerate(orcs):
             before = o.kmc_step
             o.run(steps if limits is None else int(min(steps, limits[i])))
@@ -88,8 +104,9 @@ def test_layers_stop_where_the_oracle_stops(engine, oracle):
     b.close()
 
 
+@pytest.mark.parametrize("overlap", [-1, 0], ids=["fused", "generic"])
 @pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
-def test_moves_match_oracle(engine, oracle, backend):
+def test_moves_match_oracle(engine, oracle, backend, overlap):
     """Particle moves, written one step after their hop: launches that end
     on a hop, particles without a number (adsorbed after the start), a
     trajectory that fills up inside a launch, a stopped replica."""
@@ -113,6 +130,7 @@ def test_moves_match_oracle(engine, oracle, backend):
     b.set_config(configs)
     b.msd_init(ids["A"], hops, disp)
     b.msd_trajectory(300)
+    b.set_overlap(overlap)
     orcs = []
     for i, s in enumerate(sizes):
         o = oracle_replica(oracle, cm, s, int(seeds[i]), i, rates[i], configs[i])
@@ -121,6 +139,7 @@ def test_moves_match_oracle(engine, oracle, backend):
         orcs.append(o)
     for steps in (1, 2, 61, 1, 140, 395):
         b.run_displacement(steps, traj_on=True)
+        assert b.last_form() == (0 if overlap == 0 else R.form)
         for i, o in enumerate(orcs):
             o.run_displacement(steps, traj_on=True)
             got, want = b.msd_state(i), o.msd_state()

@@ -10,16 +10,19 @@ import pytest
 
 from kmos_amd import workloads as W
 from kmos_amd.compiler import compile_model
-from paritylib import compare_state, oracle_replica
+from paritylib import compare_state, oracle_replica, pdopd_project, random_config
+from test_fused_records import Records
 
 pytestmark = pytest.mark.gpu
 
 SIZES = [(6, 5), (20, 20), (9, 9), (13, 4)]
+# (extents the fused loop takes)
+WIDE = SIZES[:-1] + [(13, 6)]
 
 
-def _twin(engine, m, cm, rates, configs):
-    b = engine.Batch(m, [list(s) + [1] for s in SIZES])
-    b.init(np.arange(len(SIZES), dtype=np.uint32) + 41, np.zeros(len(SIZES), np.uint32))
+def _twin(engine, m, cm, rates, configs, sizes):
+    b = engine.Batch(m, [list(s) + [1] for s in sizes])
+    b.init(np.arange(len(sizes), dtype=np.uint32) + 41, np.zeros(len(sizes), np.uint32))
     b.set_rates(rates)
     b.set_config(configs)
     return b
@@ -35,25 +38,30 @@ def _same(a, b, where):
         np.testing.assert_array_equal(a.integ_rates(r), b.integ_rates(r), err_msg=where)
 
 
-def test_graph_replays_match_direct_launches(engine, oracle):
-    cm = compile_model(W.ruo2_project(), "local_smart")
+@pytest.mark.parametrize("factory,backend,sizes", [
+    (W.ruo2_project, "local_smart", SIZES), (W.ruo2_project, "local_smart", WIDE), (W.ruo2_project, "lat_int", WIDE),
+    # several layers: a run is two kernels
+    (pdopd_project, "local_smart", [(6, 5), (8, 8), (4, 3), (5, 4)]),
+], ids=["generic", "fused", "fused_li", "fused_layers"])
+def test_graph_replays_match_direct_launches(engine, oracle, factory, backend, sizes):
+    cm = compile_model(factory(), backend)
+    form = 0 if sizes is SIZES else Records(cm).form
     g = np.random.default_rng(3)
     P = cm.nr_of_proc
-    rates = 10.0 ** g.uniform(-2, 6, (len(SIZES), P))
-    ids = sorted(cm.project.species_ids().values())
+    rates = 10.0 ** g.uniform(-2, 6, (len(sizes), P))
     m = engine.Model(cm)
-    configs = [g.choice(ids, size=int(v)).astype(np.int8) for v in
-               (np.array([s[0] * s[1] for s in SIZES]) * cm.spuck)]
-    a = _twin(engine, m, cm, rates, configs)
-    b = _twin(engine, m, cm, rates, configs)
+    configs = [random_config(cm.project, s[0] * s[1] * cm.spuck, g) for s in sizes]
+    a = _twin(engine, m, cm, rates, configs, sizes)
+    b = _twin(engine, m, cm, rates, configs, sizes)
     b.set_graph(True)
-    o = oracle_replica(oracle, cm, SIZES[0], 41, 0, rates[0], configs[0])
-    allr = np.arange(len(SIZES), dtype=np.int32)
+    o = oracle_replica(oracle, cm, sizes[0], 41, 0, rates[0], configs[0])
+    allr = np.arange(len(sizes), dtype=np.int32)
     for it in range(6):
         print("case replay", it, flush=True)
-        bud = g.integers(50, 400, len(SIZES))
+        bud = g.integers(50, 400, len(sizes))
         ba = a.run(300, allr, bud)
         bb = b.run(300, allr, bud)
+        assert a.last_form() == b.last_form() == form
         np.testing.assert_array_equal(ba, bb)
         o.run(int(min(300, bud[0])))
         _same(a, b, "replay %d" % it)

@@ -13,16 +13,18 @@ from paritylib import compare_state, oracle_replica
 pytestmark = pytest.mark.gpu
 
 SIZES = [(6, 5), (20, 20), (9, 9), (20, 20), (6, 5), (13, 4)]
+# (extents the fused loop takes)
+WIDE = SIZES[:-1] + [(13, 6)]
 
 
-def _setup(engine, cm, rng_seed):
+def _setup(engine, cm, rng_seed, sizes=SIZES):
     g = np.random.default_rng(rng_seed)
     P = cm.nr_of_proc
-    rates = 10.0 ** g.uniform(-2, 6, (len(SIZES), P))
+    rates = 10.0 ** g.uniform(-2, 6, (len(sizes), P))
     m = engine.Model(cm)
-    b = engine.Batch(m, [list(s) + [1] for s in SIZES])
-    seeds = np.arange(len(SIZES), dtype=np.uint32) + 31
-    b.init(seeds, np.zeros(len(SIZES), np.uint32))
+    b = engine.Batch(m, [list(s) + [1] for s in sizes])
+    seeds = np.arange(len(sizes), dtype=np.uint32) + 31
+    b.init(seeds, np.zeros(len(sizes), np.uint32))
     b.set_rates(rates)
     ids = sorted(cm.project.species_ids().values())
     configs = [g.choice(ids, size=int(v)).astype(np.int8) for v in b.volumes]
@@ -30,15 +32,17 @@ def _setup(engine, cm, rng_seed):
     return b, rates, seeds, configs
 
 
+@pytest.mark.parametrize("forms,sizes", [((0, 1), SIZES), ((-1,), WIDE)], ids=["generic", "fused"])
 @pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
-def test_every_launch_shape_gives_the_same_trajectories(engine, oracle, backend):
+def test_every_launch_shape_gives_the_same_trajectories(engine, oracle, backend, forms, sizes):
     cm = compile_model(W.ruo2_project(), backend)
-    b, rates, seeds, configs = _setup(engine, cm, 5)
-    orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), 0, rates[i], configs[i]) for i, s in enumerate(SIZES)]
+    b, rates, seeds, configs = _setup(engine, cm, 5, sizes)
+    orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), 0, rates[i], configs[i]) for i, s in enumerate(sizes)]
     done = 0
-    # both step kernel forms (select after the replay, or overlapped with
-    # its reads) on every shape and order
-    for ov in (0, 1):
+    # both generic forms (select after the replay, or overlapped with its
+    # reads) or the fused loop (but where the lattice is kept in HBM) on
+    # every shape and order
+    for ov in forms:
         b.set_overlap(ov)
         for shape in autotune.SHAPES:
             for order in autotune.ORDERS:
@@ -46,6 +50,7 @@ def test_every_launch_shape_gives_the_same_trajectories(engine, oracle, backend)
                 b.set_launch(*shape)
                 ids = autotune.replica_order(b.volumes, order)
                 b.run(150, ids)
+                assert (b.last_form() != 0) == (ov == -1 and shape[0] != 0)
                 for o in orcs:
                     o.run(150)
                 done += 150

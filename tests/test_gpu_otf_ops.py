@@ -1,8 +1,8 @@
 """The otf step loop with one lane per list operation against the oracle at
 the edges of its rule: the smallest extents on which no two offsets of the
-operations meet (two cells either way), lists whose ends lie on and beside a
-checkpoint block of 16, and batches in which one smaller lattice sends every
-replica through the general loop."""
+operations meet, lists whose ends lie on and beside a checkpoint block of 16,
+and batches in which one smaller lattice sends every replica through the
+general loop."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("model", ["ruo2", "intzgb"])
 def test_otf_edges_match_oracle(otf_engine, otf_oracle, model, small):  # noqa: F811
     cm, base = _ruo2() if model == "ruo2" else _intzgb()
-    sizes = [(5, 5), (5, 8), (16, 1 + 4), (16, 16), (31, 11), (33, 16)] + ([(4, 6)] if small else [])
+    x, y = (2 * max(abs(op.off[d]) for ops in cm.otf_programs for op in ops) + 1 for d in range(2))
+    sizes = [(x, y), (x, y + 3), (16, y), (16, 16), (31, 11), (33, 16)] + ([(x - 1, y + 1)] if small else [])
     n, P = len(sizes), cm.nr_of_proc
     g = np.random.default_rng(41)
     rates = base[None, :] * 10.0 ** g.uniform(-0.5, 0.5, (n, P))
@@ -36,6 +37,7 @@ def test_otf_edges_match_oracle(otf_engine, otf_oracle, model, small):  # noqa: 
         orcs.append(o)
     for steps in (1, 62, 2, 700):
         b.run(steps)
+        assert b.last_form() == (0 if small else 1)
         for r, o in enumerate(orcs):
             o.run(steps)
             _compare(b, r, o, "%s %s" % (model, sizes[r]))

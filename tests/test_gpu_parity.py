@@ -11,7 +11,8 @@ import pytest
 
 from kmos_amd import workloads as W
 from kmos_amd.compiler import compile_model
-from paritylib import compare_clock, compare_state, oracle_replica, pdopd_project, random_config
+from paritylib import (compare_clock, compare_state, four_species_project, oracle_replica, pdopd_project,
+                       random_config)
 
 pytestmark = pytest.mark.gpu
 
@@ -281,10 +282,15 @@ def test_run_sampled_equals_run_then_sample(engine):
     assert list(rec_a["kmc_step"]) == [400, 250]
 
 
-@pytest.mark.parametrize("factory,backend", [(W.ruo2_project, "local_smart"), (W.pairwise_project, "lat_int")])
-def test_run_recorded_matches_oracle(engine, oracle, factory, backend):
+@pytest.mark.parametrize("overlap", [-1, 0], ids=["fused", "generic"])
+@pytest.mark.parametrize("factory,backend", [
+    (W.ruo2_project, "local_smart"), (W.pairwise_project, "lat_int"), (W.pairwise_project, "local_smart"),
+    (four_species_project, "local_smart"), (four_species_project, "lat_int"), (pdopd_project, "local_smart"),
+])
+def test_run_recorded_matches_oracle(engine, oracle, factory, backend, overlap):
     """Records written inside the step loop every 1000 steps equal the
-    oracle's state at those steps; the last record is the final state."""
+    oracle's state at those steps; the last record is the final state.
+    Several layers record in the generic loop, whatever is asked for."""
     pt = factory()
     cm = compile_model(pt, backend)
     rng = np.random.default_rng(21)
@@ -297,8 +303,10 @@ def test_run_recorded_matches_oracle(engine, oracle, factory, backend):
     configs = [_random_config(pt, int(v), rng) for v in b.volumes]
     b.set_config(configs)
     budgets = [2500, 1700, 0]
+    b.set_overlap(overlap)
     wait = b.run_recorded(2500, [0, 1, 2], budgets, 1000, 3)
     bud, recs = wait()
+    assert (b.last_form() != 0) == (overlap != 0 and factory is not pdopd_project)
     np.testing.assert_array_equal(bud, [0, 0, 0])
     for r, s in enumerate(sizes):
         o = oracle_replica(oracle, cm, s, r + 2, 0, rates[r], configs[r])

@@ -1,7 +1,8 @@
 """kmcg_set_config (the database rebuilt list by list) against the oracle's
 touchups one after the other: lists left by earlier steps and an earlier
-configuration, every backend, one and several layers, lattices whose lists
-fit LDS and one whose lists do not, a replica that has stopped."""
+configuration, every backend, one and several layers, two and three
+dimensions, lattices whose lists fit LDS (up to 127 KiB of it) and lattices
+whose lists do not."""
 import os
 
 import numpy as np
@@ -9,14 +10,31 @@ import pytest
 
 from kmos_amd import workloads as W
 from kmos_amd.compiler import compile_model
-from kmos_amd.model import load_project
+from kmos_amd.model import Process, load_project
 from paritylib import GOLDEN, compare_state, oracle_replica, pdopd_project, random_config
 
 pytestmark = pytest.mark.gpu
 
 SMALL = [(8, 8), (9, 13), (16, 17), (31, 11)]
+
+
+def zgb_3d():
+    pt = W.zgb_project()
+    pt.model_dimension = 3
+    s = lambda sp, off=(0, 0, 0): W._c(sp, "site", off, "sc")  # noqa: E731
+    pt.processes.append(Process("O2_adsorption3", "1.", [s("empty"), s("empty", (0, 0, 1))],
+                                [s("O"), s("O", (0, 0, 1))]))
+    pt.validate()
+    return pt
+
+
 CASES = [
     ("quickstart", W.quickstart_project, "local_smart", [(1, 1), (5, 3), (215, 211)]),
+    # lists of 64 KiB and more in LDS
+    ("quickstart_lds", W.quickstart_project, "local_smart", [(127, 128), (128, 128), (129, 128), (180, 180)]),
+    ("ruo2_lds", W.ruo2_project, "local_smart", [(128, 128)]),
+    ("zgb_3d", zgb_3d, "local_smart", [(5, 6, 7), (8, 5, 5)]),
+    ("zgb_3d_li", zgb_3d, "lat_int", [(5, 6, 7), (8, 5, 5)]),
     ("zgb", W.zgb_project, "local_smart", SMALL), ("zgb_li", W.zgb_project, "lat_int", SMALL),
     ("ruo2", W.ruo2_project, "local_smart", SMALL), ("ruo2_li", W.ruo2_project, "lat_int", SMALL),
     ("pairwise", W.pairwise_project, "local_smart", SMALL), ("pairwise_li", W.pairwise_project, "lat_int", SMALL),
@@ -33,7 +51,7 @@ def test_set_config_matches_oracle(engine, oracle, name, factory, backend, sizes
     n = len(sizes)
     rates = 10.0 ** g.uniform(-1, 3, (n, cm.nr_of_proc))
     seeds = g.integers(1 << 31, size=n).astype(np.uint32)
-    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b = engine.Batch(engine.Model(cm), [(s + (1,))[:3] for s in sizes])
     b.init(seeds, np.zeros(n, np.uint32))
     b.set_rates(rates)
     orcs = [oracle_replica(oracle, cm, s, int(seeds[i]), 0, rates[i]) for i, s in enumerate(sizes)]
