@@ -3789,12 +3789,17 @@ int kmcg_batch_footprint(const kmcg_model *m, int32_t n, const int32_t *sizes, i
     if (rc)
         return rc;
     const int bits = m->lattice_bits();
-    long long tot = 0;
+    // once: the op program, the fused records, the lists' leading words,
+    // the misc kernel's outputs
+    long long tot = 4LL * (((m->prog.size() + 3) & ~(size_t)3) + m->fz.size() + 64 + 16);
     for (int i = 0; i < n; ++i) {
         long long X = sizes[3 * i], Y = m->dim >= 2 ? sizes[3 * i + 1] : 1, Z = m->dim >= 3 ? sizes[3 * i + 2] : 1;
         long long V = X * Y * Z * m->spuck;
-        tot += lattice_bytes((int)V, bits) + 2LL * m->P * (V + 1) * 4;
-        tot += (long long)m->P * (4 + 8 + 8 + 8) + 64;
+        tot += lattice_bytes((int)V, bits) + (((2LL * m->P * (V + 1)) + 63) & ~63LL) * 4;
+        // per process: list size, rate, integ, procstat; species counts; per
+        // replica: dims, two offsets, two keys, ktime to budget, status to
+        // the two replica lists
+        tot += (long long)m->P * (4 + 8 + 8 + 8) + 8LL * m->S * m->spuck + 16 + 2 * 8 + 2 * 4 + 6 * 8 + 4 * 4;
     }
     *bytes = tot;
     return KMCG_OK;

@@ -57,6 +57,13 @@ def test_model_load_on_host(factory, backend):
     assert _lib.load().kmcg_batch_footprint(h, 2, sizes.ctypes.data_as(ctypes.c_void_p), ctypes.byref(fp)) == 0
     V = 20 * 20 * cm.spuck + 64 * 64 * cm.spuck
     assert fp.value >= 2 * cm.nr_of_proc * V * 4
+    # what a batch allocates beside the lists: the lattices, per process and
+    # replica 28 bytes, the program and the records of the fused loop
+    fz = np.zeros(6, np.int32)
+    assert _lib.load().kmcg_model_fused(h, fz.ctypes.data_as(ctypes.c_void_p), None) == 0
+    values = cm.nr_of_species + (cm.null_species >= 0)
+    lattices = V // 4 if values <= 3 else V
+    assert fp.value >= 8 * cm.nr_of_proc * (V + 2) + lattices + 2 * 28 * cm.nr_of_proc + 4 * int(fz[0])
     _lib.load().kmcg_model_free(h)
 
 
