@@ -65,7 +65,7 @@ def host_cores():
     return avail, min(avail, CORE_CAP)
 
 
-def profile_figure(workload, kind, key, kernel="kmc_steps_kernel"):
+def profile_figure(workload, kind, key, kernel="kmc_steps_kernel_fz"):
     """A per-kMC-step figure ('traffic' or 'lds' summary) from the rocprofv3
     counter summary committed for this workload and kernel, or None."""
     path = os.path.join(REPO, "profiles", "%s_%s_%s.md" % (kernel, workload, kind))
@@ -77,7 +77,7 @@ def profile_figure(workload, kind, key, kernel="kmc_steps_kernel"):
     return None
 
 
-def roofline(workload, bytes_per_step, steps_per_launch, avg_launch_s, kernel="kmc_steps_kernel"):
+def roofline(workload, bytes_per_step, steps_per_launch, avg_launch_s, kernel="kmc_steps_kernel_fz"):
     """HBM roofline of the step kernel: algorithmic bytes per launch over the
     mean launch time; the measured HBM traffic and the LDS bandwidth from
     the profiles' bytes per kMC step, scaled to this run's launches."""
@@ -310,13 +310,14 @@ def batched_leg(engine, wl, K, warmup, tune, cpu, spot=(0,)):
     b, wall, executed, kernel_ms, chunk, choice = run_batched(engine, model, wl, K, warmup, tune)
     _, k_after, st = b.scalars_all()
     ok = spot_check(b, wl, cm, k_after, spot)
+    kernel = model.step_kernel if b.last_form() else model.generic_kernel
     b.close()
     avg_s = float(np.mean(kernel_ms)) / 1e3
     out = {"workload": wl.name, "replicas": wl.n, "steps_per_replica": wl.steps,
            "gpu_steps_per_s": executed / wall, "wall_s": wall, "avg_launch_ms": avg_s * 1e3,
            "launch": launch_summary(choice), "parity_spot_check": ok,
            "replica_status_counts": {str(k): int(v) for k, v in zip(*np.unique(st, return_counts=True))},
-           "roofline": roofline(wl.name, algorithmic_bytes_per_step(wl), executed / K, avg_s, model.step_kernel)}
+           "roofline": roofline(wl.name, algorithmic_bytes_per_step(wl), executed / K, avg_s, kernel)}
     if cpu:
         out["cpu_baseline"] = oracle_cpu_baseline(wl, 10.0)
         out["gpu_over_cpu"] = out["gpu_steps_per_s"] / out["cpu_baseline"]["value"]
@@ -633,7 +634,8 @@ def otf_leg(K, warmup, cpu, wl=None):
     bps, work = otf_algorithmic_bytes(wl, blob)
     avg_s = float(np.mean(kernel_ms)) / 1e3
     steps_per_launch = chunk * wl.n
-    rl = roofline(wl.name, bps, steps_per_launch, avg_s, kernel="otf_steps_kernel")
+    rl = roofline(wl.name, bps, steps_per_launch, avg_s,
+                  kernel="otf_fast_kernel" if b.last_form() else "otf_steps_kernel")
     out = {"workload": wl.name, "replicas": int(wl.n), "steps_per_replica": int((K + warmup) * chunk),
            "gpu_steps_per_s": executed / wall, "kmc_steps_per_launch": steps_per_launch,
            "avg_launch_ms": avg_s * 1e3, "replica_status_counts": {k: status.count(k) for k in set(status)},

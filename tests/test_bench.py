@@ -16,9 +16,9 @@ REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, REPO)
 import bench  # noqa: E402
 
-# workload -> the step kernel the library launches for it (kmcg_model_forms)
-WORKLOADS = {"zgb_128x128_x4096": "kmc_steps_kernel", "ruo2_local_smart_mix_x2048": "kmc_steps_kernel",
-             "pairwise_lat_int_256x256_x512": "kmc_steps_kernel_li"}
+# workload -> the step kernel the library launches for it (kmcg_model_fused)
+WORKLOADS = {"zgb_128x128_x4096": "kmc_steps_kernel_fz", "ruo2_local_smart_mix_x2048": "kmc_steps_kernel_fz",
+             "pairwise_lat_int_256x256_x512": "kmc_steps_kernel_fz"}
 
 
 def test_more_than_one_gpu_is_refused():
@@ -69,7 +69,7 @@ def test_zgb_algorithmic_bytes_match_the_profile():
     wl = W.zgb()
     wl.project_blob = compile_model(wl.project, wl.backend).to_blob()
     bps = bench.algorithmic_bytes_per_step(wl)
-    text = open(os.path.join(REPO, "profiles", "kmc_steps_kernel_zgb_128x128_x4096_pmc.md")).read()
+    text = open(os.path.join(REPO, "profiles", "kmc_steps_kernel_fz_zgb_128x128_x4096_pmc.md")).read()
     assert "| %.1f |" % bps in text
 
 
@@ -85,7 +85,8 @@ def test_oracle_cpu_baseline_states_its_cores():
 
 def test_profiles_name_the_kernel_the_library_launches():
     """The kernel each workload's profiles are filed under is the form the
-    library reports for its model (kmcg_model_forms)."""
+    library reports for its model (kmcg_model_fused), and the one their first
+    lines name."""
     from kmos_amd import engine
     from kmos_amd import workloads as W
     from kmos_amd.compiler import compile_model
@@ -93,3 +94,6 @@ def test_profiles_name_the_kernel_the_library_launches():
                     ("pairwise_lat_int_256x256_x512", W.pairwise(n=2))):
         assert wl.name.rsplit("_x", 1)[0] == key.rsplit("_x", 1)[0]
         assert engine.Model(compile_model(wl.project, wl.backend)).step_kernel == WORKLOADS[key]
+        for kind in ("", "_pmc", "_lds", "_sq", "_phases"):
+            text = open(os.path.join(REPO, "profiles", "%s_%s%s.md" % (WORKLOADS[key], key, kind))).read()
+            assert "The kernel is `%s<" % WORKLOADS[key] in text
