@@ -2028,13 +2028,14 @@ __global__ __launch_bounds__(256) void kmc_init_lists_kernel(KParams kp)
 // order on the list.  With INLDS the list and its inverse index sit in LDS
 // (two bytes each per cell): an entry costs two LDS round trips instead of
 // three HBM ones; without (lattices beyond LDS) they stay in HBM.  It
-// replaces one touchup after the other on one wave, 3 us each: 24.9 -> 0.74 ms with its
-// getters for one 64x64 RuO2 lattice (8192 sites, 36 processes).
+// replaces one touchup after the other on one wave, 3 us each: 24.9 -> 0.58
+// ms with its getters for one 64x64 RuO2 lattice (8192 sites, 36 processes),
+// 304 -> 33 ms for 4096 ZGB lattices of 128x128.
 template <int BITS, bool INLDS>
 __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
 {
     extern __shared__ __align__(16) unsigned short adj[];
-    __shared__ int wave_tot[4], ev[256], count;
+    __shared__ int wave_tot[4], ev[256], count, bad;
     const int P = kp.P;
     const int p = blockIdx.x % P;
     const int r = kp.rep_ids[blockIdx.x / P];
@@ -2070,22 +2071,36 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
         return;
     }
     if (threadIdx.x == 0)
-        count = 0;
+        count = bad = 0;
     __syncthreads();
-    // in LDS: list[1..ncell] of cells, then the slot of every cell.  Every
-    // entry that will be followed is a site of this process.
+    // in LDS: list[1..ncell] of cells, then the slot of every cell.  That the
+    // two are each other's inverse is seen here, side by side, so that the
+    // one lane below follows them without a look at their bounds (with such
+    // looks 0.80 ms for RuO2 64x64 and its getters, so 0.58).
     unsigned short *list = adj, *slot = adj + ncell + 1;
-    if (INLDS)
-        for (int c = threadIdx.x; c < ncell; c += 256)
-            slot[c] = (unsigned short)bp[kp.spuck * c + n_exec];
+    int listed = 0;
+    for (int c = threadIdx.x; c < ncell; c += 256) {
+        const int k = bp[kp.spuck * c + n_exec];
+        listed += k != 0 ? 1 : 0;
+        if (INLDS)
+            slot[c] = (unsigned short)k;
+    }
+    if (listed)
+        atomicAdd(&count, listed);
+    __syncthreads();
     for (int k = threadIdx.x + 1; k <= n; k += 256) {
         const int at = sp[k] - n_exec, c = at / kp.spuck;
-        if (at < 0 || c >= ncell || at != c * kp.spuck)
-            count = -1;
-        if (INLDS)
+        if (at < 0 || c >= ncell || at != c * kp.spuck || (INLDS ? (int)slot[c] : bp[at + n_exec]) != k)
+            bad = 1;
+        else if (INLDS)
             list[k] = (unsigned short)c;
     }
     __syncthreads();
+    if (bad || count != n) {
+        if (threadIdx.x == 0)
+            kp.lists_ok[r] = LISTS_CORRUPT;
+        return;
+    }
     for (int t = 0; t < ncell; t += 256) {
         const int i = t + threadIdx.x;
         bool en = false, reg = false;
@@ -2116,20 +2131,13 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
         if (en || reg)
             ev[at] = c << 2 | (reg ? 2 : 0) | (en ? 1 : 0);
         __syncthreads();
-        if (threadIdx.x == 0 && count == 0) {
+        if (threadIdx.x == 0) {
             const int m = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
             for (int j = 0; j < m; ++j) {
                 const int e = ev[j], cell = e >> 2;
-                const int at0 = e & 2 ? (INLDS ? (int)slot[cell] : bp[kp.spuck * cell + n_exec]) : 1;
-                // an inverse index that points outside the list, or an
-                // addition to a full one
-                if (at0 < 1 || ((e & 2) && at0 > n) || (e == (cell << 2 | 1) && n >= ncell)) {
-                    count = -1;
-                    break;
-                }
                 if (INLDS) {
                     if (e & 2) {
-                        const int at2 = at0, last = list[n];
+                        const int at2 = slot[cell], last = list[n];
                         list[at2] = (unsigned short)last;
                         slot[last] = (unsigned short)at2;
                         n -= 1;
@@ -2142,7 +2150,7 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
                 } else {
                     const int site = kp.spuck * cell + n_exec;
                     if (e & 2) {
-                        const int at2 = at0, last = sp[n];
+                        const int at2 = bp[site], last = sp[n];
                         sp[at2] = last;
                         bp[last] = at2;
                         n -= 1;
@@ -2156,11 +2164,6 @@ __global__ __launch_bounds__(256) void kmc_adjust_lists_kernel(KParams kp)
             }
         }
         __syncthreads();
-    }
-    if (count < 0) {
-        if (threadIdx.x == 0)
-            kp.lists_ok[r] = LISTS_CORRUPT;
-        return;
     }
     if (threadIdx.x == 0)
         kp.nr[(long long)r * P + p] = n;
