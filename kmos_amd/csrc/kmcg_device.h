@@ -109,7 +109,7 @@ struct KParams {
     unsigned long long *rngctr;
     int *status;
     int *lists_ok;                 // per replica: lists match the lattice
-    int *out_ok;                   // misc kernel: the same for each replica of the launch, pinned
+    int *out_ok;                   // misc kernel: the host's word for each replica of the launch, pinned
     long long *executed;
     long long *budget;             // optional, per launch slot
     int *out;                      // misc kernel outputs

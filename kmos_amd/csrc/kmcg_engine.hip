@@ -1761,6 +1761,10 @@ __global__ __launch_bounds__(64 * MAX_WPG) __attribute__((amdgpu_waves_per_eu(4)
 
 #include "kmcg_fused.hip"
 
+// what the host keeps of a replica: bit 0 its lists follow its lattice, bit 1
+// it is stopped
+__device__ __forceinline__ int lists_host(int ok, int st) { return (ok ? 1 : 0) | (st != ST_OK ? 2 : 0); }
+
 // touchups, run_proc_nr, get_next_kmc_step (one replica per wave)
 template <int PPL, int BITS, bool LDS_LAT>
 __global__ __launch_bounds__(64 * MAX_WPG) void kmc_misc_kernel(KParams kp)
@@ -1850,7 +1854,7 @@ __global__ __launch_bounds__(64 * MAX_WPG) void kmc_misc_kernel(KParams kp)
         if (kp.mode != MODE_NEXT_STEP)
             ok = st == ST_OK && (ok || kp.mode == MODE_INIT || kp.mode == MODE_ADJUST);
         kp.lists_ok[r] = ok;
-        kp.out_ok[blockIdx.x * kp.wpg + (threadIdx.x >> 6)] = ok;
+        kp.out_ok[blockIdx.x * kp.wpg + (threadIdx.x >> 6)] = lists_host(ok, st);
     }
 }
 
@@ -1867,7 +1871,8 @@ __global__ void kmc_mark_lists_kernel(KParams kp, int r0, int n, int *out)
     const int r = r0 + i;
     if (kp.lists_ok[r] == LISTS_CORRUPT)
         kp.status[r] = ST_CORRUPT;
-    kp.lists_ok[r] = out[i] = kp.status[r] == ST_OK;
+    kp.lists_ok[r] = kp.status[r] == ST_OK;
+    out[i] = lists_host(kp.lists_ok[r], kp.status[r]);
 }
 
 // default species of every site (initialize_state); site defaults are the
@@ -2460,8 +2465,9 @@ struct kmcg_batch {
     // kmcg_set_config where the replica is not stopped, cleared by
     // kmcg_replace_species, kmcg_set_state and every stop on an error)
     int *lists_ok = nullptr;
-    // the same on the host (a stop inside a run is taken over by the call
-    // that lets the replica go on: until then it takes no step)
+    // The same on the host in bit 0 (a stop inside a run is taken over by the
+    // call that lets the replica go on: until then it takes no step).  Bit 1:
+    // the replica is stopped, so that its lists matter to no run.
     std::vector<unsigned char> lists_ok_h;
     // 1 per replica whose lists hold each site once, and sites of the
     // process's own type only, whatever the lattice says.  Steps on lists
@@ -3488,10 +3494,10 @@ Shape launch_shape(kmcg_batch *b, const int *ids, int n, KParams &kp, int max_wp
     size_t shared = prog;
     // the fused step loop, faster than the others at every size measured
     // (1.6 to 3.3 times, one replica of 20x20 to 4096 of 128x128), wherever
-    // it is sound: the lists of every replica follow its lattice, no two
-    // offsets of the records meet (extents of 2 * reach + 1 and more), the
-    // lattice fits LDS, and no other form was asked for.  One replica it
-    // cannot take sends the whole launch to the generic loops.
+    // it is sound: the lists of every replica that is not stopped follow its
+    // lattice, no two offsets of the records meet (extents of 2 * reach + 1
+    // and more), the lattice fits LDS, and no other form was asked for.  One
+    // replica it cannot take sends the whole launch to the generic loops.
     const size_t fz_wave = (size_t)maxlb + (64 * WIN + occ) * sizeof(int);
     s.fz = steps && !b->m->fz.empty() && (steps == 1 || b->m->fz_form != FZ_M) && b->ov_mode == -1 && b->lds_mode != 0 &&
            (size_t)b->m->fz_tab_bytes + fz_wave <= (size_t)b->max_lds;
@@ -4034,7 +4040,8 @@ namespace {
 int clear_lists_ok(kmcg_batch *b, int r0, int n)
 {
     HIPCHK(hipSetDevice(b->device));
-    std::fill(b->lists_ok_h.begin() + r0, b->lists_ok_h.begin() + r0 + n, (unsigned char)0);
+    for (int r = r0; r < r0 + n; ++r)
+        b->lists_ok_h[r] &= 2;
     HIPCHK(hipMemsetD32Async((hipDeviceptr_t)(b->lists_ok + r0), 0, n, b->stream));
     return settle(b);
 }
@@ -4231,7 +4238,8 @@ static int run_impl(kmcg_batch *b, const int32_t *replicas, int32_t n, int64_t s
     if (rc)
         return rc;
     for (int i = 0; i < n; ++i)
-        b->lists_whole_h[replicas[i]] &= b->lists_ok_h[replicas[i]];
+        if (!b->lists_ok_h[replicas[i]])
+            b->lists_whole_h[replicas[i]] = 0;
     const int first = contiguous(replicas, n);           // no list to send then
     if (first < 0)
         memcpy(b->h_ids, replicas, n * sizeof(int));
@@ -4500,7 +4508,7 @@ int kmcg_run_proc_nr(kmcg_batch *b, int32_t r, int32_t proc, int32_t site)
         return rc;
     if (proc < 1 || proc > b->m->P || site < 1 || site > b->V[r])
         return fail(KMCG_EINVAL, "process or site out of range");
-    b->lists_whole_h[r] &= b->lists_ok_h[r];
+    b->lists_whole_h[r] &= b->lists_ok_h[r] & 1;
     return run_misc(b, {r}, MODE_RUN_PROC, proc, site, 0, 0);
 }
 
@@ -5152,7 +5160,7 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
                                                : std::vector<double>(P, 0.0);
     const int running = 0;
     // (a restored state is not checked against its lattice)
-    b->lists_whole_h[r] = 0;
+    b->lists_whole_h[r] = b->lists_ok_h[r] = 0;
     if ((rc = clear_lists_ok(b, r, 1)) ||
         (rc = copy_in(b, b->lat_pool + b->lat_off[r], packed.data(), packed.size())) ||
         (rc = copy_in(b, b->avail_pool + b->avail_off[r], blk.data(), blk.size())) ||

@@ -1,7 +1,5 @@
-"""A stopped replica keeps its lists when set_config replaces its lattice.
-touchup and run_proc_nr let it go on; the lists then name processes whose
-conditions do not hold, and the run has to stop at the first of them whose
-write finds another species, as the oracle does, and must not write there.
+"""Lists that do not follow the lattice: a run has to stop where it finds
+that, as the oracle does, and must not write there.
 
 local_smart: in the oracle's state.  lat_int: at the oracle's step with a
 stop status (the deletion of an entry that is not registered is undefined in
@@ -12,6 +10,7 @@ import pytest
 from kmos_amd import workloads as W
 from kmos_amd.compiler import compile_model
 from paritylib import compare_state, oracle_replica
+from test_fused_records import Records
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("way", ["touchup", "run_proc_nr"])
 @pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
 def test_new_lattice_of_a_stopped_replica(engine, oracle, backend, way):
+    """A stopped replica keeps its lists when set_config replaces its lattice;
+    touchup and run_proc_nr let it go on."""
     pt = W.zgb_project()
     cm = compile_model(pt, backend)
     sid = pt.species_ids()
@@ -149,4 +150,44 @@ def test_restored_entries_of_another_site_type(engine, oracle):
     b.run(200)
     o.run(200)
     compare_state(b, 0, o, where="after the run")
+    b.close()
+
+
+@pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
+def test_stopped_replica_among_others(engine, oracle, backend):
+    """A stopped replica takes no step, so its lists keep no other replica
+    from the fused loop; let go on by a touchup, they do."""
+    pt = W.zgb_project()
+    cm = compile_model(pt, backend)
+    form = Records(cm).form
+    g = np.random.default_rng(12)
+    sizes = [(9, 8), (12, 10), (7, 11)]
+    rates = 10.0 ** g.uniform(-1, 1, (3, cm.nr_of_proc))
+    b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
+    b.init([5, 6, 7])
+    b.set_rates(rates)
+    b.set_rates(0.0 * rates[:1], r0=1)
+    b.run(20)
+    orcs = [oracle_replica(oracle, cm, s, 5 + r, 0, rates[r]) for r, s in enumerate(sizes)]
+    orcs[1].set_rates(0.0 * rates[1])
+    configs = [g.integers(0, cm.nr_of_species, int(v)).astype(np.int8) for v in b.volumes]
+    b.set_config(configs)
+    b.set_rates(rates)
+    b.run(100)
+    assert b.last_form() == form
+    for r, o in enumerate(orcs):
+        o.run(20)
+        if r != 1:
+            o.set_config(configs[r])
+            o.run(100)
+            compare_state(b, r, o, where="replica %d" % r)
+    assert b.scalars(1)[4] == 1 and b.scalars(1)[2] == 0
+    np.testing.assert_array_equal(b.lattice(1), configs[1])
+    b.touchup(1, 0, 0, 0, 1)
+    assert b.scalars(1)[4] == 0
+    b.run(1)
+    assert b.last_form() == 0
+    b.set_config(configs[:1])
+    b.run(1, [0, 2])
+    assert b.last_form() == form
     b.close()
