@@ -2315,8 +2315,7 @@ __global__ __launch_bounds__(256) void kmc_sample_kernel(KParams kp, double *out
 
 // The scalars of one replica into pinned host memory (kmcg_get_scalars): one
 // launch and one wait where a copy each cost five.  With `nr` its list sizes
-// as well (kmcg_get_avail: 39 us for a 20x20 lattice, 48 with a copy of their
-// own, 27 without them).
+// as well (kmcg_get_avail).
 __global__ void kmc_scalars_kernel(KParams kp, int r, double *out, int *nr)
 {
     long long *o = (long long *)out;
@@ -4509,7 +4508,10 @@ int kmcg_run_proc_nr(kmcg_batch *b, int32_t r, int32_t proc, int32_t site)
     if (proc < 1 || proc > b->m->P || site < 1 || site > b->V[r])
         return fail(KMCG_EINVAL, "process or site out of range");
     b->lists_whole_h[r] &= b->lists_ok_h[r] & 1;
-    return run_misc(b, {r}, MODE_RUN_PROC, proc, site, 0, 0);
+    const int rc2 = run_misc(b, {r}, MODE_RUN_PROC, proc, site, 0, 0);
+    if (b->lists_ok_h[r] & 2)                    // it stopped halfway
+        b->lists_whole_h[r] = 0;
+    return rc2;
 }
 
 int kmcg_touchup(kmcg_batch *b, int32_t r, int32_t x, int32_t y, int32_t z, int32_t n)
@@ -4683,19 +4685,35 @@ int kmcg_get_avail(kmcg_batch *b, int32_t r, int32_t *sites, int32_t *back)
     std::vector<int> blk(2 * P * V1);
     if ((rc = settle(b)))
         return rc;
-    // (the staging of sample records: at least two words per process)
-    int *nr = (int *)b->h_samples;
-    hipLaunchKernelGGL(kmc_scalars_kernel, dim3(1), dim3(64), 0, b->stream, make_params(b), r,
-                       b->h_samples + b->samples_len, nr);
-    HIPCHK(hipGetLastError());
+    // Slots past a list's end read 0; on the device they keep what they
+    // held.  Of a whole list the end is where the inverse index stops naming
+    // the slots; of others it comes from the device (20x20 lattice: 38 us a
+    // call, 27 with the search).
+    int *nr = nullptr;
+    if (!b->lists_whole_h[r]) {
+        nr = (int *)b->h_samples;                // (at least two words per process)
+        hipLaunchKernelGGL(kmc_scalars_kernel, dim3(1), dim3(64), 0, b->stream, make_params(b), r,
+                           b->h_samples + b->samples_len, nr);
+        HIPCHK(hipGetLastError());
+    }
     if ((rc = copy_out(b, blk.data(), b->avail_pool + b->avail_off[r], blk.size())))
         return rc;
     for (long long p = 0; p < P; ++p) {
-        // slots past the end read 0; on the device they keep what they held
-        const long long used = std::min<long long>(std::max(nr[p], 0), V1 - 1);
-        std::memcpy(sites + p * (V1 - 1), blk.data() + p * V1 + 1, used * sizeof(int));
+        const int *sp = blk.data() + p * V1, *bp = blk.data() + (P + p) * V1;
+        long long used = 0;
+        if (nr) {
+            used = std::min<long long>(std::max(nr[p], 0), V1 - 1);
+        } else {
+            long long past = V1;                 // slots 1..used are named, `past` is not
+            while (past - used > 1) {
+                const long long k = (used + past) / 2;
+                const bool named = sp[k] >= 1 && sp[k] < V1 && bp[sp[k]] == k;
+                (named ? used : past) = k;
+            }
+        }
+        std::memcpy(sites + p * (V1 - 1), sp + 1, used * sizeof(int));
         std::memset(sites + p * (V1 - 1) + used, 0, (V1 - 1 - used) * sizeof(int));
-        std::memcpy(back + p * (V1 - 1), blk.data() + (P + p) * V1 + 1, (V1 - 1) * sizeof(int));
+        std::memcpy(back + p * (V1 - 1), bp + 1, (V1 - 1) * sizeof(int));
     }
     return KMCG_OK;
 }
