@@ -75,9 +75,9 @@ int kmcg_model_forms(const kmcg_model *m, int32_t *li);
 /* The fused step loop's records (per process the list updates of its
  * routines as one flat list; layout in kmos_amd/csrc/kmcg_fused.hip): info6
  * = words in all (0: the model has none), form (1 one open condition, 4
- * four, 3 several layers, 2 lat_int), chunks of 64 records per process, largest offset, word
- * offset and bytes of the lat_int tables; `words` may be NULL.  No
- * counterpart in the reference (a test aid). */
+ * four, 3 several layers, 2 lat_int), chunks of 64 records per process,
+ * largest offset, word offset and bytes of the lat_int tables; `words` may be
+ * NULL.  No counterpart in the reference (a test aid). */
 int kmcg_model_fused(const kmcg_model *m, int32_t *info6, int32_t *words);
 
 /* Device bytes a batch of n replicas of sizes[n][3] needs. */
@@ -108,7 +108,10 @@ int kmcg_get_rates(kmcg_batch *b, int32_t r, double *rates);
  * [r0, r0+n): species per site (config holds the n lattices one after the
  * other, each V values in site order), then touchups with x outermost
  * (kmos/run/__init__.py:1408-1457).  A configuration holding an unknown
- * species fails the call before any lattice is replaced. */
+ * species fails the call before any lattice is replaced.  A replica whose
+ * status is not KMCG_REPLICA_OK takes the species only: it is not touched
+ * up, and a run after kmcg_touchup or kmcg_run_proc_nr has let it go on stops
+ * where its lists and its lattice disagree. */
 int kmcg_set_config(kmcg_batch *b, int32_t r0, int32_t n, const int8_t *config);
 
 /* proclist.do_kmc_steps(steps) for the listed replicas
@@ -271,7 +274,8 @@ int kmcg_set_state(kmcg_batch *b, int32_t r, const double *time2, const int64_t 
  * list invariant add_proc/del_proc keep (base.mpy:211-301) and the
  * (process, site) pairs whose registration disagrees with the process's
  * conditions on the current lattice (the set the reference's touchups
- * build, kmos/io/__init__.py:2411-2443; lat_int: the nli case trees).  0
+ * build, kmos/io/__init__.py:2411-2443; lat_int: the nli case trees).  What
+ * the device holds in slots past a list's end is not looked at.  0
  * everywhere for a consistent state.  Synchronous. */
 int kmcg_check_lists(kmcg_batch *b, int32_t r0, int32_t n, int32_t *bad);
 /* proclist.get_occupation for replicas [r0, r0+n): out[n][S][spuck] */

@@ -740,8 +740,9 @@ __global__ __launch_bounds__(64) void otf_steps_kernel(OtfParams p)
     }
 }
 
-// The step loop with one lane per list operation (models and lattices
-// otf_fast_ok names; the others run otf_steps_kernel).
+// The step loop with one lane per list operation (for the models that
+// otf_build_fast takes and the lattices that otf_launch finds large enough;
+// the others run otf_steps_kernel).
 //
 // A step of the intZGB model has 13 to 23 deletes, 40 to 62 rate updates and
 // 5 to 13 adds on ten lists.  An owner lane that walks its own ones waits for

@@ -16,6 +16,16 @@ from test_fused_records import FORM_M, GOLDEN, Records
 
 pytestmark = pytest.mark.gpu
 
+
+
+def one_dimension(pt):
+    """The processes of a model that lie in a row."""
+    pt.model_dimension = 1
+    pt.processes = [p for p in pt.processes if not any(c.coord.offset[1] for c in p.conditions + p.actions)]
+    pt.validate()
+    return pt
+
+
 CASES = [
     # one chunk of one-condition records, several chunks of wide ones, lat_int
     ("quickstart", W.quickstart_project, "local_smart"), ("zgb", W.zgb_project, "local_smart"),
@@ -27,6 +37,8 @@ CASES = [
     # a byte per site on one layer
     ("four", four_species_project, "local_smart"), ("four_li", four_species_project, "lat_int"),
     ("four_wide", lambda: four_species_project(True), "local_smart"),
+    ("one_dimension", lambda: one_dimension(W.zgb_project()), "local_smart"),
+    ("one_dimension_li", lambda: one_dimension(W.zgb_project()), "lat_int"),
 ]
 # each with the fused loop, with one lattice below its extents (where the
 # model runs on such a one) and with the generic loop asked for
@@ -106,11 +118,13 @@ def test_layers_stop_where_the_oracle_stops(engine, oracle):
 
 @pytest.mark.parametrize("overlap", [-1, 0], ids=["fused", "generic"])
 @pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
-def test_moves_match_oracle(engine, oracle, backend, overlap):
+@pytest.mark.parametrize("factory,species", [(W.pairwise_project, "A"), (four_species_project, "N")],
+                         ids=["pairwise", "four"])
+def test_moves_match_oracle(engine, oracle, factory, species, backend, overlap):
     """Particle moves, written one step after their hop: launches that end
     on a hop, particles without a number (adsorbed after the start), a
     trajectory that fills up inside a launch, a stopped replica."""
-    pt = W.pairwise_project()
+    pt = factory()
     cm = compile_model(pt, backend)
     hops, disp = displacement_table(cm)
     R = Records(cm)
@@ -126,15 +140,15 @@ def test_moves_match_oracle(engine, oracle, backend, overlap):
     b = engine.Batch(engine.Model(cm), [s + (1,) for s in sizes])
     b.init(seeds, np.arange(n, dtype=np.uint32))
     b.set_rates(rates)
-    configs = [np.where(g.random(int(v)) < 0.4, ids["A"], ids["empty"]).astype(np.int8) for v in b.volumes]
+    configs = [np.where(g.random(int(v)) < 0.4, ids[species], ids["empty"]).astype(np.int8) for v in b.volumes]
     b.set_config(configs)
-    b.msd_init(ids["A"], hops, disp)
+    b.msd_init(ids[species], hops, disp)
     b.msd_trajectory(300)
     b.set_overlap(overlap)
     orcs = []
     for i, s in enumerate(sizes):
         o = oracle_replica(oracle, cm, s, int(seeds[i]), i, rates[i], configs[i])
-        o.msd_init(ids["A"], hops, disp)
+        o.msd_init(ids[species], hops, disp)
         o.msd_trajectory(300)
         orcs.append(o)
     for steps in (1, 2, 61, 1, 140, 395):
