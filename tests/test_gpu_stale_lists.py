@@ -191,3 +191,37 @@ def test_stopped_replica_among_others(engine, oracle, backend):
     b.run(1, [0, 2])
     assert b.last_form() == form
     b.close()
+
+
+@pytest.mark.parametrize("backend", ["local_smart", "lat_int"])
+def test_process_that_stops_halfway(engine, oracle, backend):
+    """run_proc_nr of a process whose action finds another species stops the
+    replica, in lat_int with its deletions done: the lists are not taken for
+    the lattice's when a touchup elsewhere lets it go on."""
+    pt = W.zgb_project()
+    cm = compile_model(pt, backend)
+    sid = pt.species_ids()
+    X, Y = 10, 12
+    rates = np.array([[5.0, 1.0, 1.0, 1.0, 1.0, 0.5, 0.5]])
+    b = engine.Batch(engine.Model(cm), [(X, Y, 1)])
+    b.init([5])
+    b.set_rates(rates)
+    b.run(30)
+    assert b.last_form() == Records(cm).form
+    o = oracle_replica(oracle, cm, (X, Y), 5, 0, rates[0])
+    o.run(30)
+    site = int(np.nonzero(o.lattice() == sid["CO"])[0][0]) + 1
+    proc = cm.process_names.index("CO_adsorption") + 1
+    b.run_proc_nr(0, proc, site)
+    o.run_proc_nr(proc, site)
+    assert b.scalars(0)[4] in (2, 3) and o.status == 2
+    b.touchup(0, (site - 1 + X // 2) % X, ((site - 1) // X + Y // 2) % Y, 0, 1)
+    assert b.scalars(0)[4] == 0
+    b.run(200)
+    assert b.last_form() == 0
+    if backend == "local_smart":
+        o.set_state(o.get_state(rates[0]))
+        o.touchup((site - 1 + X // 2) % X, ((site - 1) // X + Y // 2) % Y, 0, 1)
+        o.run(200)
+        compare_state(b, 0, o, where="after the touchup")
+    b.close()
